@@ -20,8 +20,14 @@ namespace {
 
 constexpr int kWinTile = 64;  // walks per block (at most)
 constexpr int kMaxContext = 32;
-constexpr int kWinSlots = (kWinTile * kMaxContext + kBlock - 1) / kBlock;
+constexpr int kLineBytes = 128;
 constexpr size_t kTileLds = 64 * 1024;  // LDS bytes for the walk rows of a tile
+
+// Walks past the tile whose windows the tile's last line of a window position
+// can reach: the entries of a line but one, in whole walks.
+__host__ __device__ __forceinline__ int halo_walks(int32_t ctx, size_t esz) {
+    return static_cast<int>((kLineBytes / esz - 1 + ctx - 1) / ctx);
+}
 
 // Window stores are streamed past the caches: nothing here reads them again.
 #ifndef MLXC_WIN_NT
@@ -36,51 +42,75 @@ __device__ __forceinline__ void put(T* p, T v) {
 #endif
 }
 
-// Writes the windows of the tile's rows (LDS, walk_nodes entries each) for
-// every window position j.
-template <typename T>
-__device__ __forceinline__ void emit_windows(const T* rw, int64_t tile, int64_t n0,
-                                             int64_t num_walks, int32_t walk_nodes, int32_t ctx,
-                                             T* __restrict__ out);
-
-template <typename T>
+// Writes the tile's part of every window position j from its rows (LDS,
+// walk_nodes entries each): the entries of its walks, with both ends moved up
+// to the next line boundary when kHalo (the rows then include the halo_walks
+// after the tile), so that every line is written by one block, whole, and
+// every wavefront store covers whole lines.  Entry e of a position (walk
+// e / ctx of the tile, offset e % ctx) is at output index
+// (j * num_walks + n0) * ctx + e.
+//
+// Bound by the write stream.  Without the shift a wavefront's 512 bytes start
+// at any 8-byte offset unless num_walks * ctx fills whole lines, and the
+// non-temporal partial lines at its ends cost as much as whole ones:
+// 1,000,003 walks of 21 nodes, ctx 10, int64 (0.96 GB): 300 -> 182 us a
+// launch, 5.3 TB/s over both window kernels; 2^20 walks, whose runs fill whole
+// lines as they are, keep their 205 us a launch.
+template <typename T, bool kHalo>
 __device__ __forceinline__ void emit_windows(const T* rw, int64_t tile, int64_t n0,
                                              int64_t num_walks, int32_t walk_nodes, int32_t ctx,
                                              T* __restrict__ out) {
+    constexpr int kLine = kLineBytes / sizeof(T);
     const int entries = static_cast<int>(tile) * ctx;  // one window of every walk in the tile
     const int windows = walk_nodes - ctx + 1;
-    // this thread's entries of a window position: (walk, offset) pairs
-    int32_t src[kWinSlots];
-#pragma unroll
-    for (int i = 0; i < kWinSlots; ++i) {
-        const int e = threadIdx.x + i * kBlock;
-        src[i] = e < entries ? (e / ctx) * walk_nodes + e % ctx : -1;
-    }
+    const bool first = n0 == 0, last = n0 + tile == num_walks;
+    // entries of a position from the tile on, as far as the rows reach
+    const int64_t left = num_walks - n0;
+    const int rest = left < kWinTile + kLineBytes ? static_cast<int>(left) * ctx : INT32_MAX;
+    // e / ctx as (e * inv) >> 16: exact while e * (ctx - 1) < 2^16, and
+    // e < kWinTile * ctx + kLine (at ctx = 32: 2,080 * 31 = 64,480)
+    static_assert((kWinTile * kMaxContext + kLineBytes / 4) * (kMaxContext - 1) < (1 << 16),
+                  "the reciprocal is exact");
+    const uint32_t inv = ((1u << 16) + ctx - 1) / ctx;
     for (int j = 0; j < windows; ++j) {
-        T* o = out + (static_cast<int64_t>(j) * num_walks + n0) * ctx;
-#pragma unroll
-        for (int i = 0; i < kWinSlots; ++i)
-            if (src[i] >= 0) put(o + threadIdx.x + i * kBlock, rw[src[i] + j]);
+        T* const o = out + (static_cast<int64_t>(j) * num_walks + n0) * ctx;
+        int lo = 0, hi = entries;
+        if (kHalo) {
+            const int at = static_cast<int>((reinterpret_cast<uintptr_t>(o) / sizeof(T)) % kLine);
+            if (!first) lo = (kLine - at) % kLine;
+            if (!last) hi += (kLine - (at + entries) % kLine) % kLine;
+            if (hi > rest) hi = rest;  // the position ends there
+        }
+        for (int e = lo + static_cast<int>(threadIdx.x); e < hi; e += kBlock) {
+            const int w = static_cast<int>((static_cast<uint32_t>(e) * inv) >> 16);
+            put(o + e, rw[w * walk_nodes + (e - w * ctx) + j]);
+        }
     }
 }
 
-// `per_block` walks per block (<= kWinTile), so that their rows fit kTileLds
-// bytes of LDS.
-template <typename T>
+// Rows in LDS of a tile at n0: per_block walks (<= kWinTile), and the halo's
+// when the launch has room for them, as far as there are walks.
+__device__ __forceinline__ int staged_walks(int64_t n0, int64_t num_walks, int32_t per_block,
+                                            int32_t halo) {
+    const int64_t left = num_walks - n0;
+    return left < per_block + halo ? static_cast<int>(left) : per_block + halo;
+}
+
+template <typename T, bool kHalo>
 __global__ __launch_bounds__(kBlock) void context_windows_kernel(const T* __restrict__ walks,
                                                                  int64_t num_walks,
                                                                  int32_t walk_nodes, int32_t ctx,
-                                                                 int32_t per_block,
+                                                                 int32_t per_block, int32_t halo,
                                                                  T* __restrict__ out) {
     extern __shared__ unsigned char smem[];
     T* rw = reinterpret_cast<T*>(smem);
     const int64_t n0 = static_cast<int64_t>(blockIdx.x) * per_block;
     const int64_t tile = num_walks - n0 < per_block ? num_walks - n0 : per_block;
-    const int cells = static_cast<int>(tile) * walk_nodes;
+    const int cells = staged_walks(n0, num_walks, per_block, halo) * walk_nodes;
     const T* in = walks + n0 * walk_nodes;  // the tile's rows are contiguous
     for (int e = threadIdx.x; e < cells; e += kBlock) rw[e] = in[e];
     __syncthreads();
-    emit_windows(rw, tile, n0, num_walks, walk_nodes, ctx, out);
+    emit_windows<T, kHalo>(rw, tile, n0, num_walks, walk_nodes, ctx, out);
 }
 
 __device__ __forceinline__ int64_t negative_node(int64_t n, int32_t l, int64_t num_nodes,
@@ -91,26 +121,25 @@ __device__ __forceinline__ int64_t negative_node(int64_t n, int32_t l, int64_t n
     return static_cast<int64_t>((static_cast<uint64_t>(c0) * static_cast<uint64_t>(num_nodes)) >> 32);
 }
 
-// `per_block` walks per block (<= kWinTile), so that their generated rows fit
-// kTileLds bytes of LDS.
-template <typename T>
+template <typename T, bool kHalo>
 __global__ __launch_bounds__(kBlock) void negative_windows_kernel(
     const int64_t* __restrict__ start, int64_t num_walks, int32_t walk_length, int32_t ctx,
-    int64_t num_nodes, uint32_t k0, uint32_t k1, int32_t per_block, T* __restrict__ out) {
+    int64_t num_nodes, uint32_t k0, uint32_t k1, int32_t per_block, int32_t halo,
+    T* __restrict__ out) {
     // the tile's walks [start, u_1..u_L] are generated once into LDS
     extern __shared__ unsigned char smem[];
     T* rw = reinterpret_cast<T*>(smem);
     const int walk_nodes = walk_length + 1;
     const int64_t n0 = static_cast<int64_t>(blockIdx.x) * per_block;
     const int64_t tile = num_walks - n0 < per_block ? num_walks - n0 : per_block;
-    const int cells = static_cast<int>(tile) * walk_nodes;
+    const int cells = staged_walks(n0, num_walks, per_block, halo) * walk_nodes;
     for (int e = threadIdx.x; e < cells; e += kBlock) {
         const int w = e / walk_nodes, l = e % walk_nodes;
         const int64_t n = n0 + w;
         rw[e] = static_cast<T>(l == 0 ? start[n] : negative_node(n, l, num_nodes, k0, k1));
     }
     __syncthreads();
-    emit_windows(rw, tile, n0, num_walks, walk_nodes, ctx, out);
+    emit_windows<T, kHalo>(rw, tile, n0, num_walks, walk_nodes, ctx, out);
 }
 
 }  // namespace
@@ -121,21 +150,57 @@ int tile_walks(int32_t walk_nodes, size_t esz) {
     return fit > static_cast<size_t>(kWinTile) ? kWinTile : static_cast<int>(fit);
 }
 
+namespace {
+
+// Grid and LDS of a window launch.  The halo's rows join the tile's where
+// both fit kTileLds (int64, ctx 10: walks of up to 124 nodes); longer walks
+// write their lines where the tiles happen to cut them.
+struct WinLaunch {
+    int per_block, halo;
+    int64_t grid;
+    size_t lds;
+};
+
+WinLaunch win_launch(int64_t num_walks, int32_t walk_nodes, int32_t ctx, size_t esz) {
+    WinLaunch w;
+    w.per_block = tile_walks(walk_nodes, esz);
+    w.halo = halo_walks(ctx, esz);
+    const size_t row = static_cast<size_t>(walk_nodes) * esz;
+    if ((w.per_block + w.halo) * row > kTileLds) w.halo = 0;
+    w.grid = w.per_block < 1 ? 0 : (num_walks + w.per_block - 1) / w.per_block;
+    w.lds = (w.per_block + w.halo) * row;
+    return w;
+}
+
+template <typename T>
+void context_windows_typed(const WinLaunch& w, const void* walks, int64_t num_walks,
+                           int32_t walk_nodes, int32_t ctx, void* out, hipStream_t stream) {
+    auto* kernel = w.halo ? context_windows_kernel<T, true> : context_windows_kernel<T, false>;
+    hipLaunchKernelGGL(kernel, dim3(w.grid), dim3(kBlock), w.lds, stream,
+                       static_cast<const T*>(walks), num_walks, walk_nodes, ctx, w.per_block,
+                       w.halo, static_cast<T*>(out));
+}
+
+template <typename T>
+void negative_windows_typed(const WinLaunch& w, const int64_t* start, int64_t num_walks,
+                            int32_t walk_length, int32_t ctx, int64_t num_nodes, uint64_t seed,
+                            void* out, hipStream_t stream) {
+    auto* kernel = w.halo ? negative_windows_kernel<T, true> : negative_windows_kernel<T, false>;
+    hipLaunchKernelGGL(kernel, dim3(w.grid), dim3(kBlock), w.lds, stream, start, num_walks,
+                       walk_length, ctx, num_nodes, static_cast<uint32_t>(seed),
+                       static_cast<uint32_t>(seed >> 32), w.per_block, w.halo,
+                       static_cast<T*>(out));
+}
+
+}  // namespace
+
 int launch_context_windows(const void* walks, int64_t num_walks, int32_t walk_nodes, int32_t ctx,
                            int32_t elem_type, void* out, hipStream_t stream) {
-    const size_t esz = elem_type == MLXC_OUT_INT32 ? 4 : 8;
-    const int per_block = tile_walks(walk_nodes, esz);
-    if (per_block < 1) return fail(MLXC_ERR_INVALID_ARGUMENT, "walks too long for windows");
-    const int64_t grid = (num_walks + per_block - 1) / per_block;
-    const size_t lds = static_cast<size_t>(per_block) * walk_nodes * esz;
-    if (elem_type == MLXC_OUT_INT32)
-        hipLaunchKernelGGL(context_windows_kernel<int32_t>, dim3(grid), dim3(kBlock), lds, stream,
-                           static_cast<const int32_t*>(walks), num_walks, walk_nodes, ctx,
-                           per_block, static_cast<int32_t*>(out));
-    else
-        hipLaunchKernelGGL(context_windows_kernel<int64_t>, dim3(grid), dim3(kBlock), lds, stream,
-                           static_cast<const int64_t*>(walks), num_walks, walk_nodes, ctx,
-                           per_block, static_cast<int64_t*>(out));
+    const bool narrow = elem_type == MLXC_OUT_INT32;
+    const WinLaunch w = win_launch(num_walks, walk_nodes, ctx, narrow ? 4 : 8);
+    if (w.per_block < 1) return fail(MLXC_ERR_INVALID_ARGUMENT, "walks too long for windows");
+    if (narrow) context_windows_typed<int32_t>(w, walks, num_walks, walk_nodes, ctx, out, stream);
+    else context_windows_typed<int64_t>(w, walks, num_walks, walk_nodes, ctx, out, stream);
     MLXC_HIP_TRY(hipGetLastError());
     return MLXC_OK;
 }
@@ -147,20 +212,15 @@ int windows_max_nodes(int32_t elem_type) {
 int launch_negative_windows(const int64_t* start, int64_t num_walks, int32_t walk_length,
                             int32_t ctx, int64_t num_nodes, uint64_t seed, int32_t out_type,
                             void* out, hipStream_t stream) {
-    const size_t esz = out_type == MLXC_OUT_INT32 ? 4 : 8;
-    const int per_block = tile_walks(walk_length + 1, esz);
-    if (per_block < 1) return fail(MLXC_ERR_INVALID_ARGUMENT, "walk_length too large");
-    const int64_t grid = (num_walks + per_block - 1) / per_block;
-    const uint32_t k0 = static_cast<uint32_t>(seed), k1 = static_cast<uint32_t>(seed >> 32);
-    const size_t lds = static_cast<size_t>(per_block) * (walk_length + 1) * esz;
-    if (out_type == MLXC_OUT_INT32)
-        hipLaunchKernelGGL(negative_windows_kernel<int32_t>, dim3(grid), dim3(kBlock), lds, stream,
-                           start, num_walks, walk_length, ctx, num_nodes, k0, k1, per_block,
-                           static_cast<int32_t*>(out));
+    const bool narrow = out_type == MLXC_OUT_INT32;
+    const WinLaunch w = win_launch(num_walks, walk_length + 1, ctx, narrow ? 4 : 8);
+    if (w.per_block < 1) return fail(MLXC_ERR_INVALID_ARGUMENT, "walk_length too large");
+    if (narrow)
+        negative_windows_typed<int32_t>(w, start, num_walks, walk_length, ctx, num_nodes, seed,
+                                        out, stream);
     else
-        hipLaunchKernelGGL(negative_windows_kernel<int64_t>, dim3(grid), dim3(kBlock), lds, stream,
-                           start, num_walks, walk_length, ctx, num_nodes, k0, k1, per_block,
-                           static_cast<int64_t*>(out));
+        negative_windows_typed<int64_t>(w, start, num_walks, walk_length, ctx, num_nodes, seed,
+                                        out, stream);
     MLXC_HIP_TRY(hipGetLastError());
     return MLXC_OK;
 }

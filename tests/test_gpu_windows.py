@@ -75,3 +75,36 @@ def test_c2_walk_windows_full_size(cuda):
     rw = oracle.negative_walks(start[s].cpu().numpy(), 20, V, 9, walk_ids=s.cpu().numpy())
     for j in range(W):
         np.testing.assert_array_equal(neg[j * N + s].cpu().numpy(), rw[:, j:j + 10])
+
+
+@pytest.mark.parametrize("N", [65, 79, 80, 127, 129, 1003])
+@pytest.mark.parametrize("nodes,C", [(4, 1), (21, 2), (21, 3), (21, 10), (33, 16), (40, 32)])
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+@pytest.mark.parametrize("shift", [0, 1, 5])
+def test_windows_line_edges(N, nodes, C, dtype, shift, cuda):
+    """Tiles whose ends are moved to line boundaries: runs of every length
+    around a tile (64 walks) and a line (16 or 32 entries), into buffers that
+    start inside a line; nothing outside the output is written."""
+    from mlx_cluster_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(N + nodes + C)
+    walks = torch.from_numpy(rng.integers(0, 2**31 - 1, (N, nodes))).to(dtype)
+    out_type = _lib.MLXC_OUT_INT32 if dtype == torch.int32 else _lib.MLXC_OUT_INT64
+    total = (nodes - C + 1) * N * C
+    d_walks, start = walks.to(cuda), walks[:, 0].long().to(cuda)
+    stream = torch.cuda.current_stream().cuda_stream
+    for negative in (False, True):
+        buf = torch.full((total + 64,), -7, dtype=dtype, device=cuda)
+        out = buf[shift:]
+        if negative:
+            rc = lib.mlxc_negative_windows(start.data_ptr(), N, nodes - 1, C, 1 << 20, 9, out_type,
+                                           out.data_ptr(), stream)
+            ref = oracle.negative_windows(start.cpu().numpy(), nodes - 1, C, 1 << 20, 9)
+        else:
+            rc = lib.mlxc_context_windows(d_walks.data_ptr(), N, nodes, C, out_type,
+                                          out.data_ptr(), stream)
+            ref = oracle.context_windows(walks.numpy(), C)
+        assert rc == 0
+        got = buf.cpu().numpy()
+        np.testing.assert_array_equal(got[shift:shift + total], ref.reshape(-1).astype(got.dtype))
+        assert (got[:shift] == -7).all() and (got[shift + total:] == -7).all()
