@@ -29,6 +29,7 @@
 // drops repeated keys.
 // rowptr is filled with the entry count, row starts are written into it, and a
 // reverse inclusive min-scan gives empty rows the start of the next row.
+#include "block_sort.h"
 #include "walk_host.h"
 
 namespace mlxc {
@@ -674,7 +675,97 @@ __global__ __launch_bounds__(kBlock) void csr_emit_kernel(Store keys,
     }
 }
 
+// ------------------------------------------------------------- small lists
+
+// The whole build of a small list in one launch: one block sorts the list's
+// keys (32 bits) in registers, drops repeats, and writes col, rowptr (a
+// binary search of the kept keys per row) and the words of `work`.
+//
+// Bound by its one compute unit's instruction rate (the network of
+// block_sort.h); the 16 launches of the radix passes on such a list each take
+// longer than their work.  10,556 pairs over 2,708 nodes: 16 launches of 74 us
+// in all -> one of 38 us, to_csr 92 -> 58 us.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void csr_small_kernel(EdgeSrc src, int total, bool dedup,
+                                                             int64_t* __restrict__ rowptr,
+                                                             int64_t* __restrict__ col_out,
+                                                             int64_t* __restrict__ work) {
+    static_assert(kSortItems == kItems, "16 keys a thread");
+    __shared__ uint32_t lds[sort_lds_keys<kThreads>()];
+    __shared__ uint32_t last[kThreads];
+    __shared__ int64_t wtot[kThreads / kWave];
+    const int t = threadIdx.x, lane = t % kWave;
+    uint32_t key[kItems];
+    bool bad = false;
+    // a wavefront's 1,024 keys, 64 consecutive entries a slot
+    const int base = (t - lane) * kItems + lane;
+    load_slots<Keys32, Src::kBoth>(key, src, Keys32{}, base, kWave, total, bad);
+#pragma unroll
+    for (int s = 0; s < kItems; ++s)
+        if (base + s * kWave >= total) key[s] = ~0u;
+    const int any_bad = __syncthreads_or(bad);
+    block_sort<kThreads>(key, total, lds);
+
+    // Keep the first of equal keys (dedup), in order.
+    last[t] = key[kItems - 1];
+    __syncthreads();
+    const uint32_t before = t > 0 ? last[t - 1] : 0u;
+    uint32_t keep = 0;
+#pragma unroll
+    for (int s = 0; s < kItems; ++s) {
+        const int i = t * kItems + s;
+        const uint32_t prev = s > 0 ? key[s > 0 ? s - 1 : 0] : before;
+        if (i < total && (!dedup || i == 0 || prev != key[s])) keep |= 1u << s;
+    }
+    int64_t all;
+    int p = static_cast<int>(
+        block_exclusive_scan<kOpSum, kThreads>(__popc(keep), wtot, &all));
+#pragma unroll
+    for (int s = 0; s < kItems; ++s)
+        if ((keep >> s) & 1u) lds[p++] = key[s];
+    __syncthreads();
+    const int n = static_cast<int>(all);
+    const uint32_t cmask = src.cbits == 0 ? 0u : ~0u >> (32 - src.cbits);
+    for (int j = t; j < n; j += kThreads) col_out[j] = static_cast<int64_t>(lds[j] & cmask);
+    // rowptr[r]: the kept keys of the rows before r, four rows a thread at a
+    // time so that their searches' reads overlap
+    constexpr int kRows = 4;
+    const int V = static_cast<int>(src.num_nodes);
+    for (int r0 = t; r0 <= V; r0 += kRows * kThreads) {
+        int lo[kRows];
+#pragma unroll
+        for (int q = 0; q < kRows; ++q) lo[q] = 0;
+        for (int step = kThreads * kItems; step > 0; step >>= 1) {
+#pragma unroll
+            for (int q = 0; q < kRows; ++q) {
+                const int r = r0 + q * kThreads;
+                const int at = lo[q] + step;
+                // keys before `at` are of rows before r
+                if (at <= n && static_cast<int64_t>(lds[at - 1] >> src.cbits) < r) lo[q] = at;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kRows; ++q) {
+            const int r = r0 + q * kThreads;
+            if (r <= V) rowptr[r] = lo[q];
+        }
+    }
+    if (t < MLXC_WORK_WORDS)
+        work[t] = t == 0 ? (any_bad ? MLXC_STATUS_BAD_NODE : 0) : t == 1 ? n : 0;
+}
+
 // ------------------------------------------------------------- host side
+
+// Lists of up to kSmallTotal entries (what one block's registers hold) over up
+// to kSmallNodes nodes are built by csr_small_kernel.  The searches of rowptr
+// cost it 4 us per 4,096 rows: to_csr of 16,384 pairs takes 80 us over 20,000
+// nodes and 124 over 65,536, with the radix passes 114 either way.  With 256
+// threads those searches cost four times as much, and pay only where rows are
+// few: 4,096 pairs over 2,708 nodes take 45 us.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallTotal = kSmallThreads * kItems;
+constexpr int64_t kSmallNodes = 32768;
+static_assert(2 * 15 <= 32, "keys over kSmallNodes nodes take 32 bits");
 
 int bits_for(int64_t num_nodes) {
     int b = 0;
@@ -888,9 +979,21 @@ int launch_csr_build(const int64_t* row, const int64_t* col, int64_t num_edges, 
                     "workspace smaller than mlxc_csr_build_workspace_bytes()");
     char* ws = static_cast<char*>(workspace);
     int64_t* work = reinterpret_cast<int64_t*>(ws);
+    const EdgeSrc src{row, col, num_edges, num_nodes, l.cbits};
+    if (l.total > 0 && l.total <= kSmallTotal && num_nodes <= kSmallNodes) {
+        const bool dedup = (flags & MLXC_CSR_DEDUP) != 0;
+        const int total = static_cast<int>(l.total);
+        if (total <= kBlock * kItems && num_nodes <= kBlock * kItems)
+            hipLaunchKernelGGL(csr_small_kernel<kBlock>, dim3(1), dim3(kBlock), 0, stream, src,
+                               total, dedup, rowptr, col_out, work);
+        else
+            hipLaunchKernelGGL(csr_small_kernel<kSmallThreads>, dim3(1), dim3(kSmallThreads), 0,
+                               stream, src, total, dedup, rowptr, col_out, work);
+        MLXC_HIP_TRY(hipGetLastError());
+        return MLXC_OK;
+    }
     if (int rc = launch_zero_work(work, stream)) return rc;
     if (l.total == 0) return fill_words(rowptr, num_nodes + 1, work + 1, stream);
-    const EdgeSrc src{row, col, num_edges, num_nodes, l.cbits};
     if (l.key_bytes == 4) return csr_build_typed<Keys32>(src, l, flags, rowptr, col_out, ws, stream);
     if (l.key_bytes == 5) return csr_build_typed<Keys40>(src, l, flags, rowptr, col_out, ws, stream);
     if (l.key_bytes == 6) return csr_build_typed<Keys48>(src, l, flags, rowptr, col_out, ws, stream);

@@ -266,3 +266,29 @@ def test_rowptr_of_2_28_nodes(cuda):
         order = np.lexsort((col, row))
         np.testing.assert_array_equal(c.cpu().numpy(), col[order])
         del rowptr, c, ref
+
+
+@pytest.mark.parametrize("E", [15, 16, 1024, 1025, 2049, 4096, 4097, 8193, 10_556, 16_383, 16_384,
+                               16_385])
+@pytest.mark.parametrize("V", [3, 2708, 4097, 32768, 32769, 65536])
+def test_small_list_edges(E, V, cuda):
+    """The one-launch build around its wavefront, block and size limits (and
+    just past them), with the largest ids, equal keys and empty rows at both
+    ends."""
+    rng = np.random.default_rng(E + V)
+    row, col = rng.integers(V // 3, V, E), rng.integers(0, V, E)
+    row[: E // 2] = row[0]          # a hub
+    row[E // 3: E // 3 + 9] = col[E // 3: E // 3 + 9] = V - 1
+    for dedup in (False, True):
+        assert_parity(row, col, V, cuda, dedup=dedup)
+    assert_parity(np.full(E, V - 1), np.full(E, V - 1), V, cuda)
+    if E <= 8193:
+        assert_parity(row, col, V, cuda, symmetrize=True, dedup=True)
+
+
+def test_small_list_bad_ids(cuda):
+    for bad in (-1, 2708, 1 << 40):
+        ei = torch.randint(0, 2708, (2, 10_556), device=cuda)
+        ei[1, 10_000] = bad
+        with pytest.raises(ValueError, match="outside"):
+            mc.to_csr(ei, 2708)
