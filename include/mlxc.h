@@ -120,6 +120,15 @@ const char* mlxc_last_error(void);
 size_t mlxc_random_walk_workspace_bytes(int64_t num_nodes, int64_t num_edges,
                                         int64_t num_walks, int32_t walk_length);
 
+/* Workspace bytes with which mlxc_random_walk is fastest for these arguments:
+ * MLXC_WORK_WORDS * 8, which selects the flat walk (no queue and no per-call
+ * layout: it reads the CSR arrays as they are), in calls up to a size, else
+ * what mlxc_random_walk_workspace_bytes returns.  A workspace of that size or
+ * larger runs the record and CSR walks whatever the call's size.  No
+ * reference counterpart. */
+size_t mlxc_random_walk_preferred_bytes(int64_t num_nodes, int64_t num_edges,
+                                        int64_t num_walks, int32_t walk_length);
+
 /* Workspace bytes for mlxc_rejection_sampling's fastest layout for these
  * arguments (same conventions).  Either edge records (16 bytes per edge), or
  * the CSR mode's layout, which reads each candidate's node id and then, only

@@ -275,6 +275,11 @@ size_t mlxc_random_walk_workspace_bytes(int64_t num_nodes, int64_t num_edges, in
     return uniform_workspace_bytes(num_nodes, num_edges, num_walks, walk_length);
 }
 
+size_t mlxc_random_walk_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
+                                        int32_t walk_length) {
+    return uniform_preferred_bytes(num_nodes, num_edges, num_walks, walk_length);
+}
+
 size_t mlxc_rejection_sampling_workspace_bytes(int64_t num_nodes, int64_t num_edges,
                                                int64_t num_walks, int32_t walk_length, double p,
                                                double q, int32_t rule) {

@@ -120,7 +120,7 @@ py::object random_walk(const at::Tensor& rowptr, const at::Tensor& col, const at
     const auto opts = at::TensorOptions().dtype(dtype).device(device);
     at::Tensor n_out = at::empty({N, L + 1}, opts);
     at::Tensor e_out = return_edges ? at::empty({N, L}, opts) : at::Tensor();
-    const size_t ws = mlxc_random_walk_workspace_bytes(V, E, N, static_cast<int32_t>(L));
+    const size_t ws = mlxc_random_walk_preferred_bytes(V, E, N, static_cast<int32_t>(L));
     at::Tensor work = at::empty({static_cast<int64_t>((ws + 7) / 8)},
                                 at::TensorOptions().dtype(at::kLong).device(device));
     hipStream_t stream = at::hip::getCurrentHIPStream().stream();

@@ -2,124 +2,19 @@
 //
 // The walk is a chain of dependent random reads, so throughput comes from
 // the number of chains in flight and the number of reads per step, not from
-// arithmetic.  Every lane runs a small state machine over W walk slots; a
+// arithmetic.  Large calls run persistent kernels (edge records, or the CSR
+// arrays): every lane runs a small state machine over W walk slots, and a
 // slot whose walk ends (or is absorbed by a node of out-degree 0) takes the
 // next walk from a per-wavefront queue refilled by one global atomic per
 // kQueueChunk (64) walks, so lanes never idle while walks remain and the
-// kernel's tail is about one walk long.  Grids are the device's resident
-// capacity.
+// kernel's tail is about one walk long; their grids are the device's resident
+// capacity.  Smaller calls run the flat walk, one walk a lane from start to
+// end, or, on graphs that fit LDS, the LDS walk.
 #include <type_traits>
 
 #include "walk_host.h"
 
 namespace mlxc {
-
-// Uniform walk without stream windows: W walk slots per lane, walks from the
-// wave queue, 8-byte loads and stores.  Serves the cases the windowed
-// kernels do not: buffers that are not 16-byte aligned, a rand tensor whose
-// size is not a multiple of 4, graphs beyond int32 ids, and a workspace too
-// small for the start records.
-template <int W, bool kEdges, bool kGen, typename OutT>
-__global__ __launch_bounds__(kBlock) void uniform_walk_kernel(WalkArgs a) {
-    const int64_t L = a.walk_length;
-    const int64_t N = a.num_walks;
-    const int64_t goff = kGen ? a.walk_base * L : 0;  // stream position of uniform 0
-    OutT* const nout = static_cast<OutT*>(a.n_out);
-    OutT* const eout = static_cast<OutT*>(a.e_out);
-    unsigned long long* counter = reinterpret_cast<unsigned long long*>(a.work + 1);
-    WaveQueue q{0, 0};
-    int64_t n[W], v[W], l[W];
-    uint32_t status = 0;
-
-#pragma unroll
-    for (int s = 0; s < W; ++s) { n[s] = -1; l[s] = L; v[s] = 0; }
-
-    while (true) {
-        // Acquire walks for empty slots; write their first column.
-        bool unretired = false;
-#pragma unroll
-        for (int s = 0; s < W; ++s) {
-            const bool need = (n[s] < N) && (l[s] >= L);  // slot idle (or never used)
-            const int64_t id = queue_take(q, need, counter);
-            if (need) {
-                n[s] = id;  // id >= N ends the slot for good
-                if (id < N) {
-                    const int64_t s0 = a.start[id];
-                    nout[id * (L + 1)] = static_cast<OutT>(s0);
-                    v[s] = s0;
-                    l[s] = 0;
-                    if (!node_ok(s0, a.num_nodes)) {
-                        status |= MLXC_STATUS_BAD_NODE;
-                        for (int64_t j = 1; j <= L; ++j) nout[id * (L + 1) + j] = static_cast<OutT>(s0);
-                        if (kEdges)
-                            for (int64_t j = 0; j < L; ++j) eout[id * L + j] = -1;
-                        l[s] = L;
-                    }
-                }
-            }
-            unretired |= (n[s] < N);
-        }
-        // The whole wave leaves together, once every slot of every lane has
-        // drawn an id past the end; until then idle lanes keep voting.
-        if (!__any(unretired)) break;
-
-        // Phase 1: rowptr pair and the step's uniform, for every live slot.
-        RowBounds rb[W];
-        float r[W];
-#pragma unroll
-        for (int s = 0; s < W; ++s) {
-            const bool live = (n[s] < N) && (l[s] < L);
-            rb[s] = {0, 0};
-            r[s] = 0.0f;
-            if (live) {
-                rb[s] = load_row(a.rowptr, v[s]);
-                r[s] = kGen ? philox_uniform_at(goff + n[s] * L + l[s], a.key0, a.key1)
-                            : __builtin_nontemporal_load(a.rand + n[s] * L + l[s]);
-            }
-        }
-        // Phase 2: candidate edge and its target, for every moving slot.
-        int64_t e[W], x[W];
-#pragma unroll
-        for (int s = 0; s < W; ++s) {
-            const bool live = (n[s] < N) && (l[s] < L);
-            e[s] = -1;
-            x[s] = v[s];
-            if (live) {
-                const int64_t deg = rb[s].end - rb[s].begin;
-                if (!row_ok(rb[s], a.num_edges)) {
-                    status |= MLXC_STATUS_BAD_ROW;
-                } else if (deg > 0) {
-                    e[s] = rb[s].begin + pick_index(r[s], deg);
-                    x[s] = a.col[e[s]];
-                }
-            }
-        }
-        // Phase 3: store, advance, and finish sunk / broken walks.
-#pragma unroll
-        for (int s = 0; s < W; ++s) {
-            const bool live = (n[s] < N) && (l[s] < L);
-            if (!live) continue;
-            OutT* out = nout + n[s] * (L + 1);
-            const bool moved = e[s] >= 0;
-            bool stop = !moved;  // deg == 0 (absorbing) or malformed row
-            out[l[s] + 1] = static_cast<OutT>(x[s]);
-            if (kEdges) eout[n[s] * L + l[s]] = static_cast<OutT>(e[s]);
-            l[s] += 1;
-            if (moved && !node_ok(x[s], a.num_nodes)) {
-                status |= MLXC_STATUS_BAD_NODE;
-                stop = true;
-            }
-            v[s] = x[s];
-            if (stop) {
-                for (int64_t j = l[s] + 1; j <= L; ++j) out[j] = static_cast<OutT>(x[s]);
-                if (kEdges)
-                    for (int64_t j = l[s]; j < L; ++j) eout[n[s] * L + j] = -1;
-                l[s] = L;
-            }
-        }
-    }
-    if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
-}
 
 // Slot phases of the windowed walks.
 enum : int {
@@ -132,9 +27,8 @@ enum : int {
     kSlotDone = 5,   // the queue is exhausted
 };
 
-// Uniform walk over edge records (requires 16-byte aligned rand, n_out and
-// e_out, num_nodes and num_edges below 2^31, num_walks * walk_length a
-// multiple of 4 and at least RW).
+// Uniform walk over edge records (requires 16-byte aligned n_out and e_out,
+// num_nodes and num_edges below 2^31, num_walks * walk_length at least RW).
 //
 // Loop invariant: every live slot issues exactly one dependent read per
 // iteration (a start record or an edge record; with packed records also the
@@ -638,6 +532,145 @@ __global__ __launch_bounds__(kLdsBlock) void uniform_walk_lds_kernel(WalkArgs a)
     if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
 }
 
+// Uniform walk over the CSR arrays as they are: one walk a lane, `per_wave`
+// walks a wavefront (a block), no queue, no workspace but the status words.
+// Any graph and any alignment.
+//
+// Bound by the walks' chains, two dependent reads a step (the row, then the
+// entry of col): by their latency in calls of few walks, which are therefore
+// spread thin over the device, and by the rate of random reads in large ones.
+// So nothing else is in the chain.  The walk goes in stretches of `steps`
+// output positions.  Before a stretch all 64 lanes read or generate its
+// uniforms into LDS, one slot a position; at each step the walk's node takes
+// the slot of the uniform it used; after the stretch all lanes store the
+// slots, consecutive lanes consecutive entries.  (A store between the reads
+// would be waited for with them: one counter orders both.)
+//
+// Measured (R-MAT 2^20, 16 M entries, against the CSR or record walk, whose
+// loops carry the queue, the rand and output windows and the drain of the
+// stores through every step): 1,300 walks of 37 steps, seeded, int32 with
+// edges, 131 -> 33 us a call; 2^20 walks of 20 steps 481 -> 324 us.  Where it
+// stops paying: flat_walk_pays.
+//
+// Slot: int32_t, or int64_t where ids do not fit it.
+template <typename Slot>
+__device__ __forceinline__ float slot_float(Slot s) {
+    return __uint_as_float(static_cast<uint32_t>(s));
+}
+template <typename Slot>
+__device__ __forceinline__ Slot float_slot(float r) {
+    return static_cast<Slot>(__float_as_uint(r));
+}
+
+template <bool kGen, bool kEdges, typename OutT, typename Slot>
+__global__ __launch_bounds__(kWave) void uniform_walk_flat_kernel(WalkArgs a, int per_wave,
+                                                                  int steps) {
+    // [walk][position], rows padded by one so that the lanes' accesses spread
+    // over the banks
+    extern __shared__ __align__(16) unsigned char flat_lds[];
+    const int row = steps + 1;
+    const int lane = threadIdx.x;
+    Slot* const nodes = reinterpret_cast<Slot*>(flat_lds);
+    Slot* const edges = nodes + per_wave * row;  // kEdges: the step into each position
+    const int64_t L = a.walk_length;
+    const int64_t n0 = static_cast<int64_t>(blockIdx.x) * per_wave;
+    const int64_t left = a.num_walks - n0;
+    const int walks = left < per_wave ? static_cast<int>(left) : per_wave;
+    OutT* const nout = static_cast<OutT*>(a.n_out) + n0 * (L + 1);
+    OutT* const eout = kEdges ? static_cast<OutT*>(a.e_out) + n0 * L : nullptr;
+    uint32_t status = 0;
+    bool alive = false;
+    int64_t v = 0;
+    if (lane < walks) {
+        v = a.start[n0 + lane];
+        nodes[lane * row] = static_cast<Slot>(v);
+        alive = node_ok(v, a.num_nodes);
+        if (!alive) status |= MLXC_STATUS_BAD_NODE;
+    }
+    // positions p0 .. p0 + len - 1 of the rows; the step into position p uses
+    // uniform p - 1
+    for (int64_t p0 = 0; p0 <= L; p0 += steps) {
+        const int len = L + 1 - p0 < steps ? static_cast<int>(L + 1 - p0) : steps;
+        const int cells = walks * len;
+        // i / len as (i * inv) >> 20: exact for i * (len - 1) < 2^20, which
+        // flat_shape keeps
+        const uint32_t inv = ((1u << 20) + len - 1) / len;
+        const int first = p0 == 0 ? 1 : 0;  // position 0 is the start
+        int reached = first;                // this walk's positions of the stretch
+        const uint64_t moving = __ballot(alive);
+        if (moving) {
+            if (kGen) {
+                // Philox blocks of four uniforms; a walk's stretch touches at
+                // most (len + 6) / 4 of them
+                const int blocks = (len + 6) / 4;
+                for (int i = lane; i < walks * blocks; i += kWave) {
+                    const int w = i / blocks;
+                    const int64_t f = (a.walk_base + n0 + w) * L + p0 - 1;
+                    const int64_t base = (f & ~int64_t{3}) + 4 * (i % blocks);
+                    // before the stream: position 0 has no uniform
+                    if (base < 0 || !((moving >> w) & 1)) continue;
+                    RandWindow<4> r;
+                    rw_gen_at(r, base, a.key0, a.key1);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int64_t j = base + k - f;
+                        if (j >= first && j < len) nodes[w * row + j] = float_slot<Slot>(r.w[k]);
+                    }
+                }
+            } else {
+                const float* const rand = a.rand + n0 * L + p0 - 1;
+                for (int i = lane; i < cells; i += kWave) {
+                    const int w = static_cast<int>((static_cast<uint32_t>(i) * inv) >> 20);
+                    const int j = i - w * len;
+                    if (j >= first && ((moving >> w) & 1))
+                        nodes[w * row + j] =
+                            float_slot<Slot>(__builtin_nontemporal_load(rand + w * L + j));
+                }
+            }
+            wave_sync();
+            for (int j = first; j < len && __any(alive); ++j) {
+                if (!alive) continue;
+                const RowBounds rb = load_row(a.rowptr, v);
+                if (!row_ok(rb, a.num_edges)) {
+                    status |= MLXC_STATUS_BAD_ROW;
+                    alive = false;
+                } else if (rb.end == rb.begin) {
+                    alive = false;  // absorbing node: the walk stays
+                } else {
+                    const int64_t e = rb.begin + pick_index(slot_float(nodes[lane * row + j]),
+                                                            rb.end - rb.begin);
+                    v = a.col[e];
+                    nodes[lane * row + j] = static_cast<Slot>(v);
+                    if (kEdges) edges[lane * row + j] = static_cast<Slot>(e);
+                    reached = j + 1;
+                    if (!node_ok(v, a.num_nodes)) {
+                        status |= MLXC_STATUS_BAD_NODE;
+                        alive = false;
+                    }
+                }
+            }
+            wave_sync();
+        }
+        // a walk that stopped stays where it is
+        for (int i0 = 0; i0 < cells; i0 += kWave) {
+            const int i = i0 + lane;
+            const bool mine = i < cells;
+            const int w = mine ? static_cast<int>((static_cast<uint32_t>(i) * inv) >> 20) : 0;
+            const int j = mine ? i - w * len : 0;
+            const int got = __shfl(reached, w, kWave);
+            const int64_t stay = __shfl(v, w, kWave);
+            if (!mine) continue;
+            nout[w * (L + 1) + p0 + j] =
+                static_cast<OutT>(j < got ? static_cast<int64_t>(nodes[w * row + j]) : stay);
+            if (kEdges && p0 + j > 0)
+                eout[w * L + p0 - 1 + j] =
+                    static_cast<OutT>(j < got ? edges[w * row + j] : Slot{-1});
+        }
+        wave_sync();
+    }
+    if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
+}
+
 // ------------------------------------------------------------- launcher
 
 // Walks in flight per lane.  Both walks run best with one slot at the
@@ -671,7 +704,7 @@ constexpr int32_t kLongWalk = 64;
 
 namespace {
 
-enum class UniformMode { kRecords, kCsr, kCsrWide, kLds, kPlain };
+enum class UniformMode { kRecords, kCsr, kCsrWide, kLds, kFlat };
 
 // Edge records cost one random read per edge to build; they pay off when the
 // call takes several steps per edge, or when the graph is small enough that
@@ -695,10 +728,27 @@ size_t init_bytes(int64_t num_walks) {
     return kRecordOffset + static_cast<size_t>(num_walks) * sizeof(EdgeRecord);
 }
 
+// Whether the flat walk beats the persistent walk the call would otherwise
+// run.  Its lanes idle once their walks are absorbed, and its walks longer
+// than a stretch store their rows in pieces, so it loses to the record walk
+// (one read a step, N * L >= 4 E) past about N * L^2 = 2^31 and to the CSR
+// walk past 2^32.  Measured, us a call, rand given, int64 (flat / persistent):
+//   E 0.5 M:  2^18 x 80  192 / 278,  2^20 x 80   690 / 671,  2^24 x 20  3,064 / 3,444
+//   E 16 M:   2^18 x 80  298 / 396,  2^20 x 80 1,009 / 999,  2^22 x 20  1,172 / 1,259,
+//             2^24 x 20  4,740 / 4,232
+//   E 263 M:  2^20 x 80  1,272 / 1,364,  2^22 x 20  1,437 / 1,668,
+//             2^22 x 80  5,171 / 4,496,  2^24 x 20  5,837 / 5,778
+bool flat_walk_pays(int64_t num_walks, int32_t walk_length, bool records) {
+    const double l = walk_length > 0 ? walk_length : 1;
+    return static_cast<double>(num_walks) * l * l <= (records ? 0x1p31 : 0x1p32);
+}
+
+// A workspace that holds the start records selects the persistent walks, one
+// of the status words alone the flat walk (uniform_preferred_bytes chooses).
 UniformMode uniform_mode(const WalkArgs& a, size_t workspace_bytes, bool gen) {
     const int64_t rtotal = a.num_walks * a.walk_length;
-    const bool rand_ok = gen || (reinterpret_cast<uintptr_t>(a.rand) % 16 == 0 && rtotal % 4 == 0 &&
-                                 rtotal >= MLXC_RAND_WINDOW);
+    // a whole rand block to read, of floats at any float's alignment
+    const bool rand_ok = gen || rtotal >= MLXC_RAND_WINDOW;
     const bool streams_ok = rand_ok && reinterpret_cast<uintptr_t>(a.n_out) % 16 == 0 &&
                             reinterpret_cast<uintptr_t>(a.e_out) % 16 == 0;  // e_out may be null
     if (streams_ok && records_fit(a.num_nodes, a.num_edges)) {
@@ -715,8 +765,43 @@ UniformMode uniform_mode(const WalkArgs& a, size_t workspace_bytes, bool gen) {
     if (workspace_bytes >= kRecordOffset &&
         lds_walk_fits(a.num_nodes, a.num_edges, a.num_walks, a.walk_length))
         return UniformMode::kLds;
-    return UniformMode::kPlain;
+    return UniformMode::kFlat;
 }
+
+// Walks of a wavefront of the flat walk, and output positions of a stretch.
+// Few walks are spread over kFlatWaves wavefronts per compute unit (8: within
+// 5% of 4, 16 and 32 from 130 to 2^18 walks) and take long stretches;
+// wavefronts of 64 walks take stretches of up to 33 positions, which leave
+// 8.7 KB of LDS a wavefront (with edges 17.4 KB), 18 of them on a compute
+// unit (stretches of 21 and 41 were slower by up to 10% at 81 positions).
+constexpr int kFlatWaves = 8;
+constexpr int kFlatSteps = 33;
+constexpr int kFlatCells = 1024;  // walks x positions of a wavefront of few walks
+
+struct FlatShape {
+    int per_wave, steps;
+    int64_t blocks;
+};
+
+FlatShape flat_shape(int64_t num_walks, int32_t walk_length, int cus) {
+    FlatShape f;
+    const int64_t waves = static_cast<int64_t>(cus) * kFlatWaves;
+    const int64_t per = (num_walks + waves - 1) / waves;
+    f.per_wave = per < kWave ? static_cast<int>(per) : kWave;
+    int64_t most = kFlatCells / f.per_wave;
+    if (most < kFlatSteps) most = kFlatSteps;
+    // the positions split evenly over the stretches they need
+    const int64_t positions = static_cast<int64_t>(walk_length) + 1;
+    const int64_t stretches = (positions + most - 1) / most;
+    f.steps = static_cast<int>((positions + stretches - 1) / stretches);
+    f.blocks = (num_walks + f.per_wave - 1) / f.per_wave;
+    return f;
+}
+// (cells - 1) * (steps - 1), the flat walk's bound on its exact division
+static_assert(kFlatCells * (kFlatCells - 1) < (1 << 20) &&
+                  kWave * kFlatSteps * (kFlatSteps - 1) < (1 << 20) &&
+                  (kFlatCells + kFlatSteps * kFlatCells / kFlatSteps) <= 2 * kFlatCells,
+              "i / len is exact");
 
 // Resident blocks per compute unit of the persistent walks (0: as many as
 // the kernel's registers allow).  The record walk runs best well below its
@@ -756,6 +841,18 @@ size_t uniform_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t num
     return records_pay_off(num_edges, num_walks, walk_length)
                ? record_bytes(num_nodes, num_edges, num_walks)
                : init_bytes(num_walks);
+}
+
+size_t uniform_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
+                               int32_t walk_length) {
+    const size_t queried = uniform_workspace_bytes(num_nodes, num_edges, num_walks, walk_length);
+    if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0 ||
+        queried == kRecordOffset)  // the LDS walk
+        return queried;
+    const bool records = records_fit(num_nodes, num_edges) &&
+                         records_pay_off(num_edges, num_walks, walk_length);
+    return flat_walk_pays(num_walks, walk_length, records) ? MLXC_WORK_WORDS * sizeof(int64_t)
+                                                           : queried;
 }
 
 namespace {
@@ -819,11 +916,37 @@ int launch_uniform_impl(const WalkArgs& a, void* workspace, size_t workspace_byt
         MLXC_HIP_TRY(hipGetLastError());
         return record_walk_event(1, stream);
     }
-    case UniformMode::kPlain:
+    case UniformMode::kFlat:
         break;
     }
+    DeviceInfo info;
+    if (int rc = device_info(info)) return rc;
     if (int rc = launch_zero_work(a.work, stream)) return rc;
-    return launch_walk_kernel(uniform_walk_kernel<2, kEdges, kGen, OutT>, 2, 0, a, stream);
+    const FlatShape f = flat_shape(a.num_walks, a.walk_length, info.cus);
+    const bool wide = !records_fit(a.num_nodes, a.num_edges);
+    const size_t lds = static_cast<size_t>(f.per_wave) * (f.steps + 1) * (kEdges ? 2 : 1) *
+                       (wide ? sizeof(int64_t) : sizeof(int32_t));
+    auto* kernel = wide ? uniform_walk_flat_kernel<kGen, kEdges, OutT, int64_t>
+                        : uniform_walk_flat_kernel<kGen, kEdges, OutT, int32_t>;
+    if (int rc = record_walk_event(0, stream)) return rc;
+    // a launch holds fewer than 2^32 work-items
+    constexpr int64_t kMostBlocks = int64_t{UINT32_MAX} / kWave;
+    for (int64_t b = 0; b < f.blocks; b += kMostBlocks) {
+        const int64_t n = b * f.per_wave;  // the launch's first walk
+        WalkArgs part = a;
+        part.start += n;
+        if (!kGen) part.rand += n * a.walk_length;
+        part.n_out = static_cast<OutT*>(a.n_out) + n * (static_cast<int64_t>(a.walk_length) + 1);
+        if (kEdges) part.e_out = static_cast<OutT*>(a.e_out) + n * a.walk_length;
+        part.num_walks -= n;
+        part.walk_base += n;
+        const int64_t blocks = f.blocks - b < kMostBlocks ? f.blocks - b : kMostBlocks;
+        part.num_walks = blocks * f.per_wave < part.num_walks ? blocks * f.per_wave : part.num_walks;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kWave), lds, stream,
+                           part, f.per_wave, f.steps);
+        MLXC_HIP_TRY(hipGetLastError());
+    }
+    return record_walk_event(1, stream);
 }
 
 }  // namespace

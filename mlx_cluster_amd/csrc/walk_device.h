@@ -201,8 +201,8 @@ struct RandWindow {
 };
 
 // First index of the rand block that serves rand[f]: the aligned block, or for
-// the array's last partial block the last RW values (total must be a multiple
-// of 4 and at least RW, so every block is 16-byte aligned and in bounds).
+// the array's last partial block the last RW values (total is at least RW, so
+// every block is in bounds; 4-byte aligned, which is all a 16-byte load needs).
 template <int RW>
 __device__ __forceinline__ int64_t rw_block_base(int64_t f, int64_t total) {
     const int64_t base = f & ~static_cast<int64_t>(RW - 1);
@@ -212,7 +212,7 @@ __device__ __forceinline__ int64_t rw_block_base(int64_t f, int64_t total) {
 template <int RW>
 __device__ __forceinline__ void rw_load_at(RandWindow<RW>& r, const float* __restrict__ rand,
                                            int64_t base) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
     const f32x4* p = reinterpret_cast<const f32x4*>(rand + base);
 #pragma unroll
     for (int i = 0; i < RW / 4; ++i) {

@@ -142,6 +142,10 @@ int launch_philox_fill(float* out, int64_t n, uint64_t seed, hipStream_t stream)
 // ---- uniform_walk.hip
 size_t uniform_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
                                int32_t walk_length);
+// The workspace whose walk is the fastest for the call (see
+// mlxc_random_walk_preferred_bytes).
+size_t uniform_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
+                               int32_t walk_length);
 // generate: the kernels compute their uniforms from the Philox key in a
 // (key0, key1) instead of reading a.rand.  out_type: MLXC_OUT_* of a.n_out
 // and a.e_out.

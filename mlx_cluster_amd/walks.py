@@ -522,7 +522,7 @@ def random_walk(rowptr: TensorLike, col: TensorLike, start: TensorLike,
 
     n_out, e_out = _run_walks(
         device, stream, handle, N, L, out_dtype, return_edges,
-        lambda n: lib.mlxc_random_walk_workspace_bytes(V, E, n, L), launch, budget, check,
+        lambda n: lib.mlxc_random_walk_preferred_bytes(V, E, n, L), launch, budget, check,
         "random_walk", (rowptr, col, start, rand))
     return (n_out, e_out) if return_edges else n_out
 

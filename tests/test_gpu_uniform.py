@@ -638,3 +638,47 @@ def test_graph_beyond_int32_edge_ids(cuda):
     assert torch.equal(n2, n) and torch.equal(e2, e)
     del col, n, e, n2, e2
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("N,L", [(1, 0), (3, 1), (2049, 31), (2049, 32), (2049, 33), (4097, 65),
+                                 (70_001, 7), (131_073, 33), (131_137, 34)])
+@pytest.mark.parametrize("seeded", [False, True])
+def test_flat_walk_edges(N, L, seeded, cuda):
+    """The flat walk (a workspace of the status words alone) around its
+    wavefront, stretch and spread limits, from buffers at every alignment of
+    their type, with sinks and with walk offsets; nothing outside the outputs
+    is written.  The same call with a workspace for start records (the CSR
+    walk, whose rand may start and end at any float) gives the same walks."""
+    from mlx_cluster_amd import _lib
+    lib = _lib.load()
+    rowptr, col = synth.rmat_csr(12, 30_000, seed=N + L, device=cuda)   # a third are sinks
+    V, E = rowptr.numel() - 1, col.numel()
+    start = (torch.arange(N, device=cuda) * 11) % V
+    offset = 5 if seeded else 0
+    rand = mc.philox_uniform((N + offset, L), 9, device=cuda)[offset:].reshape(-1)
+    n_ref, e_ref, st, _ = oracle.uniform_walk(rowptr.cpu().numpy(), col.cpu().numpy(),
+                                              start.cpu().numpy(),
+                                              rand.cpu().numpy().reshape(N, L), L,
+                                              with_edges=True)
+    assert st == 0
+    for dtype, shift in ((torch.int64, 0), (torch.int64, 1), (torch.int32, 3)):
+        out_type = _lib.MLXC_OUT_INT32 if dtype == torch.int32 else _lib.MLXC_OUT_INT64
+        r = torch.zeros(rand.numel() + 8, device=cuda)
+        r[shift:shift + rand.numel()] = rand
+        for ws_bytes in (32, 256 + 16 * N):
+            nb = torch.full((N * (L + 1) + 8,), -7, dtype=dtype, device=cuda)
+            eb = torch.full((N * L + 8,), -7, dtype=dtype, device=cuda)
+            # the CSR walk stores its outputs from 16-byte boundaries
+            at = shift if ws_bytes == 32 else 0
+            ws = torch.full((ws_bytes // 8,), 3, dtype=torch.int64, device=cuda)
+            graph = (rowptr.data_ptr(), V, col.data_ptr(), E, start.data_ptr(), N)
+            tail = (nb[at:].data_ptr(), eb[at:].data_ptr(), out_type, ws.data_ptr(), ws_bytes,
+                    torch.cuda.current_stream().cuda_stream)
+            rc = (lib.mlxc_random_walk_seeded(*graph, L, 9, offset, *tail) if seeded else
+                  lib.mlxc_random_walk(*graph, r[shift:].data_ptr(), L, *tail))
+            assert rc == 0 and int(ws[0]) == 0
+            n, e = nb.cpu().numpy(), eb.cpu().numpy()
+            np.testing.assert_array_equal(n[at:at + N * (L + 1)], n_ref.reshape(-1).astype(n.dtype))
+            np.testing.assert_array_equal(e[at:at + N * L], e_ref.reshape(-1).astype(e.dtype))
+            assert (n[:at] == -7).all() and (n[at + N * (L + 1):] == -7).all()
+            assert (e[:at] == -7).all() and (e[at + N * L:] == -7).all()
