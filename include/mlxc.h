@@ -154,6 +154,15 @@ size_t mlxc_rejection_sampling_workspace_bytes(int64_t num_nodes, int64_t num_ed
                                                int64_t num_walks, int32_t walk_length,
                                                double p, double q, int32_t rule);
 
+/* Workspace bytes with which mlxc_rejection_sampling is fastest for these
+ * arguments: 2 * MLXC_WORK_WORDS * 8, which selects the few-walks kernel (a
+ * group of lanes per walk on the CSR arrays as they are; up to 65,536 walks),
+ * in calls of few walks, else what mlxc_rejection_sampling_workspace_bytes
+ * returns.  No reference counterpart. */
+size_t mlxc_rejection_sampling_preferred_bytes(int64_t num_nodes, int64_t num_edges,
+                                               int64_t num_walks, int32_t walk_length,
+                                               double p, double q, int32_t rule);
+
 /* Layouts of mlxc_rejection_sampling, smallest first.  The call runs the
  * largest one its workspace holds, with the same results every way. */
 #define MLXC_N2V_LAYOUT_DIRECT 0        /* MLXC_WORK_WORDS words: the direct CSR kernel */

@@ -59,6 +59,7 @@ SIGNATURES = {
     "mlxc_random_walk_workspace_bytes": (_size, [_i64, _i64, _i64, _i32]),
     "mlxc_random_walk_preferred_bytes": (_size, [_i64, _i64, _i64, _i32]),
     "mlxc_rejection_sampling_workspace_bytes": (_size, [_i64, _i64, _i64, _i32, _dbl, _dbl, _i32]),
+    "mlxc_rejection_sampling_preferred_bytes": (_size, [_i64, _i64, _i64, _i32, _dbl, _dbl, _i32]),
     "mlxc_rejection_sampling_layout_bytes": (_size, [_i64, _i64, _i64, _i32, _i32]),
     "mlxc_random_walk": (
         ctypes.c_int,

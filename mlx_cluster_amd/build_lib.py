@@ -127,8 +127,8 @@ def _code_only(text: str) -> str:
 # walk_host.h is in every family: its constants (records_fit,
 # kSmallGraphEdgesPerStep) choose which kernels a call runs.
 KERNEL_SOURCES = {
-    "uniform_walk": ["walk_device.h", "walk_host.h", "prep_kernels.hip", "uniform_walk.hip"],
-    "node2vec_walk": ["walk_device.h", "walk_host.h", "prep_kernels.hip", "node2vec_walk.hip"],
+    "uniform_walk": ["walk_device.h", "walk_host.h", "csr_check.h", "prep_kernels.hip", "uniform_walk.hip"],
+    "node2vec_walk": ["walk_device.h", "walk_host.h", "csr_check.h", "prep_kernels.hip", "node2vec_walk.hip"],
     "csr_build": ["walk_device.h", "walk_host.h", "block_sort.h", "csr_build.hip"],
     "context_windows": ["walk_device.h", "walk_host.h", "windows.hip"],
     # the probe's kernel uses nothing from the walk headers (its launcher only

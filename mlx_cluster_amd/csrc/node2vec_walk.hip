@@ -3,6 +3,7 @@
 #include <cmath>
 #include <limits>
 
+#include "csr_check.h"
 #include "walk_host.h"
 
 namespace mlxc {
@@ -686,6 +687,271 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
         wave_sync();
         live = __popcll(keep);
     }
+}
+
+// node2vec walk of a call of few walks, on the CSR arrays as they are (any
+// graph, any alignment): each walk on a group of `group` lanes.
+//
+// Bound by the latency of each walk's chain of dependent reads, so the lanes
+// of a group shorten the chain: they read the candidates of consecutive
+// trials of the walk's step at once, then the rows that the undecided and the
+// accepted of those trials need at once, and search an undecided trial's row
+// together, a read narrowing it (lanes + 1)-fold.  The step takes the first
+// trial, in trial order, that accepts or meets a malformed entry, as one
+// lane trying them in turn would have.  Outputs are kept in LDS over a
+// stretch of `steps` positions and stored together, as in the uniform flat
+// walk.
+//
+// The call must validate the whole graph.  The walk does not wait for that:
+// blocks from walk_blocks on check the CSR beside it (the walk bounds every
+// index it uses itself).  Only the row order of MLXC_ROWS_DETECT matters to
+// it: it assumes sorted rows, and a second launch (rerun) repeats the walks
+// with scans when the check has found otherwise.
+//
+// Measured (us a call, symmetrized R-MAT, 40 steps, p = 0.5, q = 2, chain rule;
+// before: the record walk's tail phase or its queue, after the preparation
+// passes):  31 M entries: 1,300 walks 361 -> 165 (the check of the 251 MB of
+// col alone takes 60), 8,000 401 -> 228, 32,768 653 -> 386, 65,536
+// 1,391 -> 607;  64 K entries: 1,300 walks 173 -> 103, 65,536 686 -> 332.
+// At 200,000 walks it is 15% ahead of the records over 31 M entries and up to
+// 14% behind them over 1 M: kN2VFewWalks.
+// Trials a group tries at once, and searches it runs at once, at most: 8 and
+// 32 trials, 1, 2 and 8 searches were within 5% or slower.
+constexpr int kFewTrials = 16;
+constexpr int kFewSearches = 4;
+
+// Whether tgt is in [lo, hi) of col: a search of sorted entries or a scan, by
+// the `lanes` lanes (a power of two, lane c of them) that share the arguments;
+// `bits` selects them in a ballot shifted down by their first lane.  Every
+// lane of the wavefront calls it (with lo == hi: no search).
+template <typename Id>
+__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, bool sorted, Id lo,
+                                           Id hi, Id tgt, int lanes, int c, int first,
+                                           uint64_t bits) {
+    bool found = false;
+    while (__any(lo < hi)) {
+        const Id n = hi - lo;
+        // sorted: probes at the ends of lanes + 1 equal parts, or every entry
+        // once they are no more than the lanes; unsorted: the next entries
+        const Id part = sorted && n > lanes ? (n + lanes) / (lanes + 1) : 1;
+        const Id at = lo + (c + 1) * part - 1;
+        const bool in = at < hi;
+        Id x = 0;
+        if (in) x = static_cast<Id>(col[at]);
+        const uint64_t eq = (__ballot(in && x == tgt) >> first) & bits;
+        const int below = __popcll((__ballot(in && x < tgt) >> first) & bits);
+        if (lo < hi) {
+            if (eq) {
+                found = true;
+                lo = hi;
+            } else if (sorted) {
+                if (part == 1 && n <= lanes) {
+                    lo = hi;
+                } else {
+                    // up to the first probe that is not below tgt
+                    const Id end = lo + (below + 1) * part - 1;
+                    lo += below * part;
+                    if (below < lanes && end < hi) hi = end;
+                }
+            } else {
+                lo = lo + lanes < hi ? lo + lanes : hi;
+            }
+        }
+    }
+    return found;
+}
+
+template <int kRule, bool kEdges, typename OutT, typename Id>
+__global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int group, int steps,
+                                                              int walk_blocks, bool rerun) {
+    const int64_t* const rowptr = a.w.rowptr;
+    const int64_t* const col = a.w.col;
+    if (!rerun && blockIdx.x >= static_cast<unsigned>(walk_blocks)) {
+        CsrCheck check;
+        const int64_t stride = static_cast<int64_t>(gridDim.x - walk_blocks) * kBlock;
+        const int64_t gid =
+            static_cast<int64_t>(blockIdx.x - walk_blocks) * kBlock + threadIdx.x;
+        if (reinterpret_cast<uintptr_t>(col) % 16 == 0)
+            check.edges4(col, a.w.num_nodes, a.w.num_edges, gid, stride);
+        else
+            for (int64_t i = gid; i < a.w.num_edges; i += stride)
+                check.edge(col, a.w.num_nodes, i, col[i]);
+        check.nodes(rowptr, a.w.num_nodes, col, a.w.num_edges, gid, stride);
+        unsigned long long* w = reinterpret_cast<unsigned long long*>(a.w.work);
+        check.flush(w, MLXC_STATUS_BAD_ROW, MLXC_STATUS_BAD_NODE, w + 2);
+        return;
+    }
+    if (rerun && a.w.work[2] == a.w.work[3]) return;  // the rows are sorted
+    const bool sorted = !rerun && a.rows != MLXC_ROWS_UNSORTED;
+    extern __shared__ __align__(16) unsigned char few_lds[];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int G = group, per_wave = kWave / G;
+    const int row = steps + 1;
+    Id* const nodes =
+        reinterpret_cast<Id*>(few_lds) + wave * per_wave * row * (kEdges ? 2 : 1);
+    Id* const edges = nodes + per_wave * row;
+    const int64_t L = a.w.walk_length;
+    const int64_t n0 =
+        (static_cast<int64_t>(blockIdx.x) * (kBlock / kWave) + wave) * per_wave;
+    const int64_t left = a.w.num_walks - n0;
+    if (left <= 0) return;
+    const int walks = left < per_wave ? static_cast<int>(left) : per_wave;
+    OutT* const nout = static_cast<OutT*>(a.w.n_out) + n0 * (L + 1);
+    OutT* const eout = kEdges ? static_cast<OutT*>(a.w.e_out) + n0 * L : nullptr;
+    const int w = lane / G, k = lane % G, base = lane & ~(G - 1);
+    const uint64_t group_bits = G == kWave ? ~0ull : (1ull << G) - 1;
+    const int tries = G < kFewTrials ? G : kFewTrials;
+    const uint64_t stream = static_cast<uint64_t>(a.w.walk_base + n0 + w);
+    uint32_t status = 0, trial = 0;
+    bool alive = w < walks;
+    Id v = 0, bv = 0, dv = 0, t = 0, bt = 0, dt = 0;  // this and the last node, their rows
+    if (alive) {
+        const int64_t s = a.w.start[n0 + w];
+        v = static_cast<Id>(s);
+        if (k == 0) nodes[w * row] = v;
+        if (!node_ok(s, a.w.num_nodes)) {
+            status |= MLXC_STATUS_BAD_NODE;
+            alive = false;
+        } else if (L > 0) {
+            const RowBounds rb = load_row(rowptr, v);
+            bv = static_cast<Id>(rb.begin);
+            dv = static_cast<Id>(rb.end - rb.begin);
+            if (!row_ok(rb, a.w.num_edges)) {
+                status |= MLXC_STATUS_BAD_ROW;
+                alive = false;
+            } else if (dv == 0) {
+                alive = false;  // absorbing start node
+            }
+        }
+    }
+    for (int64_t p0 = 0; p0 <= L; p0 += steps) {
+        const int len = L + 1 - p0 < steps ? static_cast<int>(L + 1 - p0) : steps;
+        int j = p0 == 0 ? 1 : 0;  // the walk's next position of the stretch
+        while (__any(alive && j < len)) {
+            const bool busy = alive && j < len;
+            const int64_t l = p0 + j - 1;       // this step
+            const bool sure = l == 0 || dv == 1;  // the first step, or a forced one
+            const uint32_t my = trial + static_cast<uint32_t>(k);
+            // trial `my`: 0 rejected, 1 accepted, 2 undecided, else 4 | the
+            // status bit of a malformed entry
+            uint32_t outcome = 0;
+            float r = 0.0f;
+            Id e = bv, x = 0, bx = 0, dx = 0;
+            if (busy && k < (sure ? 1 : tries) && my < MLXC_MAX_TRIALS) {
+                if (dv != 1) {  // (a forced step takes its only edge)
+                    float u0;
+                    n2v_uniforms(static_cast<int64_t>(stream), static_cast<int32_t>(l), my, a.key0,
+                                 a.key1, u0, r);
+                    e = bv + static_cast<Id>(pick_index(u0, dv));
+                }
+                const int64_t xc = col[e];
+                x = static_cast<Id>(xc);
+                const bool cap = my == MLXC_MAX_TRIALS - 1;  // the cap keeps the last candidate
+                // (ids are compared as the decision needs them: whether x is t)
+                const int d = sure ? 1 : n2v_decide<kRule>(a, r, x == t ? 0 : 1, 0);
+                if (!node_ok(xc, a.w.num_nodes)) {
+                    outcome = 4u | MLXC_STATUS_BAD_NODE;
+                } else if (d == 0 && !cap) {
+                    outcome = 0;
+                } else if (d != -1 && x == t && l > 0) {
+                    outcome = 1;  // back to t, whose row the walk keeps
+                    bx = bt;
+                    dx = dt;
+                } else {
+                    const RowBounds rb = load_row(rowptr, x);
+                    bx = static_cast<Id>(rb.begin);
+                    dx = static_cast<Id>(rb.end - rb.begin);
+                    if (!row_ok(rb, a.w.num_edges)) outcome = 4u | MLXC_STATUS_BAD_ROW;
+                    else if (d != -1 || cap) outcome = 1;
+                    else if (dx == 0) outcome = n2v_resolve<kRule>(a, r, false) ? 1 : 0;
+                    else outcome = 2;
+                }
+            }
+            // The first trial that is decided, and the undecided ones before it.
+            const uint64_t done = (__ballot(outcome == 1 || outcome >= 4) >> base) & group_bits;
+            uint64_t open = (__ballot(outcome == 2) >> base) & group_bits;
+            int f = done ? __builtin_ctzll(done) : kWave;  // (kWave: none)
+            if (f < kWave) open &= (1ull << f) - 1;
+            if (__any(open != 0)) {
+                // the row an undecided trial searches (n2v_search_rows), and for what
+                const bool other = a.symmetric && dt < dx;
+                const Id s_lo = other ? bt : bx, s_hi = s_lo + (other ? dt : dx);
+                const Id s_tgt = other ? x : t;
+                while (__any(open != 0)) {
+                    // up to kFewSearches of the group's undecided trials, in
+                    // trial order, on equal shares of its lanes
+                    const int m = __popcll(open);
+                    int Q = 1;
+                    while (Q < m && Q < kFewSearches && Q < G) Q *= 2;
+                    const int C = G / Q, q = k / C, c = k % C;
+                    uint64_t rest = open;
+                    for (int i = 0; i < q; ++i) rest &= rest - 1;
+                    const bool valid = rest != 0;
+                    const int src = base + (valid ? __builtin_ctzll(rest) : 0);
+                    const Id lo = __shfl(s_lo, src, kWave);
+                    const Id hi = __shfl(s_hi, src, kWave);
+                    const Id tgt = __shfl(s_tgt, src, kWave);
+                    const float rs = __shfl(r, src, kWave);
+                    const bool found =
+                        group_find(col, sorted, lo, valid ? hi : lo, tgt, C, c, base + q * C,
+                                   C == kWave ? ~0ull : (1ull << C) - 1);
+                    const bool acc = valid && c == 0 && n2v_resolve<kRule>(a, rs, found);
+                    const uint64_t won = (__ballot(acc) >> base) & group_bits;
+                    if (won) {
+                        f = __shfl(src, base + __builtin_ctzll(won), kWave) - base;
+                        open = 0;
+                    } else {
+                        for (int i = 0; i < Q; ++i) open &= open - 1;
+                    }
+                }
+            }
+            // the decided trial, from its lane
+            const int src = base + (f < kWave ? f : 0);
+            const uint32_t got = __shfl(outcome, src, kWave);
+            const Id xg = __shfl(x, src, kWave);
+            const Id eg = __shfl(e, src, kWave);
+            const Id bg = __shfl(bx, src, kWave);
+            const Id dg = __shfl(dx, src, kWave);
+            if (!busy) continue;
+            if (f == kWave) {
+                trial += static_cast<uint32_t>(tries);
+            } else if (got >= 4) {
+                status |= got & 3u;
+                alive = false;
+            } else {
+                if (k == 0) {
+                    nodes[w * row + j] = xg;
+                    if (kEdges) edges[w * row + j] = eg;
+                }
+                j += 1;
+                t = v;
+                bt = bv;
+                dt = dv;
+                v = xg;
+                bv = bg;
+                dv = dg;
+                trial = 0;
+                if (dv == 0) alive = false;  // absorbing node: the walk stays
+            }
+        }
+        wave_sync();
+        // a walk that stopped stays where it is
+        const int cells = walks * len;
+        for (int i0 = 0; i0 < cells; i0 += kWave) {
+            const int i = i0 + lane;
+            const int wi = i < cells ? i / len : 0, ji = i < cells ? i % len : 0;
+            const int got = __shfl(j, wi * G, kWave);
+            const Id stay = __shfl(v, wi * G, kWave);
+            if (i >= cells) continue;
+            nout[wi * (L + 1) + p0 + ji] =
+                static_cast<OutT>(ji < got ? nodes[wi * row + ji] : stay);
+            if (kEdges && p0 + ji > 0)
+                eout[wi * L + p0 - 1 + ji] =
+                    static_cast<OutT>(ji < got ? edges[wi * row + ji] : Id{-1});
+        }
+        wave_sync();
+    }
+    if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.w.work), static_cast<unsigned long long>(status));
 }
 
 // node2vec walk over edge records (num_nodes, num_edges below 2^31; n_out and
@@ -1495,6 +1761,21 @@ size_t node2vec_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t nu
     return search_width > 0.0 ? lay.total : lay.total_base;
 }
 
+// The few-walks kernel's workspace: the status words and as many more, so that
+// the status words alone still select the direct kernel.
+constexpr size_t kN2VFewBytes = 2 * MLXC_WORK_WORDS * sizeof(int64_t);
+constexpr int64_t kN2VFewWalks = 65536;  // see node2vec_few_kernel
+
+size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
+                                int32_t walk_length, double search_width) {
+    const size_t queried =
+        node2vec_workspace_bytes(num_nodes, num_edges, num_walks, walk_length, search_width);
+    if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0 ||
+        queried == kRecordOffset || num_walks > kN2VFewWalks)
+        return queried;
+    return kN2VFewBytes;
+}
+
 size_t node2vec_layout_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
                              int32_t walk_length, int32_t layout) {
     if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0) return 0;
@@ -1534,6 +1815,56 @@ int64_t n2v_hub_min_degree(const WalkArgs& w, const N2VParams& p) {
     if (d >= 1e18) return INT64_MAX;
     return d > static_cast<double>(kHubMinDegree) ? static_cast<int64_t>(std::ceil(d))
                                                   : kHubMinDegree;
+}
+
+// The few-walks kernel: groups as wide as keep the call within kFewLanes lanes
+// per compute unit (1,300 walks on 31 M entries: 200 us with 256, 168 with 512
+// and 1,024, 171 with 2,048; 32,768 walks: 909, 540, 386 and 500), and
+// kFewCheckBlocks blocks per compute unit that check the graph beside them
+// (16, 8 and 4 take more of the memory's time from the walks: 220, 206 and 203
+// us against 191 with 2; 1 is too few from 5 steps a walk down: 122 against
+// 89 us).
+constexpr int kFewLanes = 1024;
+constexpr int kFewCheckBlocks = 3;
+constexpr int kFewCells = 512;  // walks x positions of a wavefront's LDS stretch
+
+template <int kRule, bool kEdges, typename OutT, typename Id>
+int launch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
+    DeviceInfo info;
+    if (int rc = device_info(info)) return rc;
+    const int64_t N = a.w.num_walks, slots = static_cast<int64_t>(info.cus) * kFewLanes;
+    int G = 2;
+    while (G < kWave && 2 * G * N <= slots) G *= 2;
+    const int per_wave = kWave / G;
+    int64_t steps = kFewCells / per_wave;
+    if (steps > a.w.walk_length + int64_t{1}) steps = a.w.walk_length + int64_t{1};
+    const int64_t waves = (N + per_wave - 1) / per_wave;
+    const int walk_blocks = static_cast<int>((waves + kBlock / kWave - 1) / (kBlock / kWave));
+    int check_blocks = 0;
+    const int64_t quads = (a.w.num_edges + 3) / 4;
+    if (int rc = stream_grid(quads > a.w.num_nodes ? quads : a.w.num_nodes, kFewCheckBlocks,
+                             check_blocks))
+        return rc;
+    const size_t lds = static_cast<size_t>(kBlock / kWave) * per_wave * (steps + 1) *
+                       (kEdges ? 2 : 1) * sizeof(Id);
+    auto kernel = node2vec_few_kernel<kRule, kEdges, OutT, Id>;
+    if (int rc = record_walk_event(0, stream)) return rc;
+    hipLaunchKernelGGL(kernel, dim3(walk_blocks + check_blocks), dim3(kBlock), lds, stream, a, G,
+                       static_cast<int>(steps), walk_blocks, false);
+    MLXC_HIP_TRY(hipGetLastError());
+    if (a.rows == MLXC_ROWS_DETECT) {
+        hipLaunchKernelGGL(kernel, dim3(walk_blocks), dim3(kBlock), lds, stream, a, G,
+                           static_cast<int>(steps), walk_blocks, true);
+        MLXC_HIP_TRY(hipGetLastError());
+    }
+    return record_walk_event(1, stream);
+}
+
+template <int kRule, bool kEdges, typename OutT>
+int dispatch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
+    return records_fit(a.w.num_nodes, a.w.num_edges)
+               ? launch_n2v_few<kRule, kEdges, OutT, int32_t>(a, stream)
+               : launch_n2v_few<kRule, kEdges, OutT, int64_t>(a, stream);
 }
 
 template <typename OutT>
@@ -1679,6 +2010,24 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
         MLXC_HIP_TRY(hipGetLastError());
         return record_walk_event(1, stream);
     }
+    const bool edges = w.e_out != nullptr;
+    // The few-walks kernel: its workspace selects it.
+    if (workspace_bytes >= kN2VFewBytes && w.num_walks <= kN2VFewWalks) {
+        N2VRecArgs a{};
+        a.w = w;
+        a.rows = p.rows;
+        a.symmetric = p.symmetric;
+        a.thr0 = float_at_or_above(p.prob0);
+        a.thr1 = float_at_or_above(p.prob1);
+        a.thr2 = float_at_or_above(p.prob2);
+        a.key0 = p.key0;
+        a.key1 = p.key1;
+        if (p.rule == MLXC_RULE_REF_CHAIN)
+            return edges ? dispatch_n2v_few<MLXC_RULE_REF_CHAIN, true, OutT>(a, stream)
+                         : dispatch_n2v_few<MLXC_RULE_REF_CHAIN, false, OutT>(a, stream);
+        return edges ? dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, true, OutT>(a, stream)
+                     : dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, false, OutT>(a, stream);
+    }
     // Graphs beyond int32, a workspace too small for the records, or output
     // buffers not 16-byte aligned: the direct CSR kernel.  The CSR check
     // validates the whole graph as the other layouts do; csr_status_kernel
@@ -1695,7 +2044,6 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
     a.key0 = p.key0;
     a.key1 = p.key1;
     a.rows = p.rows;
-    const bool edges = w.e_out != nullptr;
     return p.rule == MLXC_RULE_REF_CHAIN
                ? dispatch_n2v<MLXC_RULE_REF_CHAIN, OutT>(a, edges, stream)
                : dispatch_n2v<MLXC_RULE_NODE2VEC_EXACT, OutT>(a, edges, stream);

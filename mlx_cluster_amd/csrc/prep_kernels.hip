@@ -1,5 +1,6 @@
 // Per-call preparation kernels: workspace reset, edge records, start
 // records, CSR validation and seeded uniform fills.
+#include "csr_check.h"
 #include "walk_host.h"
 
 namespace mlxc {
@@ -12,72 +13,6 @@ __global__ void zero_words_kernel(int64_t* p, int n) {
 __global__ void copy_word_kernel(const int64_t* src, int64_t* dst) {
     if (threadIdx.x == 0) *dst = *src;
 }
-
-__device__ __forceinline__ int64_t wave_sum(int64_t x) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) x += __shfl_xor(x, off, kWave);
-    return x;
-}
-
-__device__ __forceinline__ uint32_t wave_or(uint32_t x) {
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) x |= __shfl_xor(x, off, kWave);
-    return x;
-}
-
-// CSR validation, accumulated per thread and reduced per block.  Rows are
-// sorted iff every position i >= 1 with col[i] < col[i-1] starts a non-empty
-// row, i.e. iff desc == start_desc.
-struct CsrCheck {
-    bool bad_rowptr = false;  // rowptr[0] != 0, rowptr[V] != E, or decreasing
-    bool bad_col = false;     // a col value outside [0, V)
-    int64_t desc = 0;
-    int64_t start_desc = 0;
-
-    // node-parallel part: thread gid of a grid of `stride` threads
-    __device__ void nodes(const int64_t* rowptr, int64_t V, const int64_t* col, int64_t E,
-                          int64_t gid, int64_t stride) {
-        if (gid == 0 && (rowptr[0] != 0 || rowptr[V] != E)) bad_rowptr = true;
-        for (int64_t v = gid; v < V; v += stride) {
-            const int64_t rs = rowptr[v], re = rowptr[v + 1];
-            if (re < rs) bad_rowptr = true;
-            if (rs >= 1 && re > rs && re <= E && col[rs] < col[rs - 1]) ++start_desc;
-        }
-    }
-    // edge-parallel part: entry i holding c
-    __device__ void edge(const int64_t* col, int64_t V, int64_t i, int64_t c) {
-        if (!node_ok(c, V)) bad_col = true;
-        if (i >= 1 && c < col[i - 1]) ++desc;
-    }
-    // Adds the block's totals to the given words, one atomic each from
-    // thread 0: the status bits, and the descents that start no row
-    // (desc - start_desc, zero exactly when the rows are sorted) to
-    // diff_word.  Every thread of the block calls it.  (Atomics on one word
-    // serialize: three per wavefront, 49,000 per call, took 0.3 ms of the
-    // 0.42 ms pass over configuration 3's 31 M entries.)
-    __device__ void flush(unsigned long long* bits_word, uint32_t rowptr_bit, uint32_t col_bit,
-                          unsigned long long* diff_word) {
-        __shared__ uint32_t block_bits[kBlock / kWave];
-        __shared__ int64_t block_diff[kBlock / kWave];
-        const uint32_t bits = wave_or((bad_rowptr ? rowptr_bit : 0u) | (bad_col ? col_bit : 0u));
-        const int64_t d = wave_sum(desc - start_desc);
-        if (__lane_id() == 0) {
-            block_bits[threadIdx.x / kWave] = bits;
-            block_diff[threadIdx.x / kWave] = d;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            uint32_t b = 0;
-            int64_t t = 0;
-            for (int i = 0; i < kBlock / kWave; ++i) {
-                b |= block_bits[i];
-                t += block_diff[i];
-            }
-            if (b) atomicOr(bits_word, static_cast<unsigned long long>(b));
-            if (t) atomicAdd(diff_word, static_cast<unsigned long long>(t));
-        }
-    }
-};
 
 // Record of node v as the walks read it: {v, row begin, degree, 0}, with
 // degree kRecBadNode for an id outside [0, num_nodes) and kRecBadRow for a

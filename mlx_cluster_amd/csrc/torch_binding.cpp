@@ -168,7 +168,7 @@ py::object rejection_sampling(const at::Tensor& rowptr, const at::Tensor& col,
     const auto opts = at::TensorOptions().dtype(dtype).device(device);
     at::Tensor n_out = at::empty({N, L + 1}, opts);
     at::Tensor e_out = return_edges ? at::empty({N, L}, opts) : at::Tensor();
-    const size_t ws = mlxc_rejection_sampling_workspace_bytes(V, E, N, static_cast<int32_t>(L), p,
+    const size_t ws = mlxc_rejection_sampling_preferred_bytes(V, E, N, static_cast<int32_t>(L), p,
                                                               q, rule);
     at::Tensor work = at::empty({static_cast<int64_t>((ws + 7) / 8)},
                                 at::TensorOptions().dtype(at::kLong).device(device));

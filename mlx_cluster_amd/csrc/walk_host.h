@@ -165,6 +165,10 @@ struct N2VParams {
 double n2v_search_width(const N2VParams& p);
 size_t node2vec_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
                                 int32_t walk_length, double search_width);
+// The workspace whose walk is the fastest for the call (see
+// mlxc_rejection_sampling_preferred_bytes).
+size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
+                                int32_t walk_length, double search_width);
 // Bytes of one MLXC_N2V_LAYOUT_* layout (0: not available for this call).
 size_t node2vec_layout_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
                              int32_t walk_length, int32_t layout);

@@ -652,7 +652,7 @@ def rejection_sampling(rowptr: TensorLike, col: TensorLike, start: TensorLike,
 
     n_out, e_out = _run_walks(
         device, stream, handle, N, L, out_dtype, return_edges,
-        lambda n: lib.mlxc_rejection_sampling_workspace_bytes(V, E, n, L, p, q, rid), launch,
+        lambda n: lib.mlxc_rejection_sampling_preferred_bytes(V, E, n, L, p, q, rid), launch,
         budget, check, "rejection_sampling", (rowptr, col, start))
     return (n_out, e_out) if return_edges else n_out
 

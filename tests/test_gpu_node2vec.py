@@ -665,3 +665,77 @@ def test_row_hash_tables_overflow_and_size_limit(rule, cuda):
             c = np.concatenate([col[rowptr[v]:rowptr[v + 1]][::-1] for v in range(V)])
         assert_parity(r, c, start, 12, 0.5, 2.0, 99, rule, cuda, sorted_rows=sorted_rows,
                       rows_sorted=sorted_rows)
+
+
+@pytest.mark.parametrize("N,L", [(1, 0), (1, 70), (3, 513), (2048, 7), (2049, 17), (4100, 33),
+                                 (8193, 9), (16_385, 4), (32_769, 3), (65_536, 2),
+                                 (65_537, 2)])
+@pytest.mark.parametrize("rule", [0, 1])
+def test_few_walks_kernel(N, L, rule, cuda):
+    """The few-walks kernel (a workspace of twice the status words) at every
+    group width, around its stretch limits and past its walk limit (the
+    direct kernel): sorted rows given and detected, detected unsorted rows
+    (walked again with scans), the symmetric hint, walk offsets, both output
+    types from buffers at any alignment; nothing outside them is written."""
+    from mlx_cluster_amd import _lib
+    lib = _lib.load()
+    g = synth.rmat_csr(11, 20_000, seed=N + L, device=cuda, symmetrize=True)
+    d = synth.rmat_csr(11, 20_000, seed=N + L, device=cuda)   # with sinks
+    for (rowptr, col), p, q in ((g, 0.5, 2.0), (g, 4.0, 0.25), (d, 0.25, 3.0)):
+        V, E = rowptr.numel() - 1, col.numel()
+        shuffled = col.clone()
+        rp = rowptr.tolist()
+        for v in range(0, V, 3):
+            shuffled[rp[v]:rp[v + 1]] = col[rp[v]:rp[v + 1]].flip(0)
+        start = (torch.arange(N, device=cuda) * 13) % V
+        cases = [(col, _lib.MLXC_ROWS_SORTED, torch.int64, 0),
+                 (col, _lib.MLXC_ROWS_DETECT, torch.int32, 1),
+                 (shuffled, _lib.MLXC_ROWS_DETECT, torch.int64, 1),
+                 (shuffled, _lib.MLXC_ROWS_UNSORTED, torch.int32, 3)]
+        if rowptr is g[0]:
+            cases.append((col, _lib.MLXC_ROWS_DETECT | _lib.MLXC_ROWS_SYMMETRIC, torch.int64, 0))
+        for c, rows, dtype, shift in cases:
+            n_ref, e_ref, st, _ = oracle.node2vec_walk(
+                rowptr.cpu().numpy(), c.cpu().numpy(), start.cpu().numpy(), L, p, q, 21, rule=rule,
+                rows_sorted=c is col, with_edges=True, first_walk=7)
+            assert st == 0
+            nb = torch.full((N * (L + 1) + 8,), -7, dtype=dtype, device=cuda)
+            eb = torch.full((N * L + 8,), -7, dtype=dtype, device=cuda)
+            ws = torch.full((8,), 5, dtype=torch.int64, device=cuda)
+            rc = lib.mlxc_rejection_sampling(
+                rowptr.data_ptr(), V, c.data_ptr(), E, start.data_ptr(), N, L, p, q, 21, 7, rule,
+                rows, nb[shift:].data_ptr(), eb[shift:].data_ptr(),
+                _lib.MLXC_OUT_INT32 if dtype == torch.int32 else _lib.MLXC_OUT_INT64,
+                ws.data_ptr(), 64, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0 and int(ws[0]) == 0
+            n, e = nb.cpu().numpy(), eb.cpu().numpy()
+            np.testing.assert_array_equal(n[shift:shift + N * (L + 1)],
+                                          n_ref.reshape(-1).astype(n.dtype))
+            np.testing.assert_array_equal(e[shift:shift + N * L], e_ref.reshape(-1).astype(e.dtype))
+            assert (n[:shift] == -7).all() and (n[shift + N * (L + 1):] == -7).all()
+            assert (e[:shift] == -7).all() and (e[shift + N * L:] == -7).all()
+
+
+def test_few_walks_kernel_reports_malformed_graphs(cuda):
+    """Bad entries that no walk reads are reported too (the check beside the
+    walks), as are bad starts; every walk still ends."""
+    from mlx_cluster_amd import _lib
+    lib = _lib.load()
+    rowptr, col = synth.rmat_csr(12, 60_000, seed=3, device=cuda, symmetrize=True)
+    V, E = rowptr.numel() - 1, col.numel()
+    for what, bits in (("col", _lib.MLXC_STATUS_BAD_NODE), ("rowptr", _lib.MLXC_STATUS_BAD_ROW),
+                       ("start", _lib.MLXC_STATUS_BAD_NODE)):
+        rp, cl, start = rowptr.clone(), col.clone(), torch.arange(1300, device=cuda)
+        if what == "col":
+            cl[E - 1] = V
+        elif what == "rowptr":
+            rp[V] = E - 1
+        else:
+            start[77] = -1
+        n = torch.empty((1300, 21), dtype=torch.int64, device=cuda)
+        ws = torch.zeros(8, dtype=torch.int64, device=cuda)
+        rc = lib.mlxc_rejection_sampling(rp.data_ptr(), V, cl.data_ptr(), E, start.data_ptr(), 1300,
+                                         20, 0.5, 2.0, 1, 0, 0, _lib.MLXC_ROWS_DETECT,
+                                         n.data_ptr(), None, _lib.MLXC_OUT_INT64, ws.data_ptr(),
+                                         64, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and int(ws[0]) == bits, what
