@@ -448,6 +448,15 @@ int mlxc_rejection_sampling_cpu(const int64_t* rowptr, int64_t num_nodes,
 int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream);
 
 /*
+ * Makes the calling thread's walk calls publish their status themselves, as
+ * mlxc_publish_status after each of them would, into h_status (as there; the
+ * caller zeroes h_status[0] before each call), until it is set to NULL.  Small
+ * calls save a launch that way: the one that gathers their blocks' status bits
+ * publishes them too.  No reference counterpart.
+ */
+int mlxc_set_status_target(int64_t* h_status);
+
+/*
  * Measurement hook: times the walk kernel alone, without the preparation
  * launches before it (a call's last launch is its walk kernel).  After
  * mlxc_set_walk_events(start_event, stop_event), with two hipEvent_t handles

@@ -21,6 +21,7 @@ thread_local std::string g_last_error;
 }
 
 thread_local hipEvent_t g_walk_events[2] = {nullptr, nullptr};
+thread_local StatusTarget g_status_target = {nullptr, false};
 
 int fail(int code, const std::string& msg) {
     g_last_error = msg;
@@ -224,17 +225,65 @@ HostWalk host_walk(const int64_t* rowptr, int64_t num_nodes, const int64_t* col,
                     static_cast<uint32_t>(seed >> 32), first_walk};
 }
 
-// The status word of a call (workspace word 0) into host memory, then the
-// flag that it is there: system-scope stores, the flag's with release order.
+// The status word of a call into host memory, then the flag that it is
+// there: system-scope stores, the flag's with release order.
+__device__ __forceinline__ void publish(int64_t bits, int64_t* h_status) {
+    __hip_atomic_store(h_status + 1, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(h_status, int64_t{1}, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void publish_status_kernel(const int64_t* work, int64_t* h_status) {
+    if (threadIdx.x == 0) publish(work[0], h_status);
+}
+
+// See launch_finish; h_status may be null.
+__global__ __launch_bounds__(kBlock) void finish_kernel(const uint32_t* __restrict__ block_status,
+                                                        int blocks, int64_t* __restrict__ work,
+                                                        int64_t* h_status) {
+    uint32_t bits = 0;
+    for (int i = threadIdx.x; i < blocks; i += kBlock) bits |= block_status[i];
+    const bool node = __syncthreads_or(bits & MLXC_STATUS_BAD_NODE);
+    const bool row = __syncthreads_or(bits & MLXC_STATUS_BAD_ROW);
     if (threadIdx.x == 0) {
-        const int64_t bits = work[0];
-        __hip_atomic_store(h_status + 1, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(h_status, int64_t{1}, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        const int64_t all = (node ? MLXC_STATUS_BAD_NODE : 0) | (row ? MLXC_STATUS_BAD_ROW : 0);
+        work[0] = all;
+        for (int i = 1; i < MLXC_WORK_WORDS; ++i) work[i] = 0;
+        if (h_status) publish(all, h_status);
     }
 }
 
+// Device address of host words the device can write, or null.
+int64_t* device_words(int64_t* h_status) {
+    int64_t* d = nullptr;
+    if (hipHostGetDevicePointer(reinterpret_cast<void**>(&d), h_status, 0) != hipSuccess) {
+        (void)hipGetLastError();  // not left for the next call's launch check
+        return nullptr;
+    }
+    return d;
+}
+
+// The last step of a walk call (rc: how it went so far): publishes its status
+// word if the thread has a target and the call's own launches have not.
+int end_walk(int rc, const int64_t* d_work, hipStream_t s) {
+    const bool done = g_status_target.done;
+    g_status_target.done = false;
+    if (rc != MLXC_OK || !g_status_target.words || done) return rc;
+    hipLaunchKernelGGL(publish_status_kernel, dim3(1), dim3(kWave), 0, s, d_work,
+                       g_status_target.words);
+    MLXC_HIP_TRY(hipGetLastError());
+    return MLXC_OK;
+}
+
 }  // namespace
+
+int launch_finish(const uint32_t* block_status, int64_t blocks, int64_t* work, hipStream_t stream) {
+    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(kBlock), 0, stream, block_status,
+                       static_cast<int>(blocks), work, g_status_target.words);
+    MLXC_HIP_TRY(hipGetLastError());
+    g_status_target.done = g_status_target.words != nullptr;
+    return MLXC_OK;
+}
+
 }  // namespace mlxc
 
 using namespace mlxc;
@@ -249,16 +298,26 @@ int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream
     if (int rc = check_workspace(d_workspace, MLXC_WORK_WORDS * sizeof(int64_t))) return rc;
     if (!h_status || reinterpret_cast<uintptr_t>(h_status) % 8 != 0)
         return fail(MLXC_ERR_INVALID_ARGUMENT, "h_status must be 8-byte aligned host memory");
-    int64_t* d_status = nullptr;  // the device's address of the host words
-    if (hipHostGetDevicePointer(reinterpret_cast<void**>(&d_status), h_status, 0) != hipSuccess) {
-        (void)hipGetLastError();  // not left for the next call's launch check
+    int64_t* d_status = device_words(h_status);
+    if (!d_status)
         return fail(MLXC_ERR_INVALID_ARGUMENT,
                     "h_status is not host memory the device can write (hipHostMalloc)");
-    }
     hipLaunchKernelGGL(publish_status_kernel, dim3(1), dim3(kWave), 0,
                        static_cast<hipStream_t>(stream), static_cast<const int64_t*>(d_workspace),
                        d_status);
     MLXC_HIP_TRY(hipGetLastError());
+    return MLXC_OK;
+}
+
+int mlxc_set_status_target(int64_t* h_status) {
+    g_status_target = {nullptr, false};
+    if (!h_status) return MLXC_OK;
+    if (reinterpret_cast<uintptr_t>(h_status) % 8 != 0)
+        return fail(MLXC_ERR_INVALID_ARGUMENT, "h_status must be 8-byte aligned host memory");
+    g_status_target.words = device_words(h_status);
+    if (!g_status_target.words)
+        return fail(MLXC_ERR_INVALID_ARGUMENT,
+                    "h_status is not host memory the device can write (hipHostMalloc)");
     return MLXC_OK;
 }
 
@@ -318,10 +377,11 @@ int mlxc_random_walk(const int64_t* d_rowptr, int64_t num_nodes, const int64_t* 
         return fail(MLXC_ERR_INVALID_ARGUMENT, "rand must not be NULL");
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t* d_work = static_cast<int64_t*>(d_workspace);
-    if (num_walks == 0) return launch_zero_work(d_work, s);  // (else the walk's launches zero it)
+    if (num_walks == 0)  // (else the walk's launches reset the words)
+        return end_walk(launch_zero_work(d_work, s), d_work, s);
     const WalkArgs a{d_rowptr, d_col, d_start, d_rand, d_n_out, d_e_out, d_work,
                      num_nodes, num_edges, num_walks, walk_length, 0u, 0u, 0};
-    return launch_uniform(a, d_workspace, workspace_bytes, false, out_type, s);
+    return end_walk(launch_uniform(a, d_workspace, workspace_bytes, false, out_type, s), d_work, s);
 }
 
 int mlxc_random_walk_noalloc(const int64_t* d_rowptr, int64_t num_nodes, const int64_t* d_col,
@@ -364,11 +424,12 @@ int mlxc_random_walk_seeded(const int64_t* d_rowptr, int64_t num_nodes, const in
     if (int rc = check_first_walk(first_walk, num_walks, walk_length)) return rc;
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t* d_work = static_cast<int64_t*>(d_workspace);
-    if (num_walks == 0) return launch_zero_work(d_work, s);  // (else the walk's launches zero it)
+    if (num_walks == 0)  // (else the walk's launches reset the words)
+        return end_walk(launch_zero_work(d_work, s), d_work, s);
     const WalkArgs a{d_rowptr, d_col, d_start, nullptr, d_n_out, d_e_out, d_work,
                      num_nodes, num_edges, num_walks, walk_length,
                      static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32), first_walk};
-    return launch_uniform(a, d_workspace, workspace_bytes, true, out_type, s);
+    return end_walk(launch_uniform(a, d_workspace, workspace_bytes, true, out_type, s), d_work, s);
 }
 
 int mlxc_rejection_sampling(const int64_t* d_rowptr, int64_t num_nodes, const int64_t* d_col,
@@ -386,11 +447,11 @@ int mlxc_rejection_sampling(const int64_t* d_rowptr, int64_t num_nodes, const in
     prm.out_type = out_type;
     hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t* d_work = static_cast<int64_t*>(d_workspace);
-    if (int rc = launch_zero_work(d_work, s)) return rc;
-    if (num_walks == 0) return MLXC_OK;
+    if (num_walks == 0)  // (else the walk's launches reset the words)
+        return end_walk(launch_zero_work(d_work, s), d_work, s);
     const WalkArgs a{d_rowptr, d_col, d_start, nullptr, d_n_out, d_e_out, d_work,
                      num_nodes, num_edges, num_walks, walk_length, 0u, 0u, first_walk};
-    return launch_node2vec(a, prm, d_workspace, workspace_bytes, s);
+    return end_walk(launch_node2vec(a, prm, d_workspace, workspace_bytes, s), d_work, s);
 }
 
 int mlxc_csr_check(const int64_t* d_rowptr, int64_t num_nodes, const int64_t* d_col,

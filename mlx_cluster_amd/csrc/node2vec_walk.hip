@@ -1573,7 +1573,15 @@ __global__ __launch_bounds__(kLdsBlock) void node2vec_lds_kernel(N2VRecArgs a) {
         trial = 0;
         if (l == L || deg == 0) finish();  // (deg 0: an absorbing node, the walk stays)
     }
-    if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.w.work), static_cast<unsigned long long>(status));
+    if (a.w.block_status) {
+        const bool node = __syncthreads_or(status & MLXC_STATUS_BAD_NODE);
+        const bool row = __syncthreads_or(status & MLXC_STATUS_BAD_ROW);
+        if (threadIdx.x == 0)
+            a.w.block_status[blockIdx.x] =
+                (node ? MLXC_STATUS_BAD_NODE : 0u) | (row ? MLXC_STATUS_BAD_ROW : 0u);
+    } else if (status) {
+        atomicOr(reinterpret_cast<unsigned long long*>(a.w.work), static_cast<unsigned long long>(status));
+    }
 }
 
 // ------------------------------------------------------------- launcher
@@ -1770,10 +1778,15 @@ size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t nu
                                 int32_t walk_length, double search_width) {
     const size_t queried =
         node2vec_workspace_bytes(num_nodes, num_edges, num_walks, walk_length, search_width);
-    if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0 ||
-        queried == kRecordOffset || num_walks > kN2VFewWalks)
-        return queried;
-    return kN2VFewBytes;
+    if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0) return queried;
+    if (queried == kRecordOffset) {
+        // the LDS walk, with a status word for each of its blocks (at most one
+        // a compute unit) where that is not yet the workspace of another layout
+        const size_t with_words = kRecordOffset + 256 * sizeof(uint32_t);
+        const size_t csr = n2v_layout(num_nodes, num_edges, num_walks, false).total;
+        return with_words < csr ? with_words : queried;
+    }
+    return num_walks > kN2VFewWalks ? queried : kN2VFewBytes;
 }
 
 size_t node2vec_layout_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
@@ -1885,6 +1898,7 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
     const bool hub_bitmaps = hash_tables && lay_rec.hub_max > 0 && workspace_bytes >= lay_rec.total;
     if (aligned && records_fit(w.num_nodes, w.num_edges) &&
         (records || workspace_bytes >= lay_csr.total)) {
+        if (int rc = launch_zero_work(w.work, stream)) return rc;
         const N2VLayout& lay = records ? lay_rec : lay_csr;
         N2VRecArgs a;
         a.w = w;
@@ -1965,7 +1979,6 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
     // (it stores single elements: no alignment needed)
     if (workspace_bytes >= kRecordOffset &&
         lds_walk_fits(w.num_nodes, w.num_edges, w.num_walks, w.walk_length)) {
-        // (mlxc_rejection_sampling cleared the status words before this launch)
         N2VRecArgs a{};
         a.w = w;
         a.rows = p.rows;
@@ -1994,6 +2007,10 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
         int64_t threads = (lanes + blocks - 1) / blocks;
         threads = (threads + kWave - 1) / kWave * kWave;
         threads = threads < kLdsMinWalkers ? kLdsMinWalkers : threads > kLdsBlock ? kLdsBlock : threads;
+        if (workspace_bytes >= kRecordOffset + blocks * sizeof(uint32_t))
+            a.w.block_status = reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kRecordOffset);
+        else if (int rc = launch_zero_work(w.work, stream))
+            return rc;
         a.lds_group = G;
         a.lds_walkers = static_cast<int32_t>(threads / G);
         const dim3 grid(static_cast<unsigned>(blocks));
@@ -2008,11 +2025,13 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
             else hipLaunchKernelGGL((node2vec_lds_kernel<MLXC_RULE_NODE2VEC_EXACT, false, OutT>), grid, block, 0, stream, a);
         }
         MLXC_HIP_TRY(hipGetLastError());
-        return record_walk_event(1, stream);
+        if (int rc = record_walk_event(1, stream)) return rc;
+        return a.w.block_status ? launch_finish(a.w.block_status, blocks, w.work, stream) : MLXC_OK;
     }
     const bool edges = w.e_out != nullptr;
     // The few-walks kernel: its workspace selects it.
     if (workspace_bytes >= kN2VFewBytes && w.num_walks <= kN2VFewWalks) {
+        if (int rc = launch_zero_work(w.work, stream)) return rc;
         N2VRecArgs a{};
         a.w = w;
         a.rows = p.rows;
@@ -2033,6 +2052,7 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
     // validates the whole graph as the other layouts do; csr_status_kernel
     // turns its words into the call's status bits and the row order, on the
     // device.
+    if (int rc = launch_zero_work(w.work, stream)) return rc;
     if (int rc = launch_csr_check(w.rowptr, w.num_nodes, w.col, w.num_edges, w.work, stream))
         return rc;
     if (int rc = launch_csr_status(w.work, stream)) return rc;

@@ -54,35 +54,48 @@ int64_t* status_words() {
     return words;
 }
 
-// The status word of the call just enqueued on `stream`.  The device stores
-// it into this thread's host words (mlxc_publish_status) and the host waits
-// for the flag: spinning for up to about 200 us (the reference tests' calls
-// take tens), then in hipStreamSynchronize.  Without the host words, torch's
-// scalar read (a copy ordered on the stream, about 13 us more per call).
-int64_t read_status(const at::Tensor& work, hipStream_t stream) {
-    int64_t* h = status_words();
-    if (h) {
+// For a validated call: makes the library publish the call's status word into
+// the calling thread's host words (mlxc_set_status_target).
+class StatusTarget {
+public:
+    explicit StatusTarget(bool check) {
+        int64_t* h = check ? status_words() : nullptr;
+        if (!h) return;
         __atomic_store_n(&h[0], int64_t{0}, __ATOMIC_RELAXED);
-        if (mlxc_publish_status(work.data_ptr(), h, stream) == MLXC_OK) {
-            const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-            for (unsigned i = 1;; ++i) {
-                if (__atomic_load_n(&h[0], __ATOMIC_ACQUIRE)) return __atomic_load_n(&h[1], __ATOMIC_RELAXED);
-                __builtin_ia32_pause();
-                if (i % 64 == 0 && std::chrono::steady_clock::now() > until) break;
-            }
-            if (hipStreamSynchronize(stream) != hipSuccess)
-                throw std::runtime_error(std::string("hipStreamSynchronize: ") +
-                                         hipGetErrorString(hipGetLastError()));
+        if (mlxc_set_status_target(h) == MLXC_OK) words = h;
+    }
+    ~StatusTarget() {
+        if (words) mlxc_set_status_target(nullptr);
+    }
+    int64_t* words = nullptr;
+};
+
+// The status word of the call just enqueued on `stream`.  Its last launch
+// stores it into `h` and the host waits for the flag: spinning for up to about
+// 200 us (the reference tests' calls take tens), then in hipStreamSynchronize.
+// Without the host words, torch's scalar read (a copy ordered on the stream,
+// about 13 us more per call).
+int64_t read_status(const at::Tensor& work, hipStream_t stream, const int64_t* h) {
+    if (h) {
+        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        for (unsigned i = 1;; ++i) {
             if (__atomic_load_n(&h[0], __ATOMIC_ACQUIRE)) return __atomic_load_n(&h[1], __ATOMIC_RELAXED);
+            __builtin_ia32_pause();
+            if (i % 64 == 0 && std::chrono::steady_clock::now() > until) break;
         }
+        if (hipStreamSynchronize(stream) != hipSuccess)
+            throw std::runtime_error(std::string("hipStreamSynchronize: ") +
+                                     hipGetErrorString(hipGetLastError()));
+        if (__atomic_load_n(&h[0], __ATOMIC_ACQUIRE)) return __atomic_load_n(&h[1], __ATOMIC_RELAXED);
     }
     return work.select(0, 0).item<int64_t>();
 }
 
 // Waits for the call and raises ValueError for status bits, as walks.py's
 // check=True does.
-void check_status(const at::Tensor& work, hipStream_t stream, const char* what) {
-    const int64_t bits = read_status(work, stream);
+void check_status(const at::Tensor& work, hipStream_t stream, const int64_t* words,
+                  const char* what) {
+    const int64_t bits = read_status(work, stream, words);
     if (bits == 0) return;
     std::string msg = std::string(what) + ": ";
     if (bits & MLXC_STATUS_BAD_NODE) msg += "a start or col entry is outside [0, num_nodes)";
@@ -125,6 +138,7 @@ py::object random_walk(const at::Tensor& rowptr, const at::Tensor& col, const at
                                 at::TensorOptions().dtype(at::kLong).device(device));
     hipStream_t stream = at::hip::getCurrentHIPStream().stream();
     const int out_type = int32_out ? MLXC_OUT_INT32 : MLXC_OUT_INT64;
+    const StatusTarget target(check);
     int rc;
     if (rand)
         rc = mlxc_random_walk(
@@ -144,7 +158,7 @@ py::object random_walk(const at::Tensor& rowptr, const at::Tensor& col, const at
             return_edges && e_out.numel() ? e_out.data_ptr() : nullptr, out_type,
             work.data_ptr(), static_cast<size_t>(work.numel()) * 8, stream);
     if (rc != MLXC_OK) raise_code(rc, "random_walk");
-    if (check) check_status(work, stream, "random_walk");
+    if (check) check_status(work, stream, target.words, "random_walk");
     return outputs(n_out, e_out, return_edges);
 }
 
@@ -173,6 +187,7 @@ py::object rejection_sampling(const at::Tensor& rowptr, const at::Tensor& col,
     at::Tensor work = at::empty({static_cast<int64_t>((ws + 7) / 8)},
                                 at::TensorOptions().dtype(at::kLong).device(device));
     hipStream_t stream = at::hip::getCurrentHIPStream().stream();
+    const StatusTarget target(check);
     const int rc = mlxc_rejection_sampling(
         static_cast<const int64_t*>(data_or_null(rowptr)), V,
         static_cast<const int64_t*>(data_or_null(col)), E,
@@ -182,7 +197,7 @@ py::object rejection_sampling(const at::Tensor& rowptr, const at::Tensor& col,
         int32_out ? MLXC_OUT_INT32 : MLXC_OUT_INT64, work.data_ptr(),
         static_cast<size_t>(work.numel()) * 8, stream);
     if (rc != MLXC_OK) raise_code(rc, "rejection_sampling");
-    if (check) check_status(work, stream, "rejection_sampling");
+    if (check) check_status(work, stream, target.words, "rejection_sampling");
     return outputs(n_out, e_out, return_edges);
 }
 

@@ -9,7 +9,7 @@
 // kQueueChunk (64) walks, so lanes never idle while walks remain and the
 // kernel's tail is about one walk long; their grids are the device's resident
 // capacity.  Smaller calls run the flat walk, one walk a lane from start to
-// end, or, on graphs that fit LDS, the LDS walk.
+// end.
 #include <type_traits>
 
 #include "walk_host.h"
@@ -457,81 +457,6 @@ __global__ __launch_bounds__(kBlock) void uniform_walk_csr_kernel(WalkArgs a,
     if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
 }
 
-// Uniform walk on a graph small enough for LDS, for calls bound by launch
-// latency (the reference tests' Cora-sized workload): every block copies
-// rowptr and col, as int32, into its LDS, then runs one walk per thread with
-// no global random read at all.  Uniforms are read 8 at a time (one round
-// trip per 8 steps); outputs are stored entry by entry, which only small
-// calls can afford.  Out-of-range entries are marked -1 on the copy and flag
-// the call when a walk meets them, as in the other kernels.
-
-
-template <bool kGen, bool kEdges, typename OutT>
-__global__ __launch_bounds__(kLdsBlock) void uniform_walk_lds_kernel(WalkArgs a) {
-    __shared__ int32_t graph[kLdsGraphEntries];
-    const int64_t V = a.num_nodes, E = a.num_edges, N = a.num_walks, L = a.walk_length;
-    const int64_t goff = kGen ? a.walk_base * L : 0;  // stream position of uniform 0
-    int32_t* const rp = graph;          // rowptr, -1 for an entry outside [0, E]
-    int32_t* const cl = graph + V + 1;  // col, -1 for a value outside [0, V)
-    for (int64_t i = threadIdx.x; i <= V; i += kLdsBlock) {
-        const int64_t r = a.rowptr[i];
-        rp[i] = r >= 0 && r <= E ? static_cast<int32_t>(r) : -1;
-    }
-    for (int64_t i = threadIdx.x; i < E; i += kLdsBlock) {
-        const int64_t c = a.col[i];
-        cl[i] = node_ok(c, V) ? static_cast<int32_t>(c) : -1;
-    }
-    __syncthreads();
-    OutT* const nout = static_cast<OutT*>(a.n_out);
-    OutT* const eout = static_cast<OutT*>(a.e_out);
-    uint32_t status = 0;
-    for (int64_t n = static_cast<int64_t>(blockIdx.x) * kLdsBlock + threadIdx.x; n < N;
-         n += static_cast<int64_t>(gridDim.x) * kLdsBlock) {
-        const int64_t s = a.start[n];
-        OutT* const row = nout + n * (L + 1);
-        OutT* const erow = kEdges ? eout + n * L : nullptr;
-        row[0] = static_cast<OutT>(s);
-        int64_t l = 0;                    // steps taken
-        int32_t v = static_cast<int32_t>(s);
-        bool stop = !node_ok(s, V);       // a sink or an error ends the walk
-        if (stop) status |= MLXC_STATUS_BAD_NODE;
-        while (l < L && !stop) {
-            float r[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (l + j < L)
-                    r[j] = kGen ? philox_uniform_at(goff + n * L + l + j, a.key0, a.key1) : a.rand[n * L + l + j];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (stop || l >= L) break;
-                const int32_t b = rp[v], end = rp[v + 1];
-                if (b < 0 || end < b) {
-                    status |= MLXC_STATUS_BAD_ROW;
-                    stop = true;
-                } else if (end == b) {
-                    stop = true;  // absorbing node: the walk stays
-                } else {
-                    const int32_t e = b + static_cast<int32_t>(pick_index(r[j], end - b));
-                    const int32_t x = cl[e];
-                    if (x < 0) {
-                        status |= MLXC_STATUS_BAD_NODE;
-                        stop = true;
-                    } else {
-                        row[l + 1] = static_cast<OutT>(x);
-                        if (kEdges) erow[l] = static_cast<OutT>(e);
-                        v = x;
-                        l += 1;
-                    }
-                }
-            }
-        }
-        for (int64_t j = l + 1; j <= L; ++j) row[j] = static_cast<OutT>(v);  // the walk stays
-        if (kEdges)
-            for (int64_t j = l; j < L; ++j) erow[j] = static_cast<OutT>(-1);
-    }
-    if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
-}
-
 // Uniform walk over the CSR arrays as they are: one walk a lane, `per_wave`
 // walks a wavefront (a block), no queue, no workspace but the status words.
 // Any graph and any alignment.
@@ -579,14 +504,10 @@ __global__ __launch_bounds__(kWave) void uniform_walk_flat_kernel(WalkArgs a, in
     OutT* const nout = static_cast<OutT*>(a.n_out) + n0 * (L + 1);
     OutT* const eout = kEdges ? static_cast<OutT*>(a.e_out) + n0 * L : nullptr;
     uint32_t status = 0;
-    bool alive = false;
+    // the first stretch's uniforms are read beside the start, good or not
+    bool alive = lane < walks;
     int64_t v = 0;
-    if (lane < walks) {
-        v = a.start[n0 + lane];
-        nodes[lane * row] = static_cast<Slot>(v);
-        alive = node_ok(v, a.num_nodes);
-        if (!alive) status |= MLXC_STATUS_BAD_NODE;
-    }
+    if (alive) v = a.start[n0 + lane];
     // positions p0 .. p0 + len - 1 of the rows; the step into position p uses
     // uniform p - 1
     for (int64_t p0 = 0; p0 <= L; p0 += steps) {
@@ -626,6 +547,11 @@ __global__ __launch_bounds__(kWave) void uniform_walk_flat_kernel(WalkArgs a, in
                         nodes[w * row + j] =
                             float_slot<Slot>(__builtin_nontemporal_load(rand + w * L + j));
                 }
+            }
+            if (first && alive) {
+                nodes[lane * row] = static_cast<Slot>(v);
+                alive = node_ok(v, a.num_nodes);
+                if (!alive) status |= MLXC_STATUS_BAD_NODE;
             }
             wave_sync();
             for (int j = first; j < len && __any(alive); ++j) {
@@ -668,7 +594,12 @@ __global__ __launch_bounds__(kWave) void uniform_walk_flat_kernel(WalkArgs a, in
         }
         wave_sync();
     }
-    if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
+    if (a.block_status) {
+        status = wave_status(status);
+        if (lane == 0) a.block_status[blockIdx.x] = status;
+    } else if (status) {
+        atomicOr(reinterpret_cast<unsigned long long*>(a.work), static_cast<unsigned long long>(status));
+    }
 }
 
 // ------------------------------------------------------------- launcher
@@ -704,7 +635,7 @@ constexpr int32_t kLongWalk = 64;
 
 namespace {
 
-enum class UniformMode { kRecords, kCsr, kCsrWide, kLds, kFlat };
+enum class UniformMode { kRecords, kCsr, kCsrWide, kFlat };
 
 // Edge records cost one random read per edge to build; they pay off when the
 // call takes several steps per edge, or when the graph is small enough that
@@ -760,11 +691,6 @@ UniformMode uniform_mode(const WalkArgs& a, size_t workspace_bytes, bool gen) {
                workspace_bytes >= init_bytes(a.num_walks)) {
         return UniformMode::kCsrWide;  // 2^31 or more entries
     }
-    // the LDS walk reads rand and stores its outputs one element at a time:
-    // any alignment and length will do
-    if (workspace_bytes >= kRecordOffset &&
-        lds_walk_fits(a.num_nodes, a.num_edges, a.num_walks, a.walk_length))
-        return UniformMode::kLds;
     return UniformMode::kFlat;
 }
 
@@ -777,6 +703,12 @@ UniformMode uniform_mode(const WalkArgs& a, size_t workspace_bytes, bool gen) {
 constexpr int kFlatWaves = 8;
 constexpr int kFlatSteps = 33;
 constexpr int kFlatCells = 1024;  // walks x positions of a wavefront of few walks
+
+// Blocks of the flat walk that write their status bits to words of their own
+// (2,048 walks to 2^17 run in 2,048 blocks); more OR them into one word, which
+// a launch has to zero first.
+constexpr int64_t kFlatStatusBlocks = 2048;
+constexpr size_t kStatusBytes = MLXC_WORK_WORDS * sizeof(int64_t);
 
 struct FlatShape {
     int per_wave, steps;
@@ -837,7 +769,7 @@ size_t uniform_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t num
     if (!records_fit(num_nodes, num_edges))  // the wide CSR walk, while node ids fit int32
         return num_nodes <= INT32_MAX ? init_bytes(num_walks) : minimum;
     if (lds_walk_fits(num_nodes, num_edges, num_walks, walk_length))
-        return kRecordOffset;  // the LDS walk: its size selects it
+        return kRecordOffset;  // the flat walk
     return records_pay_off(num_edges, num_walks, walk_length)
                ? record_bytes(num_nodes, num_edges, num_walks)
                : init_bytes(num_walks);
@@ -846,13 +778,14 @@ size_t uniform_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t num
 size_t uniform_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
                                int32_t walk_length) {
     const size_t queried = uniform_workspace_bytes(num_nodes, num_edges, num_walks, walk_length);
-    if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0 ||
-        queried == kRecordOffset)  // the LDS walk
-        return queried;
+    if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0) return queried;
     const bool records = records_fit(num_nodes, num_edges) &&
                          records_pay_off(num_edges, num_walks, walk_length);
-    return flat_walk_pays(num_walks, walk_length, records) ? MLXC_WORK_WORDS * sizeof(int64_t)
-                                                           : queried;
+    if (queried != kRecordOffset && !flat_walk_pays(num_walks, walk_length, records)) return queried;
+    // the status words and one more word a block, of at most as many blocks as
+    // walks (less than the start records that select the other walks)
+    const int64_t blocks = num_walks < kFlatStatusBlocks ? num_walks : kFlatStatusBlocks;
+    return kStatusBytes + static_cast<size_t>(blocks) * sizeof(uint32_t);
 }
 
 namespace {
@@ -907,22 +840,19 @@ int launch_uniform_impl(const WalkArgs& a, void* workspace, size_t workspace_byt
                                   MLXC_CSR_SLOTS, MLXC_CSR_BLOCKS_PER_CU, a, stream,
                                   static_cast<const void*>(init));
     }
-    case UniformMode::kLds: {
-        if (int rc = launch_zero_work(a.work, stream)) return rc;
-        const int64_t blocks = (a.num_walks + kLdsBlock - 1) / kLdsBlock;  // at most 1024
-        if (int rc = record_walk_event(0, stream)) return rc;
-        hipLaunchKernelGGL((uniform_walk_lds_kernel<kGen, kEdges, OutT>), dim3(static_cast<int>(blocks)),
-                           dim3(kLdsBlock), 0, stream, a);
-        MLXC_HIP_TRY(hipGetLastError());
-        return record_walk_event(1, stream);
-    }
     case UniformMode::kFlat:
         break;
     }
     DeviceInfo info;
     if (int rc = device_info(info)) return rc;
-    if (int rc = launch_zero_work(a.work, stream)) return rc;
     const FlatShape f = flat_shape(a.num_walks, a.walk_length, info.cus);
+    uint32_t* const block_status =
+        workspace_bytes >= kStatusBytes + static_cast<size_t>(f.blocks) * sizeof(uint32_t) &&
+                f.blocks <= kFlatStatusBlocks
+            ? reinterpret_cast<uint32_t*>(static_cast<char*>(workspace) + kStatusBytes)
+            : nullptr;
+    if (!block_status)
+        if (int rc = launch_zero_work(a.work, stream)) return rc;
     const bool wide = !records_fit(a.num_nodes, a.num_edges);
     const size_t lds = static_cast<size_t>(f.per_wave) * (f.steps + 1) * (kEdges ? 2 : 1) *
                        (wide ? sizeof(int64_t) : sizeof(int32_t));
@@ -934,6 +864,7 @@ int launch_uniform_impl(const WalkArgs& a, void* workspace, size_t workspace_byt
     for (int64_t b = 0; b < f.blocks; b += kMostBlocks) {
         const int64_t n = b * f.per_wave;  // the launch's first walk
         WalkArgs part = a;
+        part.block_status = block_status;
         part.start += n;
         if (!kGen) part.rand += n * a.walk_length;
         part.n_out = static_cast<OutT*>(a.n_out) + n * (static_cast<int64_t>(a.walk_length) + 1);
@@ -946,7 +877,8 @@ int launch_uniform_impl(const WalkArgs& a, void* workspace, size_t workspace_byt
                            part, f.per_wave, f.steps);
         MLXC_HIP_TRY(hipGetLastError());
     }
-    return record_walk_event(1, stream);
+    if (int rc = record_walk_event(1, stream)) return rc;
+    return block_status ? launch_finish(block_status, f.blocks, a.work, stream) : MLXC_OK;
 }
 
 }  // namespace

@@ -171,7 +171,16 @@ struct WalkArgs {
     // of walk walk_base + n, so a call over any slice of a larger batch gives
     // that slice's walks.  Generated uniform streams only (0 with a rand tensor).
     int64_t walk_base;
+    // Flat and node2vec LDS walks: a word per block for its status bits, which
+    // launch_finish gathers (null: OR-ed into work[0], zeroed before).
+    uint32_t* block_status = nullptr;
 };
+
+// Status bits of the whole wavefront (every lane calls it).
+__device__ __forceinline__ uint32_t wave_status(uint32_t status) {
+    return (__any(status & MLXC_STATUS_BAD_NODE) ? MLXC_STATUS_BAD_NODE : 0u) |
+           (__any(status & MLXC_STATUS_BAD_ROW) ? MLXC_STATUS_BAD_ROW : 0u);
+}
 
 // ------------------------------------------------- stream windows
 

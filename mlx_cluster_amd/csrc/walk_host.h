@@ -34,6 +34,21 @@ inline int record_walk_event(int which, hipStream_t stream) {
     return MLXC_OK;
 }
 
+// Where the calling thread's walk calls publish their status word (device
+// address of the caller's host words; null: nowhere), and whether the call
+// in progress already has.
+struct StatusTarget {
+    int64_t* words;
+    bool done;
+};
+extern thread_local StatusTarget g_status_target;
+
+// A walk call's end when its blocks wrote their status bits to words of their
+// own: work[0] <- their OR (the other words 0), and the status published if
+// the thread has a target.  One launch in place of the reset before the walk
+// and the publication after it.
+int launch_finish(const uint32_t* block_status, int64_t blocks, int64_t* work, hipStream_t stream);
+
 struct DeviceInfo {
     int cus = 0;  // compute units of the current device
 };
