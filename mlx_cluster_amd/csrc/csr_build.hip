@@ -677,95 +677,256 @@ __global__ __launch_bounds__(kBlock) void csr_emit_kernel(Store keys,
 
 // ------------------------------------------------------------- small lists
 
-// The whole build of a small list in one launch: one block sorts the list's
-// keys (32 bits) in registers, drops repeats, and writes col, rowptr (a
-// binary search of the kept keys per row) and the words of `work`.
+// The whole build of a small list in two launches.  Every block reads the
+// whole list and keeps the keys (32 bits) of its own range, about
+// kSmallKeys of them, between splitters that all blocks take from the same
+// sample; it sorts them in registers (block_sort.h), drops repeats and stores
+// them.  How many keys lie below its range it has counted on the way, so no
+// block waits for another.  A key's place in the list breaks ties, so ranges
+// stay even however often a pair repeats.  The second launch writes col, and
+// rowptr by a binary search per row.
 //
-// Bound by its one compute unit's instruction rate (the network of
-// block_sort.h); the 16 launches of the radix passes on such a list each take
-// longer than their work.  10,556 pairs over 2,708 nodes: 16 launches of 74 us
-// in all -> one of 38 us, to_csr 92 -> 58 us.
-template <int kThreads>
-__global__ __launch_bounds__(kThreads) void csr_small_kernel(EdgeSrc src, int total, bool dedup,
-                                                             int64_t* __restrict__ rowptr,
-                                                             int64_t* __restrict__ col_out,
-                                                             int64_t* __restrict__ work) {
-    static_assert(kSortItems == kItems, "16 keys a thread");
-    __shared__ uint32_t lds[sort_lds_keys<kThreads>()];
-    __shared__ uint32_t last[kThreads];
-    __shared__ int64_t wtot[kThreads / kWave];
-    const int t = threadIdx.x, lane = t % kWave;
-    uint32_t key[kItems];
-    bool bad = false;
-    // a wavefront's 1,024 keys, 64 consecutive entries a slot
-    const int base = (t - lane) * kItems + lane;
-    load_slots<Keys32, Src::kBoth>(key, src, Keys32{}, base, kWave, total, bad);
-#pragma unroll
-    for (int s = 0; s < kItems; ++s)
-        if (base + s * kWave >= total) key[s] = ~0u;
-    const int any_bad = __syncthreads_or(bad);
-    block_sort<kThreads>(key, total, lds);
+// Bound by latencies: two loads and their use, a network of 55 stages in one
+// wavefront, the search's 10 dependent reads.  Radix passes need 16 to 19
+// launches for such a list.  10,556 pairs over 2,708 nodes: 74 us of radix
+// kernels, 38 us when one block sorted the whole list, now 23 + 7 us; to_csr
+// 92 -> 58 -> 50 us.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallKeys = 512;      // keys of a block's range, on average
+constexpr int kSmallSamples = 4;     // samples per range
+// Ranges at most.  Every block reads the whole list: to_csr of 88,648 pairs
+// takes 105 us (radix passes 116), of 131,072 138 us (117).
+constexpr int kSmallWays = 192;
+constexpr int64_t kSmallTotal = static_cast<int64_t>(kSmallWays) * kSmallKeys;
+constexpr int kSmallCap = kSmallThreads * kItems;  // keys a block sorts at once
+constexpr int kIndexBits = 17;
+static_assert(kSmallTotal <= (int64_t{1} << kIndexBits), "an entry's place fits its field");
 
-    // Keep the first of equal keys (dedup), in order.
-    last[t] = key[kItems - 1];
-    __syncthreads();
-    const uint32_t before = t > 0 ? last[t - 1] : 0u;
-    uint32_t keep = 0;
-#pragma unroll
-    for (int s = 0; s < kItems; ++s) {
-        const int i = t * kItems + s;
-        const uint32_t prev = s > 0 ? key[s > 0 ? s - 1 : 0] : before;
-        if (i < total && (!dedup || i == 0 || prev != key[s])) keep |= 1u << s;
+struct SmallRange {
+    int32_t base;         // where the range's keys start
+    int32_t kept;         // and how many there are
+    uint32_t first, last; // the smallest and the largest
+};
+
+// A fixed scramble of sample numbers.
+__host__ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
+    x ^= x >> 16;
+    x *= 0x7feb352du;
+    x ^= x >> 15;
+    x *= 0x846ca68bu;
+    return x ^ (x >> 16);
+}
+// Sample i of `count` of the n > 0 entries: one in each of `count` equal parts.
+__host__ __device__ __forceinline__ int sample_at(int i, int count, int n) {
+    const int a = static_cast<int>(static_cast<int64_t>(i) * n / count);
+    const int b = static_cast<int>(static_cast<int64_t>(i + 1) * n / count);
+    return a + (b > a ? static_cast<int>(mix32(i) % static_cast<uint32_t>(b - a)) : 0);
+}
+
+// Key of entry i with its place below it: distinct for every entry.
+__device__ __forceinline__ uint64_t placed_key(const EdgeSrc& src, int i, bool& bad) {
+    return (static_cast<uint64_t>(read_entry<Keys32, Src::kBoth>(src, Keys32{}, i, bad))
+            << kIndexBits) | static_cast<uint32_t>(i);
+}
+
+__global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
+    EdgeSrc src, int total, int ways, bool dedup, uint32_t* __restrict__ keys,
+    SmallRange* __restrict__ ranges, int64_t* __restrict__ work) {
+    static_assert(kSortItems == kItems, "16 keys a thread");
+    __shared__ uint32_t lds[sort_lds_keys<kSmallThreads>()];
+    __shared__ uint64_t sample[kSmallWays * kSmallSamples];
+    __shared__ uint32_t last[kSmallThreads];
+    __shared__ int64_t wtot[kSmallThreads / kWave];
+    __shared__ uint64_t ends[2];
+    __shared__ int count[2];  // keys taken, keys below the range
+    const int t = threadIdx.x, lane = t % kWave, b = blockIdx.x;
+    bool bad = false;
+    if (t == 0) {
+        ends[0] = 0;      // the first range starts below every key
+        ends[1] = ~0ull;  // the last one ends above them
+        count[0] = count[1] = 0;
     }
-    int64_t all;
-    int p = static_cast<int>(
-        block_exclusive_scan<kOpSum, kThreads>(__popc(keep), wtot, &all));
-#pragma unroll
-    for (int s = 0; s < kItems; ++s)
-        if ((keep >> s) & 1u) lds[p++] = key[s];
+    const int ns = ways * kSmallSamples;
+    uint64_t mine = 0;
+    if (t < ns) sample[t] = mine = placed_key(src, sample_at(t, ns, total), bad);
     __syncthreads();
-    const int n = static_cast<int>(all);
-    const uint32_t cmask = src.cbits == 0 ? 0u : ~0u >> (32 - src.cbits);
-    for (int j = t; j < n; j += kThreads) col_out[j] = static_cast<int64_t>(lds[j] & cmask);
-    // rowptr[r]: the kept keys of the rows before r, four rows a thread at a
-    // time so that their searches' reads overlap
-    constexpr int kRows = 4;
-    const int V = static_cast<int>(src.num_nodes);
-    for (int r0 = t; r0 <= V; r0 += kRows * kThreads) {
-        int lo[kRows];
+    // A sample's rank is its number among all of them; equal samples (lists
+    // shorter than the sample) by number.
+    if (t < ns) {
+        int rank = 0;
+        for (int j = 0; j < ns; ++j)
+            rank += sample[j] < mine || (sample[j] == mine && j < t);
+        if (b > 0 && rank == b * kSmallSamples) ends[0] = mine;
+        if (rank == (b + 1) * kSmallSamples) ends[1] = mine;
+    }
+    __syncthreads();
+    // The range [lo, hi), and of it, as a rule whole, the next stretch [from,
+    // to) of at most kSmallCap keys.
+    const uint64_t lo = ends[0], hi = ends[1];
+    uint64_t from = lo, to = hi;
+    int below = 0, kept = 0;
+    uint32_t prev_last = 0, first = 0;
+    while (from < hi) {
+        constexpr int kLoads = 8;  // (16 spill at 1,024 threads)
+        for (int i0 = 0; i0 < total; i0 += kLoads * kSmallThreads) {
+            uint32_t raw[kLoads];
 #pragma unroll
-        for (int q = 0; q < kRows; ++q) lo[q] = 0;
-        for (int step = kThreads * kItems; step > 0; step >>= 1) {
-#pragma unroll
-            for (int q = 0; q < kRows; ++q) {
-                const int r = r0 + q * kThreads;
-                const int at = lo[q] + step;
-                // keys before `at` are of rows before r
-                if (at <= n && static_cast<int64_t>(lds[at - 1] >> src.cbits) < r) lo[q] = at;
+            for (int q = 0; q < kLoads; ++q) {
+                const int i = i0 + q * kSmallThreads + t;
+                raw[q] = read_entry<Keys32, Src::kBoth>(src, Keys32{}, i < total ? i : total - 1,
+                                                        bad);
             }
-        }
+            int less = 0;
 #pragma unroll
-        for (int q = 0; q < kRows; ++q) {
-            const int r = r0 + q * kThreads;
-            if (r <= V) rowptr[r] = lo[q];
+            for (int q = 0; q < kLoads; ++q) {
+                const int i = i0 + q * kSmallThreads + t;
+                const uint64_t key =
+                    i < total ? (static_cast<uint64_t>(raw[q]) << kIndexBits) | static_cast<uint32_t>(i)
+                              : ~0ull;
+                less += key < lo;
+                const bool take = key >= from && key < to;
+                const uint64_t m = __ballot(take);
+                if (m == 0) continue;
+                int at = 0;
+                if (lane == 0) at = atomicAdd(&count[0], __popcll(m));
+                at = __builtin_amdgcn_readfirstlane(at) + lane_rank(m);
+                if (take && at < kSmallCap) lds[at] = raw[q];
+            }
+            for (int o = kWave / 2; o > 0; o >>= 1) less += __shfl_xor(less, o, kWave);
+            if (lane == 0 && less) atomicAdd(&count[1], less);
         }
+        __syncthreads();
+        const int n = count[0];
+        if (from == lo) below = count[1];
+        __syncthreads();
+        if (t == 0) count[0] = count[1] = 0;
+        if (n > kSmallCap) {
+            // A sample this uneven takes a list made for it.  The longest
+            // stretch from `from` that fits, by bisection of its end.
+            uint64_t fits = from, over = to;
+            while (over - fits > 1) {
+                const uint64_t mid = fits + (over - fits) / 2;
+                int c = 0;
+                for (int i = t; i < total; i += kSmallThreads) {
+                    const uint64_t k = placed_key(src, i, bad);
+                    c += k >= from && k < mid;
+                }
+                int64_t all;
+                block_exclusive_scan<kOpSum, kSmallThreads>(c, wtot, &all);
+                if (all <= kSmallCap) fits = mid;
+                else over = mid;
+            }
+            to = fits;
+            __syncthreads();
+            continue;
+        }
+        uint32_t key[kItems];
+        const int at = (t - lane) * kItems + lane;
+#pragma unroll
+        for (int q = 0; q < kItems; ++q) key[q] = at + q * kWave < n ? lds[at + q * kWave] : ~0u;
+        __syncthreads();
+        block_sort<kSmallThreads>(key, n, lds);
+        last[t] = key[kItems - 1];
+        __syncthreads();
+        const uint32_t before = t > 0 ? last[t - 1] : prev_last;
+        uint32_t keep = 0;
+#pragma unroll
+        for (int q = 0; q < kItems; ++q) {
+            const int i = t * kItems + q;
+            const uint32_t prev = q > 0 ? key[q > 0 ? q - 1 : 0] : before;
+            if (i < n && (!dedup || (i == 0 && kept == 0) || prev != key[q])) keep |= 1u << q;
+        }
+        int64_t all;
+        int p = kept + static_cast<int>(block_exclusive_scan<kOpSum, kSmallThreads>(
+                           __popc(keep), wtot, &all));
+#pragma unroll
+        for (int q = 0; q < kItems; ++q)
+            if ((keep >> q) & 1u) keys[below + p++] = key[q];
+        // the stretch's first and last keys, for the next and for the range
+        if (t == 0 && n > 0) ends[0] = key[0];
+        if (n > 0 && t == (n - 1) / kItems) {
+            uint32_t x = 0;
+#pragma unroll
+            for (int q = 0; q < kItems; ++q)
+                if (q == (n - 1) % kItems) x = key[q];
+            ends[1] = x;
+        }
+        __syncthreads();
+        if (n > 0) {
+            if (from == lo || kept == 0) first = static_cast<uint32_t>(ends[0]);
+            prev_last = static_cast<uint32_t>(ends[1]);
+        }
+        kept += static_cast<int>(all);
+        from = to;
+        to = hi;
+        __syncthreads();
     }
-    if (t < MLXC_WORK_WORDS)
-        work[t] = t == 0 ? (any_bad ? MLXC_STATUS_BAD_NODE : 0) : t == 1 ? n : 0;
+    const int any_bad = __syncthreads_or(bad);
+    if (t == 0) {
+        ranges[b] = SmallRange{below, kept, first, prev_last};
+        if (b == 0) work[0] = any_bad ? MLXC_STATUS_BAD_NODE : 0;
+    }
+}
+
+// col and rowptr from the sorted ranges (block b copies range b's keys; all
+// blocks share the rows), and the words of `work` after the first.
+__global__ __launch_bounds__(kBlock) void small_emit_kernel(
+    int ways, int64_t num_nodes, int cbits, bool dedup, const uint32_t* __restrict__ keys,
+    const SmallRange* __restrict__ ranges, int64_t* __restrict__ rowptr,
+    int64_t* __restrict__ col_out, int64_t* __restrict__ work) {
+    static_assert(kSmallWays <= kBlock, "a range a thread");
+    __shared__ int32_t base[kBlock], count[kBlock], pos[kBlock];
+    __shared__ uint32_t low[kBlock];  // smallest key; of an empty range, the largest before it
+    __shared__ uint32_t high[kBlock];
+    __shared__ int64_t wtot[kWaves];
+    const int t = threadIdx.x;
+    SmallRange r{0, 0, 0, 0};
+    if (t < ways) r = ranges[t];
+    count[t] = r.kept;
+    high[t] = r.last;
+    __syncthreads();
+    int p = t < ways ? t - 1 : -1;  // the last range before this one that holds keys
+    while (p >= 0 && count[p] == 0) --p;
+    // a pair repeated across the ranges' border is in the earlier one
+    const int drop = dedup && r.kept > 0 && p >= 0 && high[p] == r.first;
+    const int n = r.kept - drop;
+    int64_t all;
+    const int64_t at = block_exclusive_scan<kOpSum>(n, wtot, &all);  // (its barriers cover count)
+    base[t] = r.base + drop;
+    count[t] = n;
+    pos[t] = static_cast<int32_t>(at);
+    low[t] = r.kept > 0 ? r.first : p >= 0 ? high[p] : 0u;
+    __syncthreads();
+    const uint32_t cmask = cbits == 0 ? 0u : ~0u >> (32 - cbits);
+    if (blockIdx.x < static_cast<unsigned>(ways)) {
+        const int b = blockIdx.x;
+        for (int j = t; j < count[b]; j += kBlock)
+            col_out[pos[b] + j] = static_cast<int64_t>(keys[base[b] + j] & cmask);
+    }
+    for (int64_t v = static_cast<int64_t>(blockIdx.x) * kBlock + t; v <= num_nodes;
+         v += static_cast<int64_t>(gridDim.x) * kBlock) {
+        // the last range that starts in a row before v, then the keys of its
+        // rows before v
+        int i = -1;
+        for (int step = kBlock / 2; step > 0; step >>= 1)
+            if (i + step < ways && static_cast<int64_t>(low[i + step] >> cbits) < v) i += step;
+        if (i + 1 < ways && static_cast<int64_t>(low[i + 1] >> cbits) < v) ++i;
+        int64_t before = 0;
+        if (i >= 0) {
+            int lo = 0;
+            const int len = count[i];
+            for (int step = 1 << (31 - __builtin_clz(len | 1)); step > 0; step >>= 1)
+                if (lo + step <= len &&
+                    static_cast<int64_t>(keys[base[i] + lo + step - 1] >> cbits) < v)
+                    lo += step;
+            before = pos[i] + lo;
+        }
+        rowptr[v] = before;
+    }
+    if (blockIdx.x == 0 && t > 0 && t < MLXC_WORK_WORDS) work[t] = t == 1 ? all : 0;
 }
 
 // ------------------------------------------------------------- host side
-
-// Lists of up to kSmallTotal entries (what one block's registers hold) over up
-// to kSmallNodes nodes are built by csr_small_kernel.  The searches of rowptr
-// cost it 4 us per 4,096 rows: to_csr of 16,384 pairs takes 80 us over 20,000
-// nodes and 124 over 65,536, with the radix passes 114 either way.  With 256
-// threads those searches cost four times as much, and pay only where rows are
-// few: 4,096 pairs over 2,708 nodes take 45 us.
-constexpr int kSmallThreads = 1024;
-constexpr int kSmallTotal = kSmallThreads * kItems;
-constexpr int64_t kSmallNodes = 32768;
-static_assert(2 * 15 <= 32, "keys over kSmallNodes nodes take 32 bits");
 
 int bits_for(int64_t num_nodes) {
     int b = 0;
@@ -980,15 +1141,19 @@ int launch_csr_build(const int64_t* row, const int64_t* col, int64_t num_edges, 
     char* ws = static_cast<char*>(workspace);
     int64_t* work = reinterpret_cast<int64_t*>(ws);
     const EdgeSrc src{row, col, num_edges, num_nodes, l.cbits};
-    if (l.total > 0 && l.total <= kSmallTotal && num_nodes <= kSmallNodes) {
+    if (l.total > 0 && l.total <= kSmallTotal && l.key_bytes == 4) {
         const bool dedup = (flags & MLXC_CSR_DEDUP) != 0;
         const int total = static_cast<int>(l.total);
-        if (total <= kBlock * kItems && num_nodes <= kBlock * kItems)
-            hipLaunchKernelGGL(csr_small_kernel<kBlock>, dim3(1), dim3(kBlock), 0, stream, src,
-                               total, dedup, rowptr, col_out, work);
-        else
-            hipLaunchKernelGGL(csr_small_kernel<kSmallThreads>, dim3(1), dim3(kSmallThreads), 0,
-                               stream, src, total, dedup, rowptr, col_out, work);
+        const int ways = (total + kSmallKeys - 1) / kSmallKeys;
+        uint32_t* keys = reinterpret_cast<uint32_t*>(ws + l.keys[0]);
+        SmallRange* ranges = reinterpret_cast<SmallRange*>(ws + l.hist);
+        hipLaunchKernelGGL(small_sort_kernel, dim3(ways), dim3(kSmallThreads), 0, stream, src, total,
+                           ways, dedup, keys, ranges, work);
+        MLXC_HIP_TRY(hipGetLastError());
+        const int64_t row_blocks = num_nodes / kBlock + 1;  // at most 257
+        hipLaunchKernelGGL(small_emit_kernel, dim3(row_blocks > ways ? row_blocks : ways),
+                           dim3(kBlock), 0, stream, ways, num_nodes, l.cbits, dedup, keys, ranges,
+                           rowptr, col_out, work);
         MLXC_HIP_TRY(hipGetLastError());
         return MLXC_OK;
     }

@@ -268,22 +268,46 @@ def test_rowptr_of_2_28_nodes(cuda):
         del rowptr, c, ref
 
 
-@pytest.mark.parametrize("E", [15, 16, 1024, 1025, 2049, 4096, 4097, 8193, 10_556, 16_383, 16_384,
-                               16_385])
-@pytest.mark.parametrize("V", [3, 2708, 4097, 32768, 32769, 65536])
+@pytest.mark.parametrize("E", [1, 15, 512, 513, 1024, 1025, 10_556, 16_385, 98_304, 98_305])
+@pytest.mark.parametrize("V", [3, 2708, 32768, 65536, 65537])
 def test_small_list_edges(E, V, cuda):
-    """The one-launch build around its wavefront, block and size limits (and
-    just past them), with the largest ids, equal keys and empty rows at both
-    ends."""
+    """The two-launch build around its range, block and size limits (and just
+    past them), with the largest ids (at 65,536 nodes the key with every bit
+    set), equal keys and empty rows at both ends."""
     rng = np.random.default_rng(E + V)
     row, col = rng.integers(V // 3, V, E), rng.integers(0, V, E)
     row[: E // 2] = row[0]          # a hub
     row[E // 3: E // 3 + 9] = col[E // 3: E // 3 + 9] = V - 1
     for dedup in (False, True):
         assert_parity(row, col, V, cuda, dedup=dedup)
-    assert_parity(np.full(E, V - 1), np.full(E, V - 1), V, cuda)
-    if E <= 8193:
+        # every key the same: only an entry's place tells them apart
+        assert_parity(np.full(E, V - 1), np.full(E, V - 1), V, cuda, dedup=dedup)
+    # few distinct keys, each across several blocks' ranges
+    assert_parity(rng.integers(0, 2, E), np.full(E, V - 1), V, cuda, dedup=True)
+    if E <= 16_385:
         assert_parity(row, col, V, cuda, symmetrize=True, dedup=True)
+
+
+@pytest.mark.parametrize("dedup", [False, True])
+def test_small_list_made_for_its_sample(dedup, cuda):
+    """A list whose sampled entries all lie above the others, so that one
+    block's range holds nearly all of it, more than a block sorts at once
+    (16,384 keys): the block takes it in stretches."""
+    def mix32(x):
+        x = np.uint64(x)
+        x ^= x >> np.uint64(16)
+        x = x * np.uint64(0x7feb352d) & np.uint64(0xffffffff)
+        x ^= x >> np.uint64(15)
+        x = x * np.uint64(0x846ca68b) & np.uint64(0xffffffff)
+        return int(x ^ (x >> np.uint64(16)))
+    E, V = 60_000, 1000
+    rng = np.random.default_rng(1)
+    row, col = rng.integers(0, 90, E), rng.integers(0, V, E)
+    ns = -(-E // 512) * 4
+    for i in range(ns):
+        a, b = i * E // ns, (i + 1) * E // ns
+        row[a + mix32(i) % (b - a)] = V - 1 - i % 9
+    assert_parity(row, col, V, cuda, dedup=dedup)
 
 
 def test_small_list_bad_ids(cuda):
