@@ -450,9 +450,10 @@ int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream
 /*
  * Makes the calling thread's walk calls publish their status themselves, as
  * mlxc_publish_status after each of them would, into h_status (as there; the
- * caller zeroes h_status[0] before each call), until it is set to NULL.  Small
- * calls save a launch that way: the one that gathers their blocks' status bits
- * publishes them too.  No reference counterpart.
+ * caller zeroes h_status[0] before each call), until it is set to NULL; and
+ * its mlxc_csr_build calls theirs, with workspace word 1 (the entry count) in
+ * a third word.  Small calls save a launch that way: the one that gathers
+ * their blocks' results publishes them too.  No reference counterpart.
  */
 int mlxc_set_status_target(int64_t* h_status);
 

@@ -20,7 +20,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .walks import (_check_stream_arg, _enter_side_stream, _leave_side_stream, _on_device,
+from .walks import (_check_stream_arg, _fast, _enter_side_stream, _leave_side_stream, _on_device,
                     _side_stream, _stream_handle, _workspace)
 
 
@@ -42,6 +42,13 @@ def to_csr(edge_index, num_nodes: Optional[int] = None, *, symmetrize: bool = Fa
 
     Raises ValueError when an id lies outside [0, num_nodes).
     """
+    if (_fast is not None and device is None and stream is None and
+            type(edge_index) is torch.Tensor and type(num_nodes) is int):
+        res = _fast.to_csr(edge_index, num_nodes,
+                           (_lib.MLXC_CSR_SYMMETRIZE if symmetrize else 0) |
+                           (_lib.MLXC_CSR_DEDUP if dedup else 0))
+        if res is not None:
+            return res
     if isinstance(edge_index, np.ndarray):
         edge_index = torch.from_numpy(edge_index)
     if not isinstance(edge_index, torch.Tensor) or edge_index.dim() != 2 or edge_index.shape[0] != 2:

@@ -864,16 +864,19 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
     const int any_bad = __syncthreads_or(bad);
     if (t == 0) {
         ranges[b] = SmallRange{below, kept, first, prev_last};
-        if (b == 0) work[0] = any_bad ? MLXC_STATUS_BAD_NODE : 0;
+        if (b == 0) {
+            work[0] = any_bad ? MLXC_STATUS_BAD_NODE : 0;
+            work[2] = work[3] = 0;  // (work[2] counts the next launch's blocks)
+        }
     }
 }
 
 // col and rowptr from the sorted ranges (block b copies range b's keys; all
-// blocks share the rows), and the words of `work` after the first.
+// blocks share the rows), and work[1].
 __global__ __launch_bounds__(kBlock) void small_emit_kernel(
     int ways, int64_t num_nodes, int cbits, bool dedup, const uint32_t* __restrict__ keys,
     const SmallRange* __restrict__ ranges, int64_t* __restrict__ rowptr,
-    int64_t* __restrict__ col_out, int64_t* __restrict__ work) {
+    int64_t* __restrict__ col_out, int64_t* __restrict__ work, int64_t* h_status) {
     static_assert(kSmallWays <= kBlock, "a range a thread");
     __shared__ int32_t base[kBlock], count[kBlock], pos[kBlock];
     __shared__ uint32_t low[kBlock];  // smallest key; of an empty range, the largest before it
@@ -923,7 +926,16 @@ __global__ __launch_bounds__(kBlock) void small_emit_kernel(
         }
         rowptr[v] = before;
     }
-    if (blockIdx.x == 0 && t > 0 && t < MLXC_WORK_WORDS) work[t] = t == 1 ? all : 0;
+    if (blockIdx.x == 0 && t == 1) work[1] = all;
+    if (!h_status) return;
+    // The last block to end publishes the status and the count: whoever waits
+    // for them may then use the arrays on any stream.
+    __syncthreads();
+    if (t == 0) {
+        __threadfence();
+        if (atomicAdd(reinterpret_cast<unsigned long long*>(work + 2), 1ull) == gridDim.x - 1)
+            publish_count(work[0], all, h_status);
+    }
 }
 
 // ------------------------------------------------------------- host side
@@ -1153,8 +1165,9 @@ int launch_csr_build(const int64_t* row, const int64_t* col, int64_t num_edges, 
         const int64_t row_blocks = num_nodes / kBlock + 1;  // at most 257
         hipLaunchKernelGGL(small_emit_kernel, dim3(row_blocks > ways ? row_blocks : ways),
                            dim3(kBlock), 0, stream, ways, num_nodes, l.cbits, dedup, keys, ranges,
-                           rowptr, col_out, work);
+                           rowptr, col_out, work, g_status_target.words);
         MLXC_HIP_TRY(hipGetLastError());
+        g_status_target.done = g_status_target.words != nullptr;
         return MLXC_OK;
     }
     if (int rc = launch_zero_work(work, stream)) return rc;

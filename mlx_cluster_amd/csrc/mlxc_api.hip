@@ -225,15 +225,10 @@ HostWalk host_walk(const int64_t* rowptr, int64_t num_nodes, const int64_t* col,
                     static_cast<uint32_t>(seed >> 32), first_walk};
 }
 
-// The status word of a call into host memory, then the flag that it is
-// there: system-scope stores, the flag's with release order.
-__device__ __forceinline__ void publish(int64_t bits, int64_t* h_status) {
-    __hip_atomic_store(h_status + 1, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    __hip_atomic_store(h_status, int64_t{1}, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-__global__ void publish_status_kernel(const int64_t* work, int64_t* h_status) {
-    if (threadIdx.x == 0) publish(work[0], h_status);
+__global__ void publish_status_kernel(const int64_t* work, int64_t* h_status, bool count) {
+    if (threadIdx.x != 0) return;
+    if (count) publish_count(work[0], work[1], h_status);
+    else publish(work[0], h_status);
 }
 
 // See launch_finish; h_status may be null.
@@ -262,17 +257,19 @@ int64_t* device_words(int64_t* h_status) {
     return d;
 }
 
-// The last step of a walk call (rc: how it went so far): publishes its status
-// word if the thread has a target and the call's own launches have not.
-int end_walk(int rc, const int64_t* d_work, hipStream_t s) {
+// The last step of a walk call or a CSR build (count: it has one; rc: how it
+// went so far): publishes its status word if the thread has a target and the
+// call's own launches have not.
+int end_call(int rc, const int64_t* d_work, bool count, hipStream_t s) {
     const bool done = g_status_target.done;
     g_status_target.done = false;
     if (rc != MLXC_OK || !g_status_target.words || done) return rc;
     hipLaunchKernelGGL(publish_status_kernel, dim3(1), dim3(kWave), 0, s, d_work,
-                       g_status_target.words);
+                       g_status_target.words, count);
     MLXC_HIP_TRY(hipGetLastError());
     return MLXC_OK;
 }
+int end_walk(int rc, const int64_t* d_work, hipStream_t s) { return end_call(rc, d_work, false, s); }
 
 }  // namespace
 
@@ -304,7 +301,7 @@ int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream
                     "h_status is not host memory the device can write (hipHostMalloc)");
     hipLaunchKernelGGL(publish_status_kernel, dim3(1), dim3(kWave), 0,
                        static_cast<hipStream_t>(stream), static_cast<const int64_t*>(d_workspace),
-                       d_status);
+                       d_status, false);
     MLXC_HIP_TRY(hipGetLastError());
     return MLXC_OK;
 }
@@ -495,8 +492,10 @@ int mlxc_csr_build(const int64_t* d_row, const int64_t* d_col, int64_t num_edges
     if (int rc = check_csr_build(d_row, d_col, num_edges, num_nodes, flags, d_rowptr, d_col_out))
         return rc;
     if (int rc = check_workspace(d_workspace, workspace_bytes)) return rc;
-    return launch_csr_build(d_row, d_col, num_edges, num_nodes, flags, d_rowptr, d_col_out,
-                            d_workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    const int rc = launch_csr_build(d_row, d_col, num_edges, num_nodes, flags, d_rowptr, d_col_out,
+                                    d_workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+    return end_call(rc, static_cast<const int64_t*>(d_workspace), true,
+                    static_cast<hipStream_t>(stream));
 }
 
 int mlxc_csr_build_cpu(const int64_t* row, const int64_t* col, int64_t num_edges,

@@ -36,14 +36,14 @@ void raise_code(int rc, const char* what) {
     throw std::runtime_error(msg);
 }
 
-// The calling thread's two host words for mlxc_publish_status: allocated at
+// The calling thread's host words for mlxc_set_status_target: allocated at
 // the thread's first validated call (one pinned page) and kept for the rest
 // of the process, since freeing them at thread exit could run after the HIP
 // runtime has shut down; null if the allocation failed.
 int64_t* status_words() {
     thread_local int64_t* words = [] {
         void* p = nullptr;
-        if (hipHostMalloc(&p, 2 * sizeof(int64_t),
+        if (hipHostMalloc(&p, 3 * sizeof(int64_t),
                           hipHostMallocCoherent | hipHostMallocMapped | hipHostMallocPortable) !=
             hipSuccess) {
             (void)hipGetLastError();
@@ -75,27 +75,30 @@ public:
 // 200 us (the reference tests' calls take tens), then in hipStreamSynchronize.
 // Without the host words, torch's scalar read (a copy ordered on the stream,
 // about 13 us more per call).
-int64_t read_status(const at::Tensor& work, hipStream_t stream, const int64_t* h) {
-    if (h) {
-        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
-        for (unsigned i = 1;; ++i) {
-            if (__atomic_load_n(&h[0], __ATOMIC_ACQUIRE)) return __atomic_load_n(&h[1], __ATOMIC_RELAXED);
-            __builtin_ia32_pause();
-            if (i % 64 == 0 && std::chrono::steady_clock::now() > until) break;
-        }
-        if (hipStreamSynchronize(stream) != hipSuccess)
-            throw std::runtime_error(std::string("hipStreamSynchronize: ") +
-                                     hipGetErrorString(hipGetLastError()));
-        if (__atomic_load_n(&h[0], __ATOMIC_ACQUIRE)) return __atomic_load_n(&h[1], __ATOMIC_RELAXED);
+bool wait_published(hipStream_t stream, const int64_t* h) {
+    if (!h) return false;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    for (unsigned i = 1;; ++i) {
+        if (__atomic_load_n(&h[0], __ATOMIC_ACQUIRE)) return true;
+        __builtin_ia32_pause();
+        if (i % 64 == 0 && std::chrono::steady_clock::now() > until) break;
     }
-    return work.select(0, 0).item<int64_t>();
+    if (hipStreamSynchronize(stream) != hipSuccess)
+        throw std::runtime_error(std::string("hipStreamSynchronize: ") +
+                                 hipGetErrorString(hipGetLastError()));
+    return __atomic_load_n(&h[0], __ATOMIC_ACQUIRE) != 0;
+}
+// Word k of the call's workspace (0, or 1 after a CSR build).
+int64_t read_word(const at::Tensor& work, hipStream_t stream, const int64_t* h, int k) {
+    if (wait_published(stream, h)) return __atomic_load_n(&h[1 + k], __ATOMIC_RELAXED);
+    return work.select(0, k).item<int64_t>();
 }
 
 // Waits for the call and raises ValueError for status bits, as walks.py's
 // check=True does.
 void check_status(const at::Tensor& work, hipStream_t stream, const int64_t* words,
                   const char* what) {
-    const int64_t bits = read_status(work, stream, words);
+    const int64_t bits = read_word(work, stream, words, 0);
     if (bits == 0) return;
     std::string msg = std::string(what) + ": ";
     if (bits & MLXC_STATUS_BAD_NODE) msg += "a start or col entry is outside [0, num_nodes)";
@@ -201,10 +204,40 @@ py::object rejection_sampling(const at::Tensor& rowptr, const at::Tensor& col,
     return outputs(n_out, e_out, return_edges);
 }
 
+// to_csr(edge_index, num_nodes, flags) -> (rowptr, col) or None.
+py::object to_csr(const at::Tensor& edge_index, int64_t num_nodes, int32_t flags) {
+    if (!edge_index.is_cuda() || edge_index.dim() != 2 || edge_index.size(0) != 2 || num_nodes < 0)
+        return py::none();
+    const at::Device device = edge_index.device();
+    if (device.index() != c10::hip::current_device() || !usable(edge_index, at::kLong, device))
+        return py::none();
+    const int64_t E = edge_index.size(1);
+    const size_t ws = mlxc_csr_build_workspace_bytes(num_nodes, E, flags);
+    if (ws == 0) return py::none();
+    const int64_t* row = E ? edge_index.data_ptr<int64_t>() : nullptr;
+    const int64_t* col = E ? row + E : nullptr;
+    const auto opts = at::TensorOptions().dtype(at::kLong).device(device);
+    at::Tensor rowptr = at::empty({num_nodes + 1}, opts);
+    at::Tensor col_out = at::empty({flags & MLXC_CSR_SYMMETRIZE ? 2 * E : E}, opts);
+    at::Tensor work = at::empty({static_cast<int64_t>((ws + 7) / 8)}, opts);
+    hipStream_t stream = at::hip::getCurrentHIPStream().stream();
+    const StatusTarget target(true);
+    const int rc = mlxc_csr_build(row, col, E, num_nodes, flags, rowptr.data_ptr<int64_t>(),
+                                  col_out.numel() ? col_out.data_ptr<int64_t>() : nullptr,
+                                  work.data_ptr(), static_cast<size_t>(work.numel()) * 8, stream);
+    if (rc != MLXC_OK) raise_code(rc, "to_csr");
+    const int64_t bits = read_word(work, stream, target.words, 0);
+    const int64_t count = read_word(work, stream, target.words, 1);
+    if (bits & MLXC_STATUS_BAD_NODE)
+        throw py::value_error("edge_index holds ids outside [0, num_nodes)");
+    return py::make_tuple(rowptr, col_out.narrow(0, 0, count));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_mlxc_torch, m) {
-    m.doc() = "Compiled fast path of mlx_cluster_amd.random_walk / rejection_sampling";
+    m.doc() = "Compiled fast path of mlx_cluster_amd.random_walk / rejection_sampling / to_csr";
     m.def("random_walk", &random_walk);
     m.def("rejection_sampling", &rejection_sampling);
+    m.def("to_csr", &to_csr);
 }

@@ -176,6 +176,18 @@ struct WalkArgs {
     uint32_t* block_status = nullptr;
 };
 
+// The status word of a call into host memory, then the flag that it is
+// there: system-scope stores, the flag's with release order.
+__device__ __forceinline__ void publish(int64_t bits, int64_t* h_status) {
+    __hip_atomic_store(h_status + 1, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(h_status, int64_t{1}, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// ... with the entry count of a CSR build in the word after it.
+__device__ __forceinline__ void publish_count(int64_t bits, int64_t count, int64_t* h_status) {
+    __hip_atomic_store(h_status + 2, count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    publish(bits, h_status);
+}
+
 // Status bits of the whole wavefront (every lane calls it).
 __device__ __forceinline__ uint32_t wave_status(uint32_t status) {
     return (__any(status & MLXC_STATUS_BAD_NODE) ? MLXC_STATUS_BAD_NODE : 0u) |

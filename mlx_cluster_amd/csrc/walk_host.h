@@ -34,9 +34,9 @@ inline int record_walk_event(int which, hipStream_t stream) {
     return MLXC_OK;
 }
 
-// Where the calling thread's walk calls publish their status word (device
-// address of the caller's host words; null: nowhere), and whether the call
-// in progress already has.
+// Where the calling thread's walk calls publish their status word, and its CSR
+// builds theirs and their entry count (device address of the caller's host
+// words; null: nowhere), and whether the call in progress already has.
 struct StatusTarget {
     int64_t* words;
     bool done;

@@ -316,3 +316,20 @@ def test_small_list_bad_ids(cuda):
         ei[1, 10_000] = bad
         with pytest.raises(ValueError, match="outside"):
             mc.to_csr(ei, 2708)
+
+
+@pytest.mark.parametrize("E", [10_556, 90_000, 200_000])
+def test_result_is_whole_when_the_call_returns(E, cuda):
+    """to_csr waits for the build, not only for its count: what it returns can
+    be read on another stream at once."""
+    other = torch.cuda.Stream(cuda)
+    ei = torch.randint(0, 20_000, (2, E), device=cuda)
+    ref_rowptr, ref_col = oracle.csr_build(*ei.cpu().numpy(), 20_000, dedup=True)
+    ref_rowptr, ref_col = (torch.from_numpy(a).to(cuda) for a in (ref_rowptr, ref_col))
+    for _ in range(20):
+        torch.cuda.synchronize()
+        rowptr, col = mc.to_csr(ei, 20_000, dedup=True)
+        with torch.cuda.stream(other):
+            same = torch.equal(rowptr, ref_rowptr) and torch.equal(col, ref_col)
+        other.synchronize()
+        assert same
