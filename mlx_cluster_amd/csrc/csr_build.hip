@@ -680,27 +680,32 @@ __global__ __launch_bounds__(kBlock) void csr_emit_kernel(Store keys,
 // The whole build of a small list in two launches.  Every block reads the
 // whole list and keeps the keys (32 bits) of its own range, about
 // kSmallKeys of them, between splitters that all blocks take from the same
-// sample; it sorts them in registers (block_sort.h), drops repeats and stores
-// them.  How many keys lie below its range it has counted on the way, so no
-// block waits for another.  A key's place in the list breaks ties, so ranges
-// stay even however often a pair repeats.  The second launch writes col, and
-// rowptr by a binary search per row.
+// sample; it sorts them by their ranks (rank_keys), larger ranges by a network
+// in registers (block_sort.h), drops repeats and stores them.  How many keys
+// lie below its range it has counted on the way, so no block waits for
+// another.  A key's place in the list breaks ties, so ranges stay even however
+// often a pair repeats.  The second launch writes col, and rowptr by a binary
+// search per row.
 //
-// Bound by latencies: two loads and their use, a network of 55 stages in one
-// wavefront, the search's 10 dependent reads.  Radix passes need 16 to 19
-// launches for such a list.  10,556 pairs over 2,708 nodes: 74 us of radix
-// kernels, 38 us when one block sorted the whole list, now 23 + 7 us; to_csr
-// 92 -> 58 -> 50 us.
+// Bound by latencies and the list's pass through every block (of 10,556 pairs
+// 3 us, of 60,000 about 15).  Radix passes need 16 to 19 launches for such a
+// list.  Kernels, 10,556 pairs over 2,708 nodes: radix 74 us, one block 38,
+// ranges of 512 sorted by the network 29, now 21; 60,000 pairs 61 -> 48;
+// to_csr of the former 93 us -> 58 -> 37 -> 31.
 constexpr int kSmallThreads = 1024;
-constexpr int kSmallKeys = 512;      // keys of a block's range, on average
-constexpr int kSmallSamples = 4;     // samples per range
-// Ranges at most.  Every block reads the whole list: to_csr of 88,648 pairs
-// takes 105 us (radix passes 116), of 131,072 138 us (117).
-constexpr int kSmallWays = 192;
-constexpr int64_t kSmallTotal = static_cast<int64_t>(kSmallWays) * kSmallKeys;
+// Keys of a block's range on average, while the ranges suffice.  The sort's
+// share falls with it, the sample's grows: 10,556 pairs take 29, 26, 22 and 21
+// us at 512, 256, 192 and 128, with 96 the same.
+constexpr int kSmallKeys = 128;
+constexpr int kSmallSamples = 2;  // samples per range (4: 98,304 pairs 69 us instead of 61)
+constexpr int kSmallWays = 192;   // ranges at most
+// Entries at most: 98,304 pairs take 61 us (radix passes 86), 131,072 77 (89 to
+// 99), 163,840 90 (90 to 100), each pair through every block.
+constexpr int64_t kSmallTotal = int64_t{1} << 17;
+// Keys a block sorts by rank; a network of 1,024 keys takes 4.5 us and its
+// store 2.3, the ranks of 512 keys 3.4.
+constexpr int kSmallRank = 512;
 constexpr int kSmallCap = kSmallThreads * kItems;  // keys a block sorts at once
-constexpr int kIndexBits = 17;
-static_assert(kSmallTotal <= (int64_t{1} << kIndexBits), "an entry's place fits its field");
 
 struct SmallRange {
     int32_t base;         // where the range's keys start
@@ -718,23 +723,84 @@ __host__ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
 }
 // Sample i of `count` of the n > 0 entries: one in each of `count` equal parts.
 __host__ __device__ __forceinline__ int sample_at(int i, int count, int n) {
-    const int a = static_cast<int>(static_cast<int64_t>(i) * n / count);
-    const int b = static_cast<int>(static_cast<int64_t>(i + 1) * n / count);
-    return a + (b > a ? static_cast<int>(mix32(i) % static_cast<uint32_t>(b - a)) : 0);
+    const uint32_t a = static_cast<uint32_t>(i) * static_cast<uint32_t>(n) / count;
+    const uint32_t b = static_cast<uint32_t>(i + 1) * static_cast<uint32_t>(n) / count;
+    return static_cast<int>(a + (b > a ? mix32(i) % (b - a) : 0));
+}
+static_assert(static_cast<int64_t>(kSmallWays) * kSmallSamples * kSmallTotal < (int64_t{1} << 32),
+              "a sample's place in 32 bits");
+
+// The ids of entry i as the caller's arrays hold them (the reversed pair from
+// entry src.num_edges on), and its key; 32-bit offsets and ids, for the whole
+// list is read once a block.
+struct SmallEntry {
+    int64_t row, col;
+};
+__device__ __forceinline__ SmallEntry small_entry(const EdgeSrc& src, int i) {
+    const int n = static_cast<int>(src.num_edges);
+    const uint32_t j = i < n ? i : i - n;
+    return SmallEntry{src.row[j], src.col[j]};
+}
+__device__ __forceinline__ uint32_t small_key(const EdgeSrc& src, const SmallEntry& e, int i,
+                                              bool& bad) {
+    const uint32_t r = static_cast<uint32_t>(clamp_id(e.row, src.num_nodes, bad));
+    const uint32_t c = static_cast<uint32_t>(clamp_id(e.col, src.num_nodes, bad));
+    return i < static_cast<int>(src.num_edges) ? r << src.cbits | c : c << src.cbits | r;
+}
+// An entry's key with its place below it: distinct for every entry.
+__device__ __forceinline__ uint64_t place_key(uint32_t key, int i) {
+    return (static_cast<uint64_t>(key) << 32) | static_cast<uint32_t>(i);
+}
+__device__ __forceinline__ uint64_t placed_key(const EdgeSrc& src, int i, bool& bad) {
+    return place_key(small_key(src, small_entry(src, i), i, bad), i);
 }
 
-// Key of entry i with its place below it: distinct for every entry.
-__device__ __forceinline__ uint64_t placed_key(const EdgeSrc& src, int i, bool& bad) {
-    return (static_cast<uint64_t>(read_entry<Keys32, Src::kBoth>(src, Keys32{}, i, bad))
-            << kIndexBits) | static_cast<uint32_t>(i);
+// rank[k] += the number of keys that come before key k, equal ones in their
+// order, for n <= kSmallThreads keys, by comparing each with all: two
+// instructions a pair, no chain.  Every thread calls it; rank starts at 0 and
+// is whole after a barrier of the caller's.  keys: 16-byte aligned, ~0 from n
+// up to a multiple of 4.
+__device__ __forceinline__ void rank_keys(const uint32_t* keys, int n, int32_t* rank) {
+    const int t = threadIdx.x;
+    int log = 6;  // 2^log >= n keys, each by kSmallThreads >> log threads
+    while ((1 << log) < n) ++log;
+    const int k = t & ((1 << log) - 1);
+    const int kw = __builtin_amdgcn_readfirstlane(k);  // the wavefront's first key
+    if (kw >= n) return;
+    const int part = __builtin_amdgcn_readfirstlane(t >> log);
+    const int n4 = (n + 3) / 4, parts = kSmallThreads >> log;
+    const int from = part * n4 / parts * 4, to = (part + 1) * n4 / parts * 4;
+    const uint32_t key = keys[k < n ? k : n - 1];
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    // Before the wavefront's own keys equal ones count, after them they don't.
+    const int own = kw < from ? from : kw > to ? to : kw;
+    const int past = kw + kWave < from ? from : kw + kWave > to ? to : kw + kWave;
+    int c = 0;
+#pragma unroll 4
+    for (int j = from; j < own; j += 4) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(keys + j);
+        c += (v.x <= key) + (v.y <= key) + (v.z <= key) + (v.w <= key);
+    }
+#pragma unroll 4
+    for (int j = own; j < past; j += 4) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(keys + j);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c += v[q] < key || (v[q] == key && j + q < k);
+    }
+#pragma unroll 4
+    for (int j = past; j < to; j += 4) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(keys + j);
+        c += (v.x < key) + (v.y < key) + (v.z < key) + (v.w < key);
+    }
+    if (k < n && c) atomicAdd(&rank[k], c);
 }
 
 __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
     EdgeSrc src, int total, int ways, bool dedup, uint32_t* __restrict__ keys,
     SmallRange* __restrict__ ranges, int64_t* __restrict__ work) {
     static_assert(kSortItems == kItems, "16 keys a thread");
-    __shared__ uint32_t lds[sort_lds_keys<kSmallThreads>()];
-    __shared__ uint64_t sample[kSmallWays * kSmallSamples];
+    __shared__ __align__(16) uint32_t lds[sort_lds_keys<kSmallThreads>()];
+    __shared__ int32_t rank[kSmallThreads];
     __shared__ uint32_t last[kSmallThreads];
     __shared__ int64_t wtot[kSmallThreads / kWave];
     __shared__ uint64_t ends[2];
@@ -746,18 +812,19 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
         ends[1] = ~0ull;  // the last one ends above them
         count[0] = count[1] = 0;
     }
+    // A sample's rank is its number among all of them (whose places ascend).
     const int ns = ways * kSmallSamples;
+    static_assert(kSmallWays * kSmallSamples <= kSmallThreads, "a sample a thread");
     uint64_t mine = 0;
-    if (t < ns) sample[t] = mine = placed_key(src, sample_at(t, ns, total), bad);
+    rank[t] = 0;
+    if (t < ns) mine = placed_key(src, sample_at(t, ns, total), bad);
+    lds[t] = t < ns ? static_cast<uint32_t>(mine >> 32) : ~0u;
     __syncthreads();
-    // A sample's rank is its number among all of them; equal samples (lists
-    // shorter than the sample) by number.
+    rank_keys(lds, ns, rank);
+    __syncthreads();
     if (t < ns) {
-        int rank = 0;
-        for (int j = 0; j < ns; ++j)
-            rank += sample[j] < mine || (sample[j] == mine && j < t);
-        if (b > 0 && rank == b * kSmallSamples) ends[0] = mine;
-        if (rank == (b + 1) * kSmallSamples) ends[1] = mine;
+        if (b > 0 && rank[t] == b * kSmallSamples) ends[0] = mine;
+        if (rank[t] == (b + 1) * kSmallSamples) ends[1] = mine;
     }
     __syncthreads();
     // The range [lo, hi), and of it, as a rule whole, the next stretch [from,
@@ -767,34 +834,48 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
     int below = 0, kept = 0;
     uint32_t prev_last = 0, first = 0;
     while (from < hi) {
-        constexpr int kLoads = 8;  // (16 spill at 1,024 threads)
-        for (int i0 = 0; i0 < total; i0 += kLoads * kSmallThreads) {
-            uint32_t raw[kLoads];
+        // The next round's loads fly while this round's keys are taken.
+        constexpr int kLoads = 3;
+        constexpr int kRound = kLoads * kSmallThreads;
+        SmallEntry next[kLoads];
+        auto load = [&](int i0) {
 #pragma unroll
             for (int q = 0; q < kLoads; ++q) {
                 const int i = i0 + q * kSmallThreads + t;
-                raw[q] = read_entry<Keys32, Src::kBoth>(src, Keys32{}, i < total ? i : total - 1,
-                                                        bad);
+                next[q] = small_entry(src, i < total ? i : total - 1);
             }
-            int less = 0;
+        };
+        int less = 0;
+        load(0);
+        for (int i0 = 0; i0 < total; i0 += kRound) {
+            SmallEntry raw[kLoads];
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q) raw[q] = next[q];
+            if (i0 + kRound < total) load(i0 + kRound);
+            uint32_t key[kLoads];
+            uint64_t take[kLoads];
+            int taken = 0;
 #pragma unroll
             for (int q = 0; q < kLoads; ++q) {
                 const int i = i0 + q * kSmallThreads + t;
-                const uint64_t key =
-                    i < total ? (static_cast<uint64_t>(raw[q]) << kIndexBits) | static_cast<uint32_t>(i)
-                              : ~0ull;
-                less += key < lo;
-                const bool take = key >= from && key < to;
-                const uint64_t m = __ballot(take);
-                if (m == 0) continue;
-                int at = 0;
-                if (lane == 0) at = atomicAdd(&count[0], __popcll(m));
-                at = __builtin_amdgcn_readfirstlane(at) + lane_rank(m);
-                if (take && at < kSmallCap) lds[at] = raw[q];
+                key[q] = small_key(src, raw[q], i < total ? i : total - 1, bad);
+                const uint64_t k = i < total ? place_key(key[q], i) : ~0ull;
+                less += __popcll(__ballot(k < lo));
+                take[q] = __ballot(k >= from && k < to);
+                taken += __popcll(take[q]);
             }
-            for (int o = kWave / 2; o > 0; o >>= 1) less += __shfl_xor(less, o, kWave);
-            if (lane == 0 && less) atomicAdd(&count[1], less);
+            if (taken == 0) continue;
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&count[0], taken);
+            at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+            for (int q = 0; q < kLoads; ++q) {
+                const int slot = at + lane_rank(take[q]);
+                if (((take[q] >> lane) & 1) && slot < kSmallCap) lds[slot] = key[q];
+                at += __popcll(take[q]);
+            }
         }
+        if (lane == 0 && less) atomicAdd(&count[1], less);
         __syncthreads();
         const int n = count[0];
         if (from == lo) below = count[1];
@@ -817,6 +898,33 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
                 else over = mid;
             }
             to = fits;
+            __syncthreads();
+            continue;
+        }
+        if (n <= kSmallRank) {
+            uint32_t* const sorted = lds + kSmallThreads;
+            rank[t] = 0;
+            if (t >= n && t < n + 4) lds[t] = ~0u;
+            __syncthreads();
+            rank_keys(lds, n, rank);
+            __syncthreads();
+            if (t < n) sorted[rank[t]] = lds[t];
+            __syncthreads();
+            const uint32_t k = t < n ? sorted[t] : 0u;
+            int64_t all = n, p = t;
+            bool keep = t < n;
+            if (dedup) {
+                keep = t < n && ((t == 0 && kept == 0) || k != (t > 0 ? sorted[t - 1] : prev_last));
+                p = block_exclusive_scan<kOpSum, kSmallThreads>(keep, wtot, &all);
+            }
+            if (keep) keys[below + kept + p] = k;
+            if (n > 0) {
+                if (from == lo || kept == 0) first = sorted[0];
+                prev_last = sorted[n - 1];
+            }
+            kept += static_cast<int>(all);
+            from = to;
+            to = hi;
             __syncthreads();
             continue;
         }
@@ -1156,7 +1264,8 @@ int launch_csr_build(const int64_t* row, const int64_t* col, int64_t num_edges, 
     if (l.total > 0 && l.total <= kSmallTotal && l.key_bytes == 4) {
         const bool dedup = (flags & MLXC_CSR_DEDUP) != 0;
         const int total = static_cast<int>(l.total);
-        const int ways = (total + kSmallKeys - 1) / kSmallKeys;
+        const int want = (total + kSmallKeys - 1) / kSmallKeys;
+        const int ways = want < kSmallWays ? want : kSmallWays;
         uint32_t* keys = reinterpret_cast<uint32_t*>(ws + l.keys[0]);
         SmallRange* ranges = reinterpret_cast<SmallRange*>(ws + l.hist);
         hipLaunchKernelGGL(small_sort_kernel, dim3(ways), dim3(kSmallThreads), 0, stream, src, total,

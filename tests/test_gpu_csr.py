@@ -268,10 +268,11 @@ def test_rowptr_of_2_28_nodes(cuda):
         del rowptr, c, ref
 
 
-@pytest.mark.parametrize("E", [1, 15, 512, 513, 1024, 1025, 10_556, 16_385, 98_304, 98_305])
+@pytest.mark.parametrize("E", [1, 15, 128, 129, 512, 513, 1025, 10_556, 16_385, 24_576, 24_577,
+                               98_304, 131_072, 131_073])
 @pytest.mark.parametrize("V", [3, 2708, 32768, 65536, 65537])
 def test_small_list_edges(E, V, cuda):
-    """The two-launch build around its range, block and size limits (and just
+    """The two-launch build around its range, count and size limits (and just
     past them), with the largest ids (at 65,536 nodes the key with every bit
     set), equal keys and empty rows at both ends."""
     rng = np.random.default_rng(E + V)
@@ -303,7 +304,7 @@ def test_small_list_made_for_its_sample(dedup, cuda):
     E, V = 60_000, 1000
     rng = np.random.default_rng(1)
     row, col = rng.integers(0, 90, E), rng.integers(0, V, E)
-    ns = -(-E // 512) * 4
+    ns = min(-(-E // 128), 192) * 2
     for i in range(ns):
         a, b = i * E // ns, (i + 1) * E // ns
         row[a + mix32(i) % (b - a)] = V - 1 - i % 9
