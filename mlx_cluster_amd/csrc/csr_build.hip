@@ -1043,7 +1043,10 @@ __global__ __launch_bounds__(kBlock) void small_emit_kernel(
     if (blockIdx.x == 0 && t == 1) work[1] = all;
     if (!h_status) return;
     // The last block to end publishes the status and the count: whoever waits
-    // for them may then use the arrays on any stream.
+    // for them may then use the arrays on any stream.  Every wavefront waits
+    // for its own stores before the barrier, which orders them within the block
+    // but does not wait until they have left the compute unit.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __syncthreads();
     if (t == 0) {
         __threadfence();
