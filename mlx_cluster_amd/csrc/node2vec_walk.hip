@@ -1875,7 +1875,9 @@ int launch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
 
 template <int kRule, bool kEdges, typename OutT>
 int dispatch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
-    return records_fit(a.w.num_nodes, a.w.num_edges)
+    // A group's probes and its next stretch start up to 2 * kWave past a row's
+    // end before they are compared with it (group_find): in range of Id too.
+    return records_fit(a.w.num_nodes, a.w.num_edges) && a.w.num_edges <= INT32_MAX - 4 * kWave
                ? launch_n2v_few<kRule, kEdges, OutT, int32_t>(a, stream)
                : launch_n2v_few<kRule, kEdges, OutT, int64_t>(a, stream);
 }
