@@ -120,7 +120,7 @@ int threads_for(int allowed, int64_t steps, int64_t steps_per_thread) {
 }
 
 // Uniform walks [first, last): the loop of RandomWalk.cpp:41-60, with the
-// out-of-range handling of uniform_walk_kernel (the walk stops and repeats
+// out-of-range handling of the uniform kernels (the walk stops and repeats
 // its node, edge id -1).
 template <bool kGen, typename OutT>
 uint32_t uniform_range(const HostWalk& w, int64_t first, int64_t last) {

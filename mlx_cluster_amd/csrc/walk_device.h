@@ -770,15 +770,14 @@ struct StartRecords {
 
 constexpr size_t kRecordOffset = 256;  // bytes of workspace before the records
 
-// Walks on graphs small enough for LDS (uniform_walk_lds_kernel,
-// node2vec_lds_kernel): rowptr and col as int32 in each block's LDS, for
-// calls bound by launch latency.  A workspace of kRecordOffset bytes (less
-// than any record or start-record layout) selects them.
+// Walks on graphs small enough for LDS (node2vec_lds_kernel): rowptr and col as
+// int32 in each block's LDS, for calls bound by launch latency.  A workspace of
+// kRecordOffset bytes (less than any record or start-record layout) selects
+// it, and the uniform flat walk.
 constexpr int kLdsGraphEntries = 14336;              // rowptr + col entries (56 KB)
-// Threads per block of the LDS walks.  Every block first copies the whole
+// Threads per block of the LDS walk.  Every block first copies the whole
 // graph, so the copy is the block's serial part: 1024 threads split it four
-// times finer than 256 (the reference tests' 2,000 walks of 5 steps on the
-// Cora-like graph: 11.2 -> 6.7 us per launch).
+// times finer than 256.
 constexpr int kLdsBlock = 1024;
 // Fewest walking threads per block of the node2vec LDS walk: one wavefront
 // per SIMD of the block's compute unit.
