@@ -697,7 +697,8 @@ __global__ __launch_bounds__(kBlock) void csr_emit_kernel(Store keys,
 // 3 us, of 60,000 about 15).  Radix passes need 16 to 19 launches for such a
 // list.  Kernels, 10,556 pairs over 2,708 nodes: radix 74 us, one block 38,
 // ranges of 512 sorted by the network 29, now 21; 60,000 pairs 61 -> 48;
-// to_csr of the former 93 us -> 58 -> 37 -> 31.
+// to_csr of the former 93 us -> 58 -> 37 -> 32 (33 with the wait before its
+// count is published).
 constexpr int kSmallThreads = 1024;
 // Keys of a block's range on average, while the ranges suffice.  The sort's
 // share falls with it, the sample's grows: 10,556 pairs take 29, 26, 22 and 21
@@ -1186,7 +1187,7 @@ Keys64 key_store(char* ws, const CsrLayout& l, int b, Keys64) {
 // The digit counts take 32 bits while every output position fits them, and 64
 // in larger lists: 256 of them a tile are written once, scanned and read once
 // in each pass (262,000,000 of 2^28 pairs different, over 2^24 nodes: 7.71 -> 7.63 ms;
-// 15,000,001 pairs over 1,000,003 nodes, symmetrized: 819 -> 773 us).
+// 15,000,001 pairs over 1,000,003 nodes, symmetrized: 818 -> 806 us).
 template <typename Store, typename Cnt>
 int csr_build_counted(const EdgeSrc& src, const CsrLayout& l, int32_t flags, int64_t* rowptr,
                     int64_t* col_out, char* ws, hipStream_t s) {
