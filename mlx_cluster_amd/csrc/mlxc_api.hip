@@ -231,12 +231,23 @@ __global__ void publish_status_kernel(const int64_t* work, int64_t* h_status, bo
     else publish(work[0], h_status);
 }
 
-// See launch_finish; h_status may be null.
+// See launch_finish; h_status may be null.  Bound by its loads' latency: the
+// words of 2,000 blocks a word a read, up to eight in a row a thread, against
+// two reads of four words: a validated call of 2,000 walks x 5 steps 17.7 ->
+// 16.3 us.
 __global__ __launch_bounds__(kBlock) void finish_kernel(const uint32_t* __restrict__ block_status,
                                                         int blocks, int64_t* __restrict__ work,
                                                         int64_t* h_status) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
     uint32_t bits = 0;
-    for (int i = threadIdx.x; i < blocks; i += kBlock) bits |= block_status[i];
+    const int quads = blocks / 4;
+#pragma unroll 2
+    for (int i = threadIdx.x; i < quads; i += kBlock) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(block_status + 4 * i);
+        bits |= v.x | v.y | v.z | v.w;
+    }
+    const int rest = 4 * quads + static_cast<int>(threadIdx.x);
+    if (rest < blocks) bits |= block_status[rest];
     const bool node = __syncthreads_or(bits & MLXC_STATUS_BAD_NODE);
     const bool row = __syncthreads_or(bits & MLXC_STATUS_BAD_ROW);
     if (threadIdx.x == 0) {

@@ -682,3 +682,18 @@ def test_flat_walk_edges(N, L, seeded, cuda):
             np.testing.assert_array_equal(e[at:at + N * L], e_ref.reshape(-1).astype(e.dtype))
             assert (n[:at] == -7).all() and (n[at + N * (L + 1):] == -7).all()
             assert (e[:at] == -7).all() and (e[at + N * L:] == -7).all()
+
+
+@pytest.mark.parametrize("N", [1, 3, 4, 7, 1023, 1025, 2045, 2048])
+def test_one_bad_start_is_found_in_any_block(N, cuda):
+    """Few walks run one a block; the launch after them reads the blocks' status
+    words four at a time and the rest one by one."""
+    rowptr = torch.tensor([0, 1, 2], device=cuda)
+    col = torch.tensor([1, 0], device=cuda)
+    rand = torch.zeros(N, 2, device=cuda)
+    for at in {0, N // 2, max(N - 3, 0), N - 1}:
+        start = torch.zeros(N, dtype=torch.int64, device=cuda)
+        mc.random_walk(rowptr, col, start, rand, 2)
+        start[at] = 2
+        with pytest.raises(ValueError, match="outside"):
+            mc.random_walk(rowptr, col, start, rand, 2)
