@@ -221,13 +221,22 @@ py::object to_csr(const at::Tensor& edge_index, int64_t num_nodes, int32_t flags
     at::Tensor col_out = at::empty({flags & MLXC_CSR_SYMMETRIZE ? 2 * E : E}, opts);
     at::Tensor work = at::empty({static_cast<int64_t>((ws + 7) / 8)}, opts);
     hipStream_t stream = at::hip::getCurrentHIPStream().stream();
-    const StatusTarget target(true);
-    const int rc = mlxc_csr_build(row, col, E, num_nodes, flags, rowptr.data_ptr<int64_t>(),
-                                  col_out.numel() ? col_out.data_ptr<int64_t>() : nullptr,
-                                  work.data_ptr(), static_cast<size_t>(work.numel()) * 8, stream);
+    int rc;
+    int64_t bits = 0, count = 0;
+    {
+        // A build takes up to milliseconds: other Python threads (a data
+        // loader's) run while this one launches it and waits.
+        const py::gil_scoped_release other_threads_run;
+        const StatusTarget target(true);
+        rc = mlxc_csr_build(row, col, E, num_nodes, flags, rowptr.data_ptr<int64_t>(),
+                            col_out.numel() ? col_out.data_ptr<int64_t>() : nullptr,
+                            work.data_ptr(), static_cast<size_t>(work.numel()) * 8, stream);
+        if (rc == MLXC_OK) {
+            bits = read_word(work, stream, target.words, 0);
+            count = read_word(work, stream, target.words, 1);
+        }
+    }
     if (rc != MLXC_OK) raise_code(rc, "to_csr");
-    const int64_t bits = read_word(work, stream, target.words, 0);
-    const int64_t count = read_word(work, stream, target.words, 1);
     if (bits & MLXC_STATUS_BAD_NODE)
         throw py::value_error("edge_index holds ids outside [0, num_nodes)");
     return py::make_tuple(rowptr, col_out.narrow(0, 0, count));

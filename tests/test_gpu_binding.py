@@ -5,6 +5,9 @@ The common call (tensors of the right dtype on the current device, torch's
 current stream) goes through the compiled module; every other call through
 walks.py's general path.  Both run the same libmlxc.so entry points, so the
 walks, edge ids and errors must be the same."""
+import threading
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -98,3 +101,31 @@ def test_errors_as_in_the_general_path(cuda):
     b = mc.random_walk(rowptr.cpu().numpy(), col.cpu().numpy(), start.cpu().numpy(),
                        rand.cpu().numpy(), L)
     assert torch.equal(a, b) and torch.equal(a, mc.random_walk(rowptr, col, start, rand, L))
+
+
+def test_other_threads_run_during_a_build(cuda):
+    """to_csr leaves the interpreter to other threads while it launches a build
+    and waits for it: a thread that records the time again and again has
+    times from well inside the call (a build of 2^26 pairs takes over a
+    millisecond)."""
+    row, col = synth.rmat_edges(22, 1 << 26, seed=4, device=cuda)
+    pairs = torch.stack([row, col])
+    mc.to_csr(pairs, 1 << 22)  # compiled code loaded, memory cached
+    stamps, stop = [], threading.Event()
+
+    def record():
+        while not stop.is_set():
+            stamps.append(time.perf_counter())
+            time.sleep(1e-5)
+
+    other = threading.Thread(target=record)
+    other.start()
+    calls = []
+    for _ in range(5):
+        begin = time.perf_counter()
+        mc.to_csr(pairs, 1 << 22)
+        calls.append((begin, time.perf_counter()))
+    stop.set()
+    other.join()
+    inside = sum(b + 0.2 * (e - b) < s < e - 0.2 * (e - b) for b, e in calls for s in stamps)
+    assert inside >= len(calls)
