@@ -362,10 +362,9 @@ size_t mlxc_rejection_sampling_preferred_bytes(int64_t num_nodes, int64_t num_ed
                                                int64_t num_walks, int32_t walk_length, double p,
                                                double q, int32_t rule) {
     N2VParams prm;
-    const double width = n2v_params(p, q, 0, rule, MLXC_ROWS_DETECT, prm) == MLXC_OK
-                             ? n2v_search_width(prm)
-                             : 1.0;
-    return node2vec_preferred_bytes(num_nodes, num_edges, num_walks, walk_length, width);
+    if (n2v_params(p, q, 0, rule, MLXC_ROWS_DETECT, prm) != MLXC_OK)  // (the call will fail)
+        return node2vec_workspace_bytes(num_nodes, num_edges, num_walks, walk_length, 1.0);
+    return node2vec_preferred_bytes(num_nodes, num_edges, num_walks, walk_length, prm);
 }
 
 size_t mlxc_rejection_sampling_layout_bytes(int64_t num_nodes, int64_t num_edges,

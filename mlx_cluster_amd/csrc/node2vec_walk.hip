@@ -713,8 +713,7 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 // passes):  31 M entries: 1,300 walks 361 -> 165 (the check of the 251 MB of
 // col alone takes 60), 8,000 401 -> 228, 32,768 653 -> 386, 65,536
 // 1,391 -> 607;  64 K entries: 1,300 walks 173 -> 103, 65,536 686 -> 332.
-// At 200,000 walks it is 15% ahead of the records over 31 M entries and up to
-// 14% behind them over 1 M: kN2VFewWalks.
+// Where it is chosen: n2v_few_steps.
 // Trials a group tries at once, and searches it runs at once, at most: 8 and
 // 32 trials, 1, 2 and 8 searches were within 5% or slower.
 constexpr int kFewTrials = 16;
@@ -1772,12 +1771,62 @@ size_t node2vec_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t nu
 // The few-walks kernel's workspace: the status words and as many more, so that
 // the status words alone still select the direct kernel.
 constexpr size_t kN2VFewBytes = 2 * MLXC_WORK_WORDS * sizeof(int64_t);
-constexpr int64_t kN2VFewWalks = 65536;  // see node2vec_few_kernel
+constexpr int64_t kN2VFewWalks = 65536;
+
+namespace {
+
+// The longest walks that node2vec_preferred_bytes gives the few-walks kernel.
+// It saves the other layouts' preparation, which grows with the graph, and
+// pays for it with more dependent reads a step: the row of a candidate, and a
+// search where the records have a hash table or a bitmap.  The record walk has
+// lanes to spare for those steps up to 32,768 walks (n2v_tail on 2 to 32 lanes
+// a walk) and is at its weakest just above (one lane a walk, a few wavefronts
+// per compute unit).
+//
+// Measured on 7 graphs of 54 K to 31 M entries (one with hubs of 62,500), 512
+// to 65,536 walks of 10 to 160 steps, 11 settings of p, q and the rule: in the
+// 2,230 of 3,080 calls where it is chosen the other layout's time is 0.97 to
+// 3.2 times the few-walks kernel's, 1.7 at the median.  Some of the lines (us
+// a call, other layout / few-walks kernel; p = 4, q = 3, chain but where noted):
+//   54 K entries:    2,048 walks x 160  433 / 369,  8,192 x 40  192 / 179,  x 80
+//                    269 / 318,  32,768 x 20  189 / 169,  x 40  263 / 292,
+//                    65,536 x 40  912 / 373
+//   955 K:           16,384 x 20  154 / 168 (the CSR mode),  x 40  313 / 282
+//                    (records),  x 80  459 / 520
+//   28 M with hubs:  32,768 x 20  401 / 323;  p = 0.5, q = 2:  x 40  734 / 408;
+//                    p = 4, q = 0.25, no searches:  x 20  159 / 153,  x 40  196 / 231
+//   no searches, 54 K:  2,048 x 40  74 / 72,  x 80  106 / 113,  8,192 x 20  58 / 58,
+//                       x 40  74 / 84
+int64_t n2v_few_steps(int64_t num_edges, int64_t num_walks, int32_t walk_length,
+                      const N2VParams& p) {
+    constexpr int64_t kSmall = int64_t{1} << 17, kMiddle = int64_t{1} << 21,
+                      kLarge = int64_t{1} << 22;
+    const double width = n2v_search_width(p);
+    const bool searches = width > 0.0;
+    if (num_walks > kN2VFewWalks) return 0;
+    if (num_walks > 32768) return 48;
+    if (num_walks > 8192) {
+        // Every draw may be rejected (p below 1 and q): the groups' trials,
+        // up to 16 at once, are worth more than the reads.
+        if (p.prob1 < 1.0 && p.prob2 < 1.0) return 40;
+        if (!searches) return num_edges < kSmall ? 16 : 20;
+        if (num_edges < kMiddle &&
+            !n2v_records_pay_off(num_edges, num_walks, walk_length, width))
+            return 0;  // the CSR mode's preparation is short
+        return num_walks <= 16384 && num_edges >= kSmall ? 40 : 20;
+    }
+    const int64_t scale = num_edges < kSmall ? 1 : num_edges < kLarge ? 2 : 4;
+    if (num_walks > 2048) return (searches ? 40 : 20) * scale;
+    if (searches) return num_edges < kSmall ? 160 : INT32_MAX;
+    return 40 * scale;
+}
+
+}  // namespace
 
 size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
-                                int32_t walk_length, double search_width) {
-    const size_t queried =
-        node2vec_workspace_bytes(num_nodes, num_edges, num_walks, walk_length, search_width);
+                                int32_t walk_length, const N2VParams& p) {
+    const size_t queried = node2vec_workspace_bytes(num_nodes, num_edges, num_walks, walk_length,
+                                                    n2v_search_width(p));
     if (num_nodes < 0 || num_edges < 0 || num_walks < 0 || walk_length < 0) return queried;
     if (queried == kRecordOffset) {
         // the LDS walk, with a status word for each of its blocks (at most one
@@ -1786,7 +1835,11 @@ size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t nu
         const size_t csr = n2v_layout(num_nodes, num_edges, num_walks, false).total;
         return with_words < csr ? with_words : queried;
     }
-    return num_walks > kN2VFewWalks ? queried : kN2VFewBytes;
+    // beyond int32 the other choice is the direct kernel
+    const bool few = records_fit(num_nodes, num_edges)
+                         ? walk_length <= n2v_few_steps(num_edges, num_walks, walk_length, p)
+                         : num_walks <= kN2VFewWalks;
+    return few ? kN2VFewBytes : queried;
 }
 
 size_t node2vec_layout_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,

@@ -183,7 +183,7 @@ size_t node2vec_workspace_bytes(int64_t num_nodes, int64_t num_edges, int64_t nu
 // The workspace whose walk is the fastest for the call (see
 // mlxc_rejection_sampling_preferred_bytes).
 size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
-                                int32_t walk_length, double search_width);
+                                int32_t walk_length, const N2VParams& p);
 // Bytes of one MLXC_N2V_LAYOUT_* layout (0: not available for this call).
 size_t node2vec_layout_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
                              int32_t walk_length, int32_t layout);

@@ -262,3 +262,32 @@ def test_layout_query_orders_the_layouts():
     # the records without tables or bitmaps
     assert lib.mlxc_rejection_sampling_workspace_bytes(2**20, 31_000_000, 4 * 2**20, 40, 1.0,
                                                        1.0, 0) == sizes[3]
+
+
+@pytest.mark.parametrize("V,E,N,L,p,q,rule,few", [
+    # (entries, walks, steps) on both sides of the few-walks kernel's lines
+    (1 << 20, 31_000_000, 1_300, 40, 0.5, 2.0, 0, True),
+    (1 << 20, 31_000_000, 65_536, 48, 4.0, 0.25, 1, True),
+    (1 << 20, 31_000_000, 65_536, 49, 4.0, 0.25, 1, False),
+    (1 << 20, 31_000_000, 65_537, 5, 0.5, 2.0, 0, False),
+    (500_000, 28_000_000, 32_768, 20, 4.0, 0.25, 0, True),     # no searches
+    (500_000, 28_000_000, 32_768, 40, 4.0, 0.25, 0, False),
+    (500_000, 28_000_000, 32_768, 40, 0.5, 2.0, 0, True),      # many rejections
+    (500_000, 28_000_000, 32_768, 300, 4.0, 0.25, 1, False),
+    (65_536, 955_000, 16_384, 20, 4.0, 3.0, 0, False),         # the CSR mode
+    (65_536, 955_000, 16_384, 40, 4.0, 3.0, 0, True),          # records
+    (65_536, 955_000, 2_048, 5_000, 4.0, 3.0, 0, True),
+    (4_096, 53_531, 2_048, 160, 4.0, 0.25, 1, True),
+    (4_096, 53_531, 2_048, 161, 4.0, 0.25, 1, False),
+    (4_096, 53_531, 8_192, 300, 4.0, 0.25, 1, False),
+    (4_096, 53_531, 32_768, 300, 4.0, 0.25, 1, False),
+    (4_096, 53_531, 8_192, 40, 1.0, 1.0, 0, False),
+    (4_096, 53_531, 8_192, 20, 1.0, 1.0, 0, True),
+])
+def test_preferred_bytes_of_few_walks(V, E, N, L, p, q, rule, few):
+    """node2vec calls that the record walk or the CSR mode runs faster are not
+    given the few-walks kernel's workspace."""
+    lib = _lib.load()
+    got = lib.mlxc_rejection_sampling_preferred_bytes(V, E, N, L, p, q, rule)
+    assert got == (64 if few else
+                   lib.mlxc_rejection_sampling_workspace_bytes(V, E, N, L, p, q, rule))
