@@ -706,7 +706,8 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 // blocks from walk_blocks on check the CSR beside it (the walk bounds every
 // index it uses itself).  Only the row order of MLXC_ROWS_DETECT matters to
 // it: it assumes sorted rows, and a second launch (rerun) repeats the walks
-// with scans when the check has found otherwise.
+// with scans when the check has found otherwise.  Scans are an instantiation
+// of their own (kScan), for their loads take 32 registers.
 //
 // Measured (us a call, symmetrized R-MAT, 40 steps, p = 0.5, q = 2, chain rule;
 // before: the record walk's tail phase or its queue, after the preparation
@@ -719,20 +720,54 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 constexpr int kFewTrials = 16;
 constexpr int kFewSearches = 4;
 
-// Whether tgt is in [lo, hi) of col: a search of sorted entries or a scan, by
-// the `lanes` lanes (a power of two, lane c of them) that share the arguments;
+// Entries of an unsorted row that a lane reads in one round of a scan, all in
+// flight together: a round costs a memory round trip whatever their number.
+// Unsorted rows (detected), 40 steps, p = 0.5, q = 2, chain rule, us a call, by
+// entries a round (1, 4, 8, 16):
+//   31 M entries:   1,300 walks 2,990, 1,270, 791, 530;  65,536 133,000, 54,100, 32,100, 19,900
+//   955 K entries:  1,300 walks 487, 287, 244, 225;  65,536 17,200, 6,510, 4,390, 3,430
+#ifndef MLXC_FEW_SCAN
+#define MLXC_FEW_SCAN 16
+#endif
+constexpr int kFewScan = MLXC_FEW_SCAN;
+
+// Whether tgt is in [lo, hi) of col: a search of sorted entries or (kScan) a
+// scan, by the `lanes` lanes (a power of two, lane c of them) that share the arguments;
 // `bits` selects them in a ballot shifted down by their first lane.  Every
 // lane of the wavefront calls it (with lo == hi: no search).
-template <typename Id>
-__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, bool sorted, Id lo,
-                                           Id hi, Id tgt, int lanes, int c, int first,
-                                           uint64_t bits) {
+template <bool kScan, typename Id>
+__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, Id lo, Id hi, Id tgt,
+                                           int lanes, int c, int first, uint64_t bits) {
     bool found = false;
+    if (kScan) {
+        while (__any(lo < hi)) {
+            bool hit = false;
+            const Id left = hi - lo;
+            if (lo < hi) {
+                // loaded unconditionally, the indices clamped to the row's last entry
+                Id v[kFewScan];
+#pragma unroll
+                for (int k = 0; k < kFewScan; ++k) {
+                    const Id i = k * lanes + c;
+                    v[k] = static_cast<Id>(col[i < left ? lo + i : hi - 1]);
+                }
+#pragma unroll
+                for (int k = 0; k < kFewScan; ++k) hit |= v[k] == tgt;
+            }
+            const uint64_t eq = (__ballot(hit) >> first) & bits;
+            if (lo < hi) {
+                if (eq) found = true;
+                const Id round = kFewScan * lanes;
+                lo = eq || left <= round ? hi : lo + round;
+            }
+        }
+        return found;
+    }
     while (__any(lo < hi)) {
         const Id n = hi - lo;
-        // sorted: probes at the ends of lanes + 1 equal parts, or every entry
-        // once they are no more than the lanes; unsorted: the next entries
-        const Id part = sorted && n > lanes ? (n + lanes) / (lanes + 1) : 1;
+        // probes at the ends of lanes + 1 equal parts, or every entry once
+        // they are no more than the lanes
+        const Id part = n > lanes ? (n + lanes) / (lanes + 1) : 1;
         const Id at = lo + (c + 1) * part - 1;
         const bool in = at < hi;
         Id x = 0;
@@ -743,24 +778,20 @@ __device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, bool
             if (eq) {
                 found = true;
                 lo = hi;
-            } else if (sorted) {
-                if (part == 1 && n <= lanes) {
-                    lo = hi;
-                } else {
-                    // up to the first probe that is not below tgt
-                    const Id end = lo + (below + 1) * part - 1;
-                    lo += below * part;
-                    if (below < lanes && end < hi) hi = end;
-                }
+            } else if (part == 1 && n <= lanes) {
+                lo = hi;
             } else {
-                lo = lo + lanes < hi ? lo + lanes : hi;
+                // up to the first probe that is not below tgt
+                const Id end = lo + (below + 1) * part - 1;
+                lo += below * part;
+                if (below < lanes && end < hi) hi = end;
             }
         }
     }
     return found;
 }
 
-template <int kRule, bool kEdges, typename OutT, typename Id>
+template <int kRule, bool kEdges, typename OutT, typename Id, bool kScan>
 __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int group, int steps,
                                                               int walk_blocks, bool rerun) {
     const int64_t* const rowptr = a.w.rowptr;
@@ -781,7 +812,6 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
         return;
     }
     if (rerun && a.w.work[2] == a.w.work[3]) return;  // the rows are sorted
-    const bool sorted = !rerun && a.rows != MLXC_ROWS_UNSORTED;
     extern __shared__ __align__(16) unsigned char few_lds[];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int G = group, per_wave = kWave / G;
@@ -892,8 +922,8 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
                     const Id tgt = __shfl(s_tgt, src, kWave);
                     const float rs = __shfl(r, src, kWave);
                     const bool found =
-                        group_find(col, sorted, lo, valid ? hi : lo, tgt, C, c, base + q * C,
-                                   C == kWave ? ~0ull : (1ull << C) - 1);
+                        group_find<kScan>(col, lo, valid ? hi : lo, tgt, C, c, base + q * C,
+                                          C == kWave ? ~0ull : (1ull << C) - 1);
                     const bool acc = valid && c == 0 && n2v_resolve<kRule>(a, rs, found);
                     const uint64_t won = (__ballot(acc) >> base) & group_bits;
                     if (won) {
@@ -1895,7 +1925,7 @@ constexpr int kFewCheckBlocks = 3;
 constexpr int kFewCells = 512;  // walks x positions of a wavefront's LDS stretch
 
 template <int kRule, bool kEdges, typename OutT, typename Id>
-int launch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
+int launch_n2v_few(const N2VRecArgs& a, bool searches, hipStream_t stream) {
     DeviceInfo info;
     if (int rc = device_info(info)) return rc;
     const int64_t N = a.w.num_walks, slots = static_cast<int64_t>(info.cus) * kFewLanes;
@@ -1913,13 +1943,15 @@ int launch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
         return rc;
     const size_t lds = static_cast<size_t>(kBlock / kWave) * per_wave * (steps + 1) *
                        (kEdges ? 2 : 1) * sizeof(Id);
-    auto kernel = node2vec_few_kernel<kRule, kEdges, OutT, Id>;
+    auto* search = node2vec_few_kernel<kRule, kEdges, OutT, Id, false>;
+    auto* scan = node2vec_few_kernel<kRule, kEdges, OutT, Id, true>;
     if (int rc = record_walk_event(0, stream)) return rc;
-    hipLaunchKernelGGL(kernel, dim3(walk_blocks + check_blocks), dim3(kBlock), lds, stream, a, G,
+    hipLaunchKernelGGL(a.rows == MLXC_ROWS_UNSORTED && searches ? scan : search,
+                       dim3(walk_blocks + check_blocks), dim3(kBlock), lds, stream, a, G,
                        static_cast<int>(steps), walk_blocks, false);
     MLXC_HIP_TRY(hipGetLastError());
-    if (a.rows == MLXC_ROWS_DETECT) {
-        hipLaunchKernelGGL(kernel, dim3(walk_blocks), dim3(kBlock), lds, stream, a, G,
+    if (a.rows == MLXC_ROWS_DETECT && searches) {  // (else the order does not matter)
+        hipLaunchKernelGGL(scan, dim3(walk_blocks), dim3(kBlock), lds, stream, a, G,
                            static_cast<int>(steps), walk_blocks, true);
         MLXC_HIP_TRY(hipGetLastError());
     }
@@ -1927,12 +1959,12 @@ int launch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
 }
 
 template <int kRule, bool kEdges, typename OutT>
-int dispatch_n2v_few(const N2VRecArgs& a, hipStream_t stream) {
-    // A group's probes and its next stretch start up to 2 * kWave past a row's
-    // end before they are compared with it (group_find): in range of Id too.
+int dispatch_n2v_few(const N2VRecArgs& a, bool searches, hipStream_t stream) {
+    // A group's probes lie up to kWave past a row's end before they are compared
+    // with it (group_find): in range of Id too.
     return records_fit(a.w.num_nodes, a.w.num_edges) && a.w.num_edges <= INT32_MAX - 4 * kWave
-               ? launch_n2v_few<kRule, kEdges, OutT, int32_t>(a, stream)
-               : launch_n2v_few<kRule, kEdges, OutT, int64_t>(a, stream);
+               ? launch_n2v_few<kRule, kEdges, OutT, int32_t>(a, searches, stream)
+               : launch_n2v_few<kRule, kEdges, OutT, int64_t>(a, searches, stream);
 }
 
 template <typename OutT>
@@ -2086,6 +2118,7 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
     const bool edges = w.e_out != nullptr;
     // The few-walks kernel: its workspace selects it.
     if (workspace_bytes >= kN2VFewBytes && w.num_walks <= kN2VFewWalks) {
+        const bool searches = n2v_search_width(p) > 0.0;
         if (int rc = launch_zero_work(w.work, stream)) return rc;
         N2VRecArgs a{};
         a.w = w;
@@ -2097,10 +2130,10 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
         a.key0 = p.key0;
         a.key1 = p.key1;
         if (p.rule == MLXC_RULE_REF_CHAIN)
-            return edges ? dispatch_n2v_few<MLXC_RULE_REF_CHAIN, true, OutT>(a, stream)
-                         : dispatch_n2v_few<MLXC_RULE_REF_CHAIN, false, OutT>(a, stream);
-        return edges ? dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, true, OutT>(a, stream)
-                     : dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, false, OutT>(a, stream);
+            return edges ? dispatch_n2v_few<MLXC_RULE_REF_CHAIN, true, OutT>(a, searches, stream)
+                         : dispatch_n2v_few<MLXC_RULE_REF_CHAIN, false, OutT>(a, searches, stream);
+        return edges ? dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, true, OutT>(a, searches, stream)
+                     : dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, false, OutT>(a, searches, stream);
     }
     // Graphs beyond int32, a workspace too small for the records, or output
     // buffers not 16-byte aligned: the direct CSR kernel.  The CSR check

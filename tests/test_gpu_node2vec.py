@@ -739,3 +739,39 @@ def test_few_walks_kernel_reports_malformed_graphs(cuda):
                                          n.data_ptr(), None, _lib.MLXC_OUT_INT64, ws.data_ptr(),
                                          64, torch.cuda.current_stream().cuda_stream)
         assert rc == 0 and int(ws[0]) == bits, what
+
+
+@pytest.mark.parametrize("N,L", [(300, 9), (5_000, 7), (9_000, 6), (40_000, 5), (65_536, 4)])
+@pytest.mark.parametrize("rule", [0, 1])
+def test_few_walks_kernel_on_unsorted_rows(N, L, rule, cuda):
+    """The few-walks kernel on unsorted rows of lengths around whole rounds of a
+    scan for every group width (16 entries a lane), given and detected; the
+    neighbour looked for stands anywhere in the row, or is not there."""
+    from mlx_cluster_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(N)
+    V = 6000
+    deg = rng.integers(1, 12, V)
+    deg[:18] = [15, 16, 17, 31, 32, 33, 63, 64, 65, 255, 256, 257, 1023, 1024, 1025, 2048, 2049, 0]
+    rowptr = np.concatenate([[0], np.cumsum(deg)])
+    col = rng.integers(0, V, rowptr[-1])
+    for v in range(18):  # much of a long row lies in the other long rows
+        row = rng.permutation(V)[:deg[v]]
+        row[: deg[v] // 2] = rng.integers(0, 18, deg[v] // 2)
+        col[rowptr[v]:rowptr[v + 1]] = rng.permutation(row)
+    start = np.where(np.arange(N) % 3 < 2, np.arange(N) % 18, rng.integers(0, V, N))
+    n_ref, e_ref, st, _ = oracle.node2vec_walk(rowptr, col, start, L, 0.5, 3.0, 5, rule=rule,
+                                               rows_sorted=False, with_edges=True)
+    assert st == 0
+    rp, cl, s = (torch.from_numpy(a.astype(np.int64)).to(cuda) for a in (rowptr, col, start))
+    for rows in (_lib.MLXC_ROWS_UNSORTED, _lib.MLXC_ROWS_DETECT):
+        n = torch.empty((N, L + 1), dtype=torch.int64, device=cuda)
+        e = torch.empty((N, L), dtype=torch.int64, device=cuda)
+        ws = torch.full((8,), 5, dtype=torch.int64, device=cuda)
+        rc = lib.mlxc_rejection_sampling(
+            rp.data_ptr(), V, cl.data_ptr(), cl.numel(), s.data_ptr(), N, L, 0.5, 3.0, 5, 0, rule,
+            rows, n.data_ptr(), e.data_ptr(), _lib.MLXC_OUT_INT64, ws.data_ptr(), 64,
+            torch.cuda.current_stream().cuda_stream)
+        assert rc == 0 and int(ws[0]) == 0
+        np.testing.assert_array_equal(n.cpu().numpy(), n_ref)
+        np.testing.assert_array_equal(e.cpu().numpy(), e_ref)
