@@ -1815,8 +1815,8 @@ namespace {
 //
 // Measured on 7 graphs of 54 K to 31 M entries (one with hubs of 62,500), 512
 // to 65,536 walks of 10 to 160 steps, 11 settings of p, q and the rule: in the
-// 2,230 of 3,080 calls where it is chosen the other layout's time is 0.97 to
-// 3.2 times the few-walks kernel's, 1.7 at the median.  Some of the lines (us
+// 2,426 of 3,080 calls where it is chosen the other layout's time is 0.97 to
+// 3.9 times the few-walks kernel's, 1.7 at the median.  Some of the lines (us
 // a call, other layout / few-walks kernel; p = 4, q = 3, chain but where noted):
 //   54 K entries:    2,048 walks x 160  433 / 369,  8,192 x 40  192 / 179,  x 80
 //                    269 / 318,  32,768 x 20  189 / 169,  x 40  263 / 292,
@@ -1834,11 +1834,13 @@ int64_t n2v_few_steps(int64_t num_edges, int64_t num_walks, int32_t walk_length,
     const double width = n2v_search_width(p);
     const bool searches = width > 0.0;
     if (num_walks > kN2VFewWalks) return 0;
-    if (num_walks > 32768) return 48;
+    // Where every draw may be rejected (p below 1 and q) the groups' trials, up
+    // to 16 at once, are worth more than the reads.
+    const bool rejects = p.prob1 < 1.0 && p.prob2 < 1.0;
+    if (num_walks > 32768)
+        return rejects ? 320 : searches && p.rule == MLXC_RULE_REF_CHAIN ? 160 : 48;
     if (num_walks > 8192) {
-        // Every draw may be rejected (p below 1 and q): the groups' trials,
-        // up to 16 at once, are worth more than the reads.
-        if (p.prob1 < 1.0 && p.prob2 < 1.0) return 40;
+        if (rejects) return 40;
         if (!searches) return num_edges < kSmall ? 16 : 20;
         if (num_edges < kMiddle &&
             !n2v_records_pay_off(num_edges, num_walks, walk_length, width))
@@ -1847,8 +1849,7 @@ int64_t n2v_few_steps(int64_t num_edges, int64_t num_walks, int32_t walk_length,
     }
     const int64_t scale = num_edges < kSmall ? 1 : num_edges < kLarge ? 2 : 4;
     if (num_walks > 2048) return (searches ? 40 : 20) * scale;
-    if (searches) return num_edges < kSmall ? 160 : INT32_MAX;
-    return 40 * scale;
+    return searches ? INT32_MAX : 40 * scale;
 }
 
 }  // namespace

@@ -277,8 +277,12 @@ def test_layout_query_orders_the_layouts():
     (65_536, 955_000, 16_384, 20, 4.0, 3.0, 0, False),         # the CSR mode
     (65_536, 955_000, 16_384, 40, 4.0, 3.0, 0, True),          # records
     (65_536, 955_000, 2_048, 5_000, 4.0, 3.0, 0, True),
-    (4_096, 53_531, 2_048, 160, 4.0, 0.25, 1, True),
-    (4_096, 53_531, 2_048, 161, 4.0, 0.25, 1, False),
+    (1 << 20, 31_000_000, 65_536, 160, 4.0, 3.0, 0, True),
+    (1 << 20, 31_000_000, 65_536, 161, 4.0, 3.0, 0, False),
+    (1 << 20, 31_000_000, 65_536, 320, 0.5, 2.0, 1, True),
+    (1 << 20, 31_000_000, 65_536, 321, 0.5, 2.0, 1, False),
+    (4_096, 53_531, 2_048, 300, 4.0, 0.25, 1, True),
+    (4_096, 53_531, 2_049, 300, 4.0, 0.25, 1, False),
     (4_096, 53_531, 8_192, 300, 4.0, 0.25, 1, False),
     (4_096, 53_531, 32_768, 300, 4.0, 0.25, 1, False),
     (4_096, 53_531, 8_192, 40, 1.0, 1.0, 0, False),
