@@ -60,33 +60,39 @@ struct CsrCheck {
             }
         }
     }
-    // Adds the block's totals to the given words, one atomic each from
-    // thread 0: the status bits, and the descents that start no row
-    // (desc - start_desc, zero exactly when the rows are sorted) to
-    // diff_word.  Every thread of the block calls it.  (Atomics on one word
-    // serialize: three per wavefront, 49,000 per call, took 0.3 ms of the
-    // 0.42 ms pass over configuration 3's 31 M entries.)
-    __device__ void flush(unsigned long long* bits_word, uint32_t rowptr_bit, uint32_t col_bit,
-                          unsigned long long* diff_word) {
+    // The block's totals, in thread 0: the status bits, and the descents that
+    // start no row (desc - start_desc, over all blocks zero exactly when the
+    // rows are sorted).  Every thread of the block calls it.
+    __device__ void totals(uint32_t rowptr_bit, uint32_t col_bit, uint32_t& bits, int64_t& diff) {
         __shared__ uint32_t block_bits[kBlock / kWave];
         __shared__ int64_t block_diff[kBlock / kWave];
-        const uint32_t bits = wave_or((bad_rowptr ? rowptr_bit : 0u) | (bad_col ? col_bit : 0u));
+        const uint32_t wave_bits =
+            wave_or((bad_rowptr ? rowptr_bit : 0u) | (bad_col ? col_bit : 0u));
         const int64_t d = wave_sum(desc - start_desc);
         if (__lane_id() == 0) {
-            block_bits[threadIdx.x / kWave] = bits;
+            block_bits[threadIdx.x / kWave] = wave_bits;
             block_diff[threadIdx.x / kWave] = d;
         }
         __syncthreads();
+        bits = 0;
+        diff = 0;
         if (threadIdx.x == 0) {
-            uint32_t b = 0;
-            int64_t t = 0;
             for (int i = 0; i < kBlock / kWave; ++i) {
-                b |= block_bits[i];
-                t += block_diff[i];
+                bits |= block_bits[i];
+                diff += block_diff[i];
             }
-            if (b) atomicOr(bits_word, static_cast<unsigned long long>(b));
-            if (t) atomicAdd(diff_word, static_cast<unsigned long long>(t));
         }
+    }
+    // Adds the totals to the given words, one atomic each from thread 0.
+    // (Atomics on one word serialize: three per wavefront, 49,000 per call,
+    // took 0.3 ms of the 0.42 ms pass over configuration 3's 31 M entries.)
+    __device__ void flush(unsigned long long* bits_word, uint32_t rowptr_bit, uint32_t col_bit,
+                          unsigned long long* diff_word) {
+        uint32_t bits;
+        int64_t diff;
+        totals(rowptr_bit, col_bit, bits, diff);
+        if (bits) atomicOr(bits_word, static_cast<unsigned long long>(bits));
+        if (diff) atomicAdd(diff_word, static_cast<unsigned long long>(diff));
     }
 };
 

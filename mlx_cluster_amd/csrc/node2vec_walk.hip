@@ -705,9 +705,10 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 // The call must validate the whole graph.  The walk does not wait for that:
 // blocks from walk_blocks on check the CSR beside it (the walk bounds every
 // index it uses itself).  Only the row order of MLXC_ROWS_DETECT matters to
-// it: it assumes sorted rows, and a second launch (rerun) repeats the walks
+// it: it assumes sorted rows, and a second launch (kAgain) repeats the walks
 // with scans when the check has found otherwise.  Scans are an instantiation
-// of their own (kScan), for their loads take 32 registers.
+// of their own (kScan), for their loads take 32 registers.  Calls with row
+// tables check first (kChecked).
 //
 // Measured (us a call, symmetrized R-MAT, 40 steps, p = 0.5, q = 2, chain rule;
 // before: the record walk's tail phase or its queue, after the preparation
@@ -720,6 +721,13 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 constexpr int kFewTrials = 16;
 constexpr int kFewSearches = 4;
 
+// What a launch of the few-walks kernel does.
+enum class FewPass {
+    kBeside,   // walks, and checks the graph in blocks beside them
+    kAgain,    // walks again, with scans, if that check found unsorted rows
+    kChecked,  // walks after few_check_kernel and few_table_kernel
+};
+
 // Entries of an unsorted row that a lane reads in one round of a scan, all in
 // flight together: a round costs a memory round trip whatever their number.
 // Unsorted rows (detected), 40 steps, p = 0.5, q = 2, chain rule, us a call, by
@@ -731,15 +739,153 @@ constexpr int kFewSearches = 4;
 #endif
 constexpr int kFewScan = MLXC_FEW_SCAN;
 
-// Whether tgt is in [lo, hi) of col: a search of sorted entries or (kScan) a
-// scan, by the `lanes` lanes (a power of two, lane c of them) that share the arguments;
+// Row tables: for calls whose other layout would be the records with their
+// hash tables, a hash set of every row, so that an unsorted row is not scanned
+// here either.  Row [b, e) has the 2 (e - b) slots from 2 b on (ids, -1: empty),
+// filled by linear probing from row_slot; half of them stay empty, so a probe
+// ends, and as a rule in the first read of a group's lanes.  Filled only once
+// the check has found the graph well formed and its rows (DETECT) unsorted.
+//
+// Such a call checks the graph first (few_check_kernel, a word pair a block, no
+// reset before it), then gathers the pairs and fills the tables in one launch
+// (few_table_kernel): on graphs this small for the call that costs sorted rows
+// no more than the launch that would repeat the walks.
+// Unsorted rows (detected), 40 steps, us a call, records / scans / tables:
+//   54 K entries, p = 0.5, q = 2, chain:   1,300 walks 178 / 171 / 114,
+//                                          65,536 walks 839 / 1,088 / 251
+//   955 K, p = 4, q = 0.25, analytic:      1,300 walks 273 / 288 / 192,
+//                                          65,536 walks 531 / 6,267 / 363
+__device__ __forceinline__ uint32_t row_slot(int32_t id, int64_t slots) {
+    return static_cast<uint32_t>(
+        (static_cast<uint64_t>(static_cast<uint32_t>(id) * 0x9E3779B1u) * static_cast<uint64_t>(slots)) >> 32);
+}
+
+// What one block of few_check_kernel found.
+struct FewChecked {
+    int64_t diff;  // see CsrCheck::totals
+    int64_t bits;  // MLXC_STATUS_*
+};
+constexpr int kFewChecked = 512;  // blocks of few_check_kernel at most
+
+// The check of the graph, as the blocks beside the walks do it, and -1 in
+// every slot of the tables.
+__global__ __launch_bounds__(kBlock) void few_check_kernel(const int64_t* __restrict__ rowptr,
+                                                           int64_t V,
+                                                           const int64_t* __restrict__ col,
+                                                           int64_t E, int4* __restrict__ table,
+                                                           FewChecked* __restrict__ found) {
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
+    const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    for (int64_t i = gid; 2 * i < E; i += stride) table[i] = make_int4(-1, -1, -1, -1);
+    CsrCheck check;
+    if (reinterpret_cast<uintptr_t>(col) % 16 == 0)
+        check.edges4(col, V, E, gid, stride);
+    else
+        for (int64_t i = gid; i < E; i += stride) check.edge(col, V, i, col[i]);
+    check.nodes(rowptr, V, col, E, gid, stride);
+    uint32_t bits;
+    int64_t diff;
+    check.totals(MLXC_STATUS_BAD_ROW, MLXC_STATUS_BAD_NODE, bits, diff);
+    if (threadIdx.x == 0) found[blockIdx.x] = FewChecked{diff, static_cast<int64_t>(bits)};
+}
+
+// Sets the call's words: 0 to the check's status bits, 1 to whether the walks
+// may use the tables, 2 and 3 to compare equal when the rows are sorted; and
+// inserts every entry into its row's table: runs of kTableRun consecutive
+// entries a thread, whatever the rows' lengths.
+constexpr int kTableRun = 4;
+__global__ __launch_bounds__(kBlock) void few_table_kernel(const int64_t* __restrict__ rowptr,
+                                                           int64_t V,
+                                                           const int64_t* __restrict__ col,
+                                                           int64_t E, int32_t rows,
+                                                           const FewChecked* __restrict__ found,
+                                                           int blocks, int64_t* __restrict__ work,
+                                                           int32_t* table) {
+    __shared__ int64_t wave_diff[kBlock / kWave];
+    int64_t d = 0, all = 0;
+    uint32_t b0 = 0;
+    for (int i = threadIdx.x; i < blocks; i += kBlock) {
+        d += found[i].diff;
+        b0 |= static_cast<uint32_t>(found[i].bits);
+    }
+    d = wave_sum(d);
+    if (__lane_id() == 0) wave_diff[threadIdx.x / kWave] = d;
+    const bool bad_node = __syncthreads_or(b0 & MLXC_STATUS_BAD_NODE);
+    const bool bad_row = __syncthreads_or(b0 & MLXC_STATUS_BAD_ROW);
+    for (int i = 0; i < kBlock / kWave; ++i) all += wave_diff[i];
+    // (a malformed graph has no tables: the walks scan it)
+    const bool fill = !bad_node && !bad_row && (rows == MLXC_ROWS_UNSORTED || all != 0);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        work[0] = (bad_node ? MLXC_STATUS_BAD_NODE : 0) | (bad_row ? MLXC_STATUS_BAD_ROW : 0);
+        work[1] = fill ? 1 : 0;
+        work[2] = all;
+        work[3] = 0;
+    }
+    if (!fill) return;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
+    const int64_t gid = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    for (int64_t i0 = gid * kTableRun; i0 < E; i0 += stride * kTableRun) {
+        const int64_t i1 = i0 + kTableRun < E ? i0 + kTableRun : E;
+        int64_t b = 0, e = 0;
+        for (int64_t i = i0; i < i1; ++i) {
+            if (i >= e) {  // the row of entry i: the last that starts at or before it
+                int64_t lo = 0, hi = V;  // rowptr[lo] <= i < rowptr[hi]
+                while (hi - lo > 1) {
+                    const int64_t mid = (lo + hi) / 2;
+                    if (rowptr[mid] <= i) lo = mid;
+                    else hi = mid;
+                }
+                b = rowptr[lo];
+                e = rowptr[lo + 1];
+            }
+            const int64_t slots = 2 * (e - b);
+            const int32_t id = static_cast<int32_t>(col[i]);
+            int32_t* const row = table + 2 * b;
+            int64_t s = row_slot(id, slots);
+            while (true) {  // fewer entries than slots: one is empty or holds id
+                const int32_t was = atomicCAS(row + s, -1, id);
+                if (was == -1 || was == id) break;
+                s = s + 1 == slots ? 0 : s + 1;
+            }
+        }
+    }
+}
+
+// Whether tgt is in the row [lo, hi) by its table; arguments as group_find's.
+__device__ __forceinline__ bool group_lookup(const int32_t* __restrict__ table, int32_t lo,
+                                             int32_t hi, int32_t tgt, int lanes, int c, int first,
+                                             uint64_t bits) {
+    const int64_t slots = 2 * (static_cast<int64_t>(hi) - lo);
+    const int32_t* const row = table + 2 * static_cast<int64_t>(lo);
+    const int64_t home = row_slot(tgt, slots);
+    bool found = false;
+    int64_t tried = 0;
+    while (__any(tried < slots)) {
+        int32_t x = -2;
+        if (tried + c < slots) {
+            const int64_t s = home + tried + c;
+            x = row[s < slots ? s : s - slots];
+        }
+        const uint64_t eq = (__ballot(x == tgt) >> first) & bits;
+        const uint64_t open = (__ballot(x == -1) >> first) & bits;
+        if (tried < slots) {
+            if (eq) found = true;
+            tried = eq || open ? slots : tried + lanes;
+        }
+    }
+    return found;
+}
+
+// Whether tgt is in [lo, hi) of col: a search of sorted entries or a scan,
+// by the `lanes` lanes (a power of two, lane c of them) that share the arguments;
 // `bits` selects them in a ballot shifted down by their first lane.  Every
 // lane of the wavefront calls it (with lo == hi: no search).
-template <bool kScan, typename Id>
-__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, Id lo, Id hi, Id tgt,
-                                           int lanes, int c, int first, uint64_t bits) {
+template <typename Id>
+__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, bool scan, Id lo,
+                                           Id hi, Id tgt, int lanes, int c, int first,
+                                           uint64_t bits) {
     bool found = false;
-    if (kScan) {
+    if (scan) {
         while (__any(lo < hi)) {
             bool hit = false;
             const Id left = hi - lo;
@@ -793,10 +939,11 @@ __device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, Id l
 
 template <int kRule, bool kEdges, typename OutT, typename Id, bool kScan>
 __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int group, int steps,
-                                                              int walk_blocks, bool rerun) {
+                                                              int walk_blocks, FewPass pass,
+                                                              const int32_t* table) {
     const int64_t* const rowptr = a.w.rowptr;
     const int64_t* const col = a.w.col;
-    if (!rerun && blockIdx.x >= static_cast<unsigned>(walk_blocks)) {
+    if (pass == FewPass::kBeside && blockIdx.x >= static_cast<unsigned>(walk_blocks)) {
         CsrCheck check;
         const int64_t stride = static_cast<int64_t>(gridDim.x - walk_blocks) * kBlock;
         const int64_t gid =
@@ -811,7 +958,11 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
         check.flush(w, MLXC_STATUS_BAD_ROW, MLXC_STATUS_BAD_NODE, w + 2);
         return;
     }
-    if (rerun && a.w.work[2] == a.w.work[3]) return;  // the rows are sorted
+    if (pass == FewPass::kAgain && a.w.work[2] == a.w.work[3]) return;  // the rows are sorted
+    // (kScan false: the rows are taken as sorted)
+    const bool scan = kScan && (pass != FewPass::kChecked || a.rows == MLXC_ROWS_UNSORTED ||
+                                a.w.work[2] != a.w.work[3]);
+    const bool tables = kScan && scan && pass == FewPass::kChecked && a.w.work[1] == 1;
     extern __shared__ __align__(16) unsigned char few_lds[];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int G = group, per_wave = kWave / G;
@@ -921,9 +1072,13 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
                     const Id hi = __shfl(s_hi, src, kWave);
                     const Id tgt = __shfl(s_tgt, src, kWave);
                     const float rs = __shfl(r, src, kWave);
+                    const uint64_t bits = C == kWave ? ~0ull : (1ull << C) - 1;
                     const bool found =
-                        group_find<kScan>(col, lo, valid ? hi : lo, tgt, C, c, base + q * C,
-                                          C == kWave ? ~0ull : (1ull << C) - 1);
+                        tables ? group_lookup(table, static_cast<int32_t>(lo),
+                                              static_cast<int32_t>(valid ? hi : lo),
+                                              static_cast<int32_t>(tgt), C, c, base + q * C, bits)
+                               : group_find(col, scan, lo, valid ? hi : lo, tgt, C, c, base + q * C,
+                                            bits);
                     const bool acc = valid && c == 0 && n2v_resolve<kRule>(a, rs, found);
                     const uint64_t won = (__ballot(acc) >> base) & group_bits;
                     if (won) {
@@ -1805,6 +1960,24 @@ constexpr int64_t kN2VFewWalks = 65536;
 
 namespace {
 
+// ... with row tables: two int32 slots an entry, stored in fours, and the
+// check's results.
+size_t few_table_bytes(int64_t num_edges) {
+    return kN2VFewBytes + static_cast<size_t>(num_edges + 1) / 2 * sizeof(int4) +
+           kFewChecked * sizeof(FewChecked);
+}
+
+// Whether unsorted rows take the tables, where the records would pay.  In
+// shorter calls scans are no slower than the records (54 K entries, p = 4,
+// q = 3, chain, records / scans: 1,300 walks x 20 136 / 124 us a call, x 40
+// 187 / 214, 8,192 x 5 101 / 74, 4,096 x 20 135 / 150), and sorted rows are
+// spared the 2 us by which the check before the walks is longer than the one
+// beside them (8,192 x 5, detected: 50 and 52 us; x 40 151 and 154).
+bool few_tables_pay(int64_t num_edges, int64_t num_walks, int32_t walk_length, double width) {
+    return width > 0.0 && num_edges > 0 && (walk_length > 20 || num_walks * walk_length > 65536) &&
+           n2v_records_pay_off(num_edges, num_walks, walk_length, width);
+}
+
 // The longest walks that node2vec_preferred_bytes gives the few-walks kernel.
 // It saves the other layouts' preparation, which grows with the graph, and
 // pays for it with more dependent reads a step: the row of a candidate, and a
@@ -1870,7 +2043,11 @@ size_t node2vec_preferred_bytes(int64_t num_nodes, int64_t num_edges, int64_t nu
     const bool few = records_fit(num_nodes, num_edges)
                          ? walk_length <= n2v_few_steps(num_edges, num_walks, walk_length, p)
                          : num_walks <= kN2VFewWalks;
-    return few ? kN2VFewBytes : queried;
+    if (!few) return queried;
+    return records_fit(num_nodes, num_edges) &&
+                   few_tables_pay(num_edges, num_walks, walk_length, n2v_search_width(p))
+               ? few_table_bytes(num_edges)
+               : kN2VFewBytes;
 }
 
 size_t node2vec_layout_bytes(int64_t num_nodes, int64_t num_edges, int64_t num_walks,
@@ -1926,7 +2103,7 @@ constexpr int kFewCheckBlocks = 3;
 constexpr int kFewCells = 512;  // walks x positions of a wavefront's LDS stretch
 
 template <int kRule, bool kEdges, typename OutT, typename Id>
-int launch_n2v_few(const N2VRecArgs& a, bool searches, hipStream_t stream) {
+int launch_n2v_few(const N2VRecArgs& a, bool searches, int32_t* table, hipStream_t stream) {
     DeviceInfo info;
     if (int rc = device_info(info)) return rc;
     const int64_t N = a.w.num_walks, slots = static_cast<int64_t>(info.cus) * kFewLanes;
@@ -1946,31 +2123,84 @@ int launch_n2v_few(const N2VRecArgs& a, bool searches, hipStream_t stream) {
                        (kEdges ? 2 : 1) * sizeof(Id);
     auto* search = node2vec_few_kernel<kRule, kEdges, OutT, Id, false>;
     auto* scan = node2vec_few_kernel<kRule, kEdges, OutT, Id, true>;
+    const dim3 block(kBlock);
+    const int len = static_cast<int>(steps);
+    if (table) {
+        const WalkArgs& w = a.w;
+        FewChecked* const found =
+            reinterpret_cast<FewChecked*>(reinterpret_cast<int4*>(table) + (w.num_edges + 1) / 2);
+        int checks = 0, grid = 0;
+        if (int rc = stream_grid(quads > w.num_nodes ? quads : w.num_nodes, 2, checks)) return rc;
+        if (checks > kFewChecked) checks = kFewChecked;
+        hipLaunchKernelGGL(few_check_kernel, dim3(checks), block, 0, stream, w.rowptr, w.num_nodes,
+                           w.col, w.num_edges, reinterpret_cast<int4*>(table), found);
+        MLXC_HIP_TRY(hipGetLastError());
+        if (int rc = stream_grid((w.num_edges + kTableRun - 1) / kTableRun, 2, grid)) return rc;
+        hipLaunchKernelGGL(few_table_kernel, dim3(grid), block, 0, stream, w.rowptr, w.num_nodes,
+                           w.col, w.num_edges, a.rows, found, checks, w.work, table);
+        MLXC_HIP_TRY(hipGetLastError());
+        if (int rc = record_walk_event(0, stream)) return rc;
+        hipLaunchKernelGGL(scan, dim3(walk_blocks), block, lds, stream, a, G, len, walk_blocks,
+                           FewPass::kChecked, table);
+        MLXC_HIP_TRY(hipGetLastError());
+        return record_walk_event(1, stream);
+    }
+    if (int rc = launch_zero_work(a.w.work, stream)) return rc;
     if (int rc = record_walk_event(0, stream)) return rc;
     hipLaunchKernelGGL(a.rows == MLXC_ROWS_UNSORTED && searches ? scan : search,
-                       dim3(walk_blocks + check_blocks), dim3(kBlock), lds, stream, a, G,
-                       static_cast<int>(steps), walk_blocks, false);
+                       dim3(walk_blocks + check_blocks), block, lds, stream, a, G, len,
+                       walk_blocks, FewPass::kBeside, nullptr);
     MLXC_HIP_TRY(hipGetLastError());
     if (a.rows == MLXC_ROWS_DETECT && searches) {  // (else the order does not matter)
-        hipLaunchKernelGGL(scan, dim3(walk_blocks), dim3(kBlock), lds, stream, a, G,
-                           static_cast<int>(steps), walk_blocks, true);
+        hipLaunchKernelGGL(scan, dim3(walk_blocks), block, lds, stream, a, G, len, walk_blocks,
+                           FewPass::kAgain, nullptr);
         MLXC_HIP_TRY(hipGetLastError());
     }
     return record_walk_event(1, stream);
 }
 
 template <int kRule, bool kEdges, typename OutT>
-int dispatch_n2v_few(const N2VRecArgs& a, bool searches, hipStream_t stream) {
+int dispatch_n2v_few(const N2VRecArgs& a, bool searches, int32_t* table, hipStream_t stream) {
     // A group's probes lie up to kWave past a row's end before they are compared
     // with it (group_find): in range of Id too.
     return records_fit(a.w.num_nodes, a.w.num_edges) && a.w.num_edges <= INT32_MAX - 4 * kWave
-               ? launch_n2v_few<kRule, kEdges, OutT, int32_t>(a, searches, stream)
-               : launch_n2v_few<kRule, kEdges, OutT, int64_t>(a, searches, stream);
+               ? launch_n2v_few<kRule, kEdges, OutT, int32_t>(a, searches, table, stream)
+               : launch_n2v_few<kRule, kEdges, OutT, int64_t>(a, searches, nullptr, stream);
+}
+
+// table: few_table_bytes() - kN2VFewBytes of workspace for the row tables, or
+// null for none.
+template <typename OutT>
+int launch_n2v_few_typed(const WalkArgs& w, const N2VParams& p, int32_t* table,
+                         hipStream_t stream) {
+    N2VRecArgs a{};
+    a.w = w;
+    a.rows = p.rows;
+    a.symmetric = p.symmetric;
+    a.thr0 = float_at_or_above(p.prob0);
+    a.thr1 = float_at_or_above(p.prob1);
+    a.thr2 = float_at_or_above(p.prob2);
+    a.key0 = p.key0;
+    a.key1 = p.key1;
+    const bool searches = n2v_search_width(p) > 0.0;
+    if (!searches || p.rows == MLXC_ROWS_SORTED || w.num_edges == 0) table = nullptr;
+    const bool edges = w.e_out != nullptr;
+    if (p.rule == MLXC_RULE_REF_CHAIN)
+        return edges ? dispatch_n2v_few<MLXC_RULE_REF_CHAIN, true, OutT>(a, searches, table, stream)
+                     : dispatch_n2v_few<MLXC_RULE_REF_CHAIN, false, OutT>(a, searches, table, stream);
+    return edges ? dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, true, OutT>(a, searches, table, stream)
+                 : dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, false, OutT>(a, searches, table, stream);
 }
 
 template <typename OutT>
 int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace,
                           size_t workspace_bytes, hipStream_t stream) {
+    // The few-walks kernel with row tables: exactly its workspace selects it,
+    // which other layouts would fit into too.
+    if (w.num_walks <= kN2VFewWalks && records_fit(w.num_nodes, w.num_edges) &&
+        workspace_bytes == few_table_bytes(w.num_edges))
+        return launch_n2v_few_typed<OutT>(
+            w, p, reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + kN2VFewBytes), stream);
     const bool aligned = reinterpret_cast<uintptr_t>(w.n_out) % 16 == 0 &&
                          reinterpret_cast<uintptr_t>(w.e_out) % 16 == 0;  // e_out may be null
     const N2VLayout lay_rec = n2v_layout(w.num_nodes, w.num_edges, w.num_walks, true);
@@ -2116,26 +2346,9 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
         if (int rc = record_walk_event(1, stream)) return rc;
         return a.w.block_status ? launch_finish(a.w.block_status, blocks, w.work, stream) : MLXC_OK;
     }
-    const bool edges = w.e_out != nullptr;
     // The few-walks kernel: its workspace selects it.
-    if (workspace_bytes >= kN2VFewBytes && w.num_walks <= kN2VFewWalks) {
-        const bool searches = n2v_search_width(p) > 0.0;
-        if (int rc = launch_zero_work(w.work, stream)) return rc;
-        N2VRecArgs a{};
-        a.w = w;
-        a.rows = p.rows;
-        a.symmetric = p.symmetric;
-        a.thr0 = float_at_or_above(p.prob0);
-        a.thr1 = float_at_or_above(p.prob1);
-        a.thr2 = float_at_or_above(p.prob2);
-        a.key0 = p.key0;
-        a.key1 = p.key1;
-        if (p.rule == MLXC_RULE_REF_CHAIN)
-            return edges ? dispatch_n2v_few<MLXC_RULE_REF_CHAIN, true, OutT>(a, searches, stream)
-                         : dispatch_n2v_few<MLXC_RULE_REF_CHAIN, false, OutT>(a, searches, stream);
-        return edges ? dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, true, OutT>(a, searches, stream)
-                     : dispatch_n2v_few<MLXC_RULE_NODE2VEC_EXACT, false, OutT>(a, searches, stream);
-    }
+    if (workspace_bytes >= kN2VFewBytes && w.num_walks <= kN2VFewWalks)
+        return launch_n2v_few_typed<OutT>(w, p, nullptr, stream);
     // Graphs beyond int32, a workspace too small for the records, or output
     // buffers not 16-byte aligned: the direct CSR kernel.  The CSR check
     // validates the whole graph as the other layouts do; csr_status_kernel
@@ -2153,6 +2366,7 @@ int launch_node2vec_typed(const WalkArgs& w, const N2VParams& p, void* workspace
     a.key0 = p.key0;
     a.key1 = p.key1;
     a.rows = p.rows;
+    const bool edges = w.e_out != nullptr;
     return p.rule == MLXC_RULE_REF_CHAIN
                ? dispatch_n2v<MLXC_RULE_REF_CHAIN, OutT>(a, edges, stream)
                : dispatch_n2v<MLXC_RULE_NODE2VEC_EXACT, OutT>(a, edges, stream);

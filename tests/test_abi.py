@@ -287,11 +287,18 @@ def test_layout_query_orders_the_layouts():
     (4_096, 53_531, 32_768, 300, 4.0, 0.25, 1, False),
     (4_096, 53_531, 8_192, 40, 1.0, 1.0, 0, False),
     (4_096, 53_531, 8_192, 20, 1.0, 1.0, 0, True),
+    (4_096, 53_531, 8_192, 4, 0.5, 2.0, 0, True),              # no tables
 ])
 def test_preferred_bytes_of_few_walks(V, E, N, L, p, q, rule, few):
     """node2vec calls that the record walk or the CSR mode runs faster are not
     given the few-walks kernel's workspace."""
     lib = _lib.load()
     got = lib.mlxc_rejection_sampling_preferred_bytes(V, E, N, L, p, q, rule)
-    assert got == (64 if few else
-                   lib.mlxc_rejection_sampling_workspace_bytes(V, E, N, L, p, q, rule))
+    other = lib.mlxc_rejection_sampling_workspace_bytes(V, E, N, L, p, q, rule)
+    if not few:
+        assert got == other
+    elif (L > 20 or N * L > 65536) and other >= lib.mlxc_rejection_sampling_layout_bytes(
+            V, E, N, L, _lib.MLXC_N2V_LAYOUT_RECORDS_HASH):
+        assert got == 64 + (E + 1) // 2 * 16 + 8192  # the row tables, for unsorted rows
+    else:
+        assert got == 64

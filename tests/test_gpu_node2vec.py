@@ -745,8 +745,11 @@ def test_few_walks_kernel_reports_malformed_graphs(cuda):
 @pytest.mark.parametrize("rule", [0, 1])
 def test_few_walks_kernel_on_unsorted_rows(N, L, rule, cuda):
     """The few-walks kernel on unsorted rows of lengths around whole rounds of a
-    scan for every group width (16 entries a lane), given and detected; the
-    neighbour looked for stands anywhere in the row, or is not there."""
+    scan for every group width (16 entries a lane), given and detected, by
+    scans (a workspace of 64 bytes) and by row tables (two int32 an entry
+    more, and nothing past them written); the neighbour looked for stands
+    anywhere in the row, or is not there.  With the tables' workspace sorted
+    rows and a malformed graph are taken too."""
     from mlx_cluster_amd import _lib
     lib = _lib.load()
     rng = np.random.default_rng(N)
@@ -763,15 +766,30 @@ def test_few_walks_kernel_on_unsorted_rows(N, L, rule, cuda):
     n_ref, e_ref, st, _ = oracle.node2vec_walk(rowptr, col, start, L, 0.5, 3.0, 5, rule=rule,
                                                rows_sorted=False, with_edges=True)
     assert st == 0
-    rp, cl, s = (torch.from_numpy(a.astype(np.int64)).to(cuda) for a in (rowptr, col, start))
-    for rows in (_lib.MLXC_ROWS_UNSORTED, _lib.MLXC_ROWS_DETECT):
-        n = torch.empty((N, L + 1), dtype=torch.int64, device=cuda)
-        e = torch.empty((N, L), dtype=torch.int64, device=cuda)
-        ws = torch.full((8,), 5, dtype=torch.int64, device=cuda)
-        rc = lib.mlxc_rejection_sampling(
-            rp.data_ptr(), V, cl.data_ptr(), cl.numel(), s.data_ptr(), N, L, 0.5, 3.0, 5, 0, rule,
-            rows, n.data_ptr(), e.data_ptr(), _lib.MLXC_OUT_INT64, ws.data_ptr(), 64,
-            torch.cuda.current_stream().cuda_stream)
-        assert rc == 0 and int(ws[0]) == 0
-        np.testing.assert_array_equal(n.cpu().numpy(), n_ref)
-        np.testing.assert_array_equal(e.cpu().numpy(), e_ref)
+    in_order = np.concatenate([np.sort(col[rowptr[v]:rowptr[v + 1]]) for v in range(V)])
+    n_ord, e_ord, st, _ = oracle.node2vec_walk(rowptr, in_order, start, L, 0.5, 3.0, 5, rule=rule,
+                                               rows_sorted=True, with_edges=True)
+    assert st == 0
+    broken = in_order.copy()
+    broken[-1] = V
+    E = col.size
+    rp, s, *cols = (torch.from_numpy(a.astype(np.int64)).to(cuda)
+                    for a in (rowptr, start, col, in_order, broken))
+    unsorted, detect = _lib.MLXC_ROWS_UNSORTED, _lib.MLXC_ROWS_DETECT
+    for ws_bytes in (64, 64 + (E + 1) // 2 * 16 + 8192):
+        for cl, rows, want in ((cols[0], unsorted, (n_ref, e_ref)), (cols[0], detect, (n_ref, e_ref)),
+                               (cols[1], detect, (n_ord, e_ord)), (cols[1], unsorted, (n_ord, e_ord)),
+                               (cols[1], _lib.MLXC_ROWS_SORTED, (n_ord, e_ord)),
+                               (cols[2], detect, None)):
+            n = torch.empty((N, L + 1), dtype=torch.int64, device=cuda)
+            e = torch.empty((N, L), dtype=torch.int64, device=cuda)
+            ws = torch.full((ws_bytes // 8 + 4,), 5, dtype=torch.int64, device=cuda)
+            rc = lib.mlxc_rejection_sampling(
+                rp.data_ptr(), V, cl.data_ptr(), E, s.data_ptr(), N, L, 0.5, 3.0, 5, 0, rule,
+                rows, n.data_ptr(), e.data_ptr(), _lib.MLXC_OUT_INT64, ws.data_ptr(), ws_bytes,
+                torch.cuda.current_stream().cuda_stream)
+            assert rc == 0 and (ws[ws_bytes // 8:] == 5).all()
+            assert int(ws[0]) == (0 if want else _lib.MLXC_STATUS_BAD_NODE)
+            if want:
+                np.testing.assert_array_equal(n.cpu().numpy(), want[0])
+                np.testing.assert_array_equal(e.cpu().numpy(), want[1])

@@ -10,7 +10,10 @@ for node2vec each MLXC_N2V_LAYOUT_* size the layout query gives, or the
 workspace query's.  node2vec cases also draw p and q, both acceptance rules,
 rows sorted, unsorted or detected, and the symmetric-graph hint on symmetric
 graphs.  Every case must equal the oracle bit for bit (nodes and edge ids)
-and leave no status bit; 2,000 cases per run, from fixed seeds.
+and leave no status bit; 2,000 cases per run, from fixed seeds.  600 more
+cases draw the workspaces that the Python layer asks for (the preferred
+queries), the node2vec few-walks kernel's with and without row tables among
+them, and the symmetric hint also for unsorted rows.
 
 Oracle: RandomWalk.cpp:41-60 and BiasedRandomWalk.cpp:20-28,52-100 as
 restated in oracle/walk_oracle.c.
@@ -32,6 +35,7 @@ L_N2V = [0, 1, 2, 3, 5, 8, 16, 17, 30, 33, 40]
 PQ = [(0.5, 2.0), (4.0, 0.25), (1.0, 3.0), (2.0, 0.5), (1.0, 1.0), (0.25, 4.0)]
 N2V_LAYOUTS = {"direct": 0, "lds": 1, "csr": 2, "records": 3, "records_hash": 4,
                "records_full": 5, "query": None}
+UNIFORM_MODES = ["query", "records", "csr", "lds", "minimum"]
 
 
 def _unsorted(rowptr, col, seed):
@@ -86,7 +90,7 @@ def _compare(name, ws, n_out, e_out, ref, ref_e, failures):
             failures.append(f"{name}: edge ids differ first at {at}: {got_e[at]} vs {ref_e[at]}")
 
 
-def _uniform_case(rng, graphs, device, lib, stream, failures):
+def _uniform_case(rng, graphs, device, lib, stream, failures, modes=UNIFORM_MODES):
     gname = str(rng.choice(["rmat7", "rmat12", "rmat16", "bahub", "rmat11s"]))
     rowptr, col, rp, cl = graphs[gname]
     V, E = rp.size - 1, cl.size
@@ -96,7 +100,7 @@ def _uniform_case(rng, graphs, device, lib, stream, failures):
     first = int(rng.choice([0, 0, 5, 1 << 33])) if seeded else 0
     seed = int(rng.integers(1 << 62))
     int32, edges = bool(rng.integers(2)), bool(rng.integers(2))
-    mode = str(rng.choice(["query", "records", "csr", "lds", "minimum"]))
+    mode = str(rng.choice(modes))
     start_h = rng.integers(0, V, N).astype(np.int64)
     rand_h = (oracle.philox_uniform(N * L, seed, first * L) if seeded
               else rng.random(N * L, dtype=np.float32))
@@ -104,6 +108,7 @@ def _uniform_case(rng, graphs, device, lib, stream, failures):
     assert st == 0
     ws_bytes = {"query": lib.mlxc_random_walk_workspace_bytes(V, E, N, L),
                 "records": 256 + 16 * (E + N), "csr": 256 + 16 * N, "lds": 256,
+                "preferred": lib.mlxc_random_walk_preferred_bytes(V, E, N, L),
                 "minimum": 32}[mode]
     ws = torch.empty((max(ws_bytes, 32) + 7) // 8, dtype=torch.int64, device=device)
     n_out, e_out, n_p, e_p, ot = _outputs(N, L, int32, edges, device)
@@ -125,7 +130,7 @@ def _uniform_case(rng, graphs, device, lib, stream, failures):
     _compare(name, ws, n_out, e_out, ref, ref_e, failures)
 
 
-def _n2v_case(rng, graphs, device, lib, stream, failures):
+def _n2v_case(rng, graphs, device, lib, stream, failures, layouts=tuple(N2V_LAYOUTS)):
     gname = str(rng.choice(["rmat7", "rmat12", "rmat11s", "bahub", "rmat11s_unsorted",
                             "rmat12_unsorted", "rmat16"]))
     rowptr, col, rp, cl = graphs[gname]
@@ -140,16 +145,22 @@ def _n2v_case(rng, graphs, device, lib, stream, failures):
     symmetric_graph = gname in ("rmat11s", "bahub")
     if symmetric_graph and rows != _lib.MLXC_ROWS_UNSORTED and rng.integers(2):
         rows |= _lib.MLXC_ROWS_SYMMETRIC
+    if "few" in layouts and gname == "rmat11s_unsorted" and rng.integers(2):
+        rows |= _lib.MLXC_ROWS_SYMMETRIC
     first = int(rng.choice([0, 0, 7, 1 << 35]))
     seed = int(rng.integers(1 << 62))
     int32, edges = bool(rng.integers(2)), bool(rng.integers(2))
-    layout = str(rng.choice(list(N2V_LAYOUTS)))
+    layout = str(rng.choice(layouts))
     start_h = rng.integers(0, V, N).astype(np.int64)
     ref, ref_e, st, _ = oracle.node2vec_walk(rp, cl, start_h, L, p, q, seed, rule=rule,
                                              rows_sorted=not unsorted, with_edges=True,
                                              first_walk=first)
     assert st == 0
-    if N2V_LAYOUTS[layout] is None:
+    if layout == "preferred":
+        ws_bytes = lib.mlxc_rejection_sampling_preferred_bytes(V, E, N, L, p, q, rule)
+    elif layout in ("few", "few_tables"):
+        ws_bytes = 64 if layout == "few" else 64 + (E + 1) // 2 * 16 + 8192
+    elif N2V_LAYOUTS[layout] is None:
         ws_bytes = lib.mlxc_rejection_sampling_workspace_bytes(V, E, N, L, p, q, rule)
     else:
         ws_bytes = lib.mlxc_rejection_sampling_layout_bytes(V, E, N, L, N2V_LAYOUTS[layout])
@@ -179,3 +190,18 @@ def test_random_cases_match_the_oracle(seed, graphs, cuda):
         case = _uniform_case if i % 2 == 0 else _n2v_case
         case(rng, graphs, cuda, lib, stream, failures)
     assert not failures, f"{len(failures)} of 500 cases differ:\n" + "\n".join(failures[:10])
+
+
+@pytest.mark.parametrize("seed", [21, 22])
+def test_random_cases_with_the_preferred_workspaces(seed, graphs, cuda):
+    rng = np.random.default_rng(seed)
+    lib = _lib.load()
+    stream = torch.cuda.current_stream(cuda).cuda_stream
+    failures = []
+    for i in range(300):
+        if i % 3 == 0:
+            _uniform_case(rng, graphs, cuda, lib, stream, failures, modes=["preferred"])
+        else:
+            _n2v_case(rng, graphs, cuda, lib, stream, failures,
+                      layouts=["preferred", "few", "few_tables"])
+    assert not failures, f"{len(failures)} of 300 cases differ:\n" + "\n".join(failures[:10])
