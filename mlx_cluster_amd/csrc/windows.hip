@@ -20,6 +20,7 @@ namespace {
 
 constexpr int kWinTile = 64;  // walks per block (at most)
 constexpr int kMaxContext = 32;
+constexpr int kWinSlots = (kWinTile * kMaxContext + kBlock - 1) / kBlock;
 constexpr int kLineBytes = 128;
 constexpr size_t kTileLds = 64 * 1024;  // LDS bytes for the walk rows of a tile
 
@@ -63,6 +64,22 @@ __device__ __forceinline__ void emit_windows(const T* rw, int64_t tile, int64_t 
     constexpr int kLine = kLineBytes / sizeof(T);
     const int entries = static_cast<int>(tile) * ctx;  // one window of every walk in the tile
     const int windows = walk_nodes - ctx + 1;
+    if (!kHalo) {
+        // this thread's entries of a window position: places in the rows
+        int32_t src[kWinSlots];
+#pragma unroll
+        for (int i = 0; i < kWinSlots; ++i) {
+            const int e = threadIdx.x + i * kBlock;
+            src[i] = e < entries ? (e / ctx) * walk_nodes + e % ctx : -1;
+        }
+        for (int j = 0; j < windows; ++j) {
+            T* const o = out + (static_cast<int64_t>(j) * num_walks + n0) * ctx;
+#pragma unroll
+            for (int i = 0; i < kWinSlots; ++i)
+                if (src[i] >= 0) put(o + threadIdx.x + i * kBlock, rw[src[i] + j]);
+        }
+        return;
+    }
     const bool first = n0 == 0, last = n0 + tile == num_walks;
     // entries of a position from the tile on, as far as the rows reach
     const int64_t left = num_walks - n0;
@@ -75,12 +92,10 @@ __device__ __forceinline__ void emit_windows(const T* rw, int64_t tile, int64_t 
     for (int j = 0; j < windows; ++j) {
         T* const o = out + (static_cast<int64_t>(j) * num_walks + n0) * ctx;
         int lo = 0, hi = entries;
-        if (kHalo) {
-            const int at = static_cast<int>((reinterpret_cast<uintptr_t>(o) / sizeof(T)) % kLine);
-            if (!first) lo = (kLine - at) % kLine;
-            if (!last) hi += (kLine - (at + entries) % kLine) % kLine;
-            if (hi > rest) hi = rest;  // the position ends there
-        }
+        const int at = static_cast<int>((reinterpret_cast<uintptr_t>(o) / sizeof(T)) % kLine);
+        if (!first) lo = (kLine - at) % kLine;
+        if (!last) hi += (kLine - (at + entries) % kLine) % kLine;
+        if (hi > rest) hi = rest;  // the position ends there
         for (int e = lo + static_cast<int>(threadIdx.x); e < hi; e += kBlock) {
             const int w = static_cast<int>((static_cast<uint32_t>(e) * inv) >> 16);
             put(o + e, rw[w * walk_nodes + (e - w * ctx) + j]);
@@ -152,22 +167,51 @@ int tile_walks(int32_t walk_nodes, size_t esz) {
 
 namespace {
 
-// Grid and LDS of a window launch.  The halo's rows join the tile's where
-// both fit kTileLds (int64, ctx 10: walks of up to 124 nodes); longer walks
-// write their lines where the tiles happen to cut them.
+// Grid and LDS of a window launch.  The halo's rows join the tile's where it
+// pays (lines_pay) and both fit kTileLds (int64, ctx 10: walks of up to 124
+// nodes); other calls write their lines where the tiles happen to cut them.
 struct WinLaunch {
     int per_block, halo;
     int64_t grid;
     size_t lds;
 };
 
-WinLaunch win_launch(int64_t num_walks, int32_t walk_nodes, int32_t ctx, size_t esz) {
+// Whether moving the tiles' ends to line boundaries is worth its halo and the
+// walk that each entry of it has to find.  Not where every run fills whole
+// lines as it is; not below two blocks or so a compute unit, where a block's
+// own time counts; not where the caches put the partial lines together; and
+// not for pairs, whose runs are short and whose halo is long.  Kernel us,
+// tiles as they are / moved, int64 but where noted:
+//   21 nodes, ctx 10:  30,011 walks (29 MB) 8.9 / 7.1, 60,013 (58 MB) 17.9 / 12.8,
+//                      1,000,003 (960 MB) 294 / 181;  10,007 (10 MB) 6.5 / 6.4
+//   81 nodes, ctx 10:  10,007 (58 MB, 157 blocks) 19.1 / 22.6, 30,011 int32 (86 MB) 33.8 / 24.5
+//   31 nodes, ctx 16:  30,011 int32 (31 MB) 7.9 / 8.9, 60,013 int32 (61 MB) 14.9 / 13.6,
+//                      10,007 (20 MB, whole lines) 7.8 / 8.9
+//   30 nodes, ctx 3:   60,013 int32 (20 MB) 9.7 / 11.5, 100,003 int32 (34 MB) 14.9 / 15.4,
+//                      200,003 int32 (67 MB) 32.0 / 25.9, 60,013 (40 MB) 13.2 / 11.3
+//   11 nodes, ctx 2:   1,000,003 (160 MB) 44.8 / 47.4, int32 (80 MB) 33.8 / 43.8
+bool lines_pay(const WinLaunch& w, int64_t num_walks, int32_t walk_nodes, int32_t ctx, size_t esz,
+               const void* out) {
+    const size_t run = static_cast<size_t>(ctx) * esz;  // bytes a walk and a window position
+    if (static_cast<size_t>(num_walks) * run % kLineBytes == 0 &&
+        static_cast<size_t>(w.per_block) * run % kLineBytes == 0 &&
+        reinterpret_cast<uintptr_t>(out) % kLineBytes == 0)
+        return false;
+    if (ctx <= 2 || w.grid < 400) return false;
+    const size_t bytes = static_cast<size_t>(walk_nodes - ctx + 1) * num_walks * run;
+    return bytes >= (w.halo <= 7 && w.grid >= 768 ? size_t{24} << 20 : size_t{64} << 20);
+}
+
+WinLaunch win_launch(int64_t num_walks, int32_t walk_nodes, int32_t ctx, size_t esz,
+                     const void* out) {
     WinLaunch w;
     w.per_block = tile_walks(walk_nodes, esz);
     w.halo = halo_walks(ctx, esz);
     const size_t row = static_cast<size_t>(walk_nodes) * esz;
-    if ((w.per_block + w.halo) * row > kTileLds) w.halo = 0;
     w.grid = w.per_block < 1 ? 0 : (num_walks + w.per_block - 1) / w.per_block;
+    if ((w.per_block + w.halo) * row > kTileLds ||
+        !lines_pay(w, num_walks, walk_nodes, ctx, esz, out))
+        w.halo = 0;
     w.lds = (w.per_block + w.halo) * row;
     return w;
 }
@@ -197,7 +241,7 @@ void negative_windows_typed(const WinLaunch& w, const int64_t* start, int64_t nu
 int launch_context_windows(const void* walks, int64_t num_walks, int32_t walk_nodes, int32_t ctx,
                            int32_t elem_type, void* out, hipStream_t stream) {
     const bool narrow = elem_type == MLXC_OUT_INT32;
-    const WinLaunch w = win_launch(num_walks, walk_nodes, ctx, narrow ? 4 : 8);
+    const WinLaunch w = win_launch(num_walks, walk_nodes, ctx, narrow ? 4 : 8, out);
     if (w.per_block < 1) return fail(MLXC_ERR_INVALID_ARGUMENT, "walks too long for windows");
     if (narrow) context_windows_typed<int32_t>(w, walks, num_walks, walk_nodes, ctx, out, stream);
     else context_windows_typed<int64_t>(w, walks, num_walks, walk_nodes, ctx, out, stream);
@@ -213,7 +257,7 @@ int launch_negative_windows(const int64_t* start, int64_t num_walks, int32_t wal
                             int32_t ctx, int64_t num_nodes, uint64_t seed, int32_t out_type,
                             void* out, hipStream_t stream) {
     const bool narrow = out_type == MLXC_OUT_INT32;
-    const WinLaunch w = win_launch(num_walks, walk_length + 1, ctx, narrow ? 4 : 8);
+    const WinLaunch w = win_launch(num_walks, walk_length + 1, ctx, narrow ? 4 : 8, out);
     if (w.per_block < 1) return fail(MLXC_ERR_INVALID_ARGUMENT, "walk_length too large");
     if (narrow)
         negative_windows_typed<int32_t>(w, start, num_walks, walk_length, ctx, num_nodes, seed,

@@ -108,3 +108,39 @@ def test_windows_line_edges(N, nodes, C, dtype, shift, cuda):
         got = buf.cpu().numpy()
         np.testing.assert_array_equal(got[shift:shift + total], ref.reshape(-1).astype(got.dtype))
         assert (got[:shift] == -7).all() and (got[shift + total:] == -7).all()
+
+
+@pytest.mark.parametrize("N,nodes,C,dtype,shift", [
+    (49_153, 40, 32, torch.int64, 0), (49_153, 40, 32, torch.int32, 5), (60_013, 21, 10, torch.int64, 1),
+    (60_079, 21, 10, torch.int32, 0), (60_013, 30, 3, torch.int64, 3), (200_065, 30, 3, torch.int32, 1),
+    (25_601, 81, 10, torch.int64, 0), (60_032, 21, 10, torch.int64, 1), (150_017, 12, 7, torch.int32, 31),
+    (70_001, 124, 10, torch.int64, 0)])
+def test_windows_line_edges_of_large_outputs(N, nodes, C, dtype, shift, cuda):
+    """The same for outputs past the sizes from which the tiles' ends are moved
+    (24 and 64 MB), against torch's unfold of the walks; (60_032 walks fill
+    whole lines, from a buffer that starts inside one)."""
+    from mlx_cluster_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device=cuda).manual_seed(N)
+    walks = torch.randint(0, 2**31 - 1, (N, nodes), generator=g, device=cuda).to(dtype)
+    out_type = _lib.MLXC_OUT_INT32 if dtype == torch.int32 else _lib.MLXC_OUT_INT64
+    total = (nodes - C + 1) * N * C
+    assert total * walks.element_size() >= 24 << 20
+    stream = torch.cuda.current_stream().cuda_stream
+    for negative in (False, True):
+        buf = torch.full((total + 64,), -7, dtype=dtype, device=cuda)
+        out = buf[shift:]
+        if negative:
+            start = walks[:, 0].long().contiguous()
+            rc = lib.mlxc_negative_windows(start.data_ptr(), N, nodes - 1, C, 1 << 20, 9, out_type,
+                                           out.data_ptr(), stream)
+            rows = torch.from_numpy(oracle.negative_walks(start.cpu().numpy(), nodes - 1, 1 << 20,
+                                                          9)).to(cuda, dtype)
+        else:
+            rc = lib.mlxc_context_windows(walks.data_ptr(), N, nodes, C, out_type, out.data_ptr(),
+                                          stream)
+            rows = walks
+        assert rc == 0
+        assert torch.equal(buf[shift:shift + total].view(nodes - C + 1, N, C),
+                           rows.unfold(1, C, 1).transpose(0, 1))
+        assert (buf[:shift] == -7).all() and (buf[shift + total:] == -7).all()
