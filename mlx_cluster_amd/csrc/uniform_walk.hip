@@ -660,18 +660,27 @@ size_t init_bytes(int64_t num_walks) {
 }
 
 // Whether the flat walk beats the persistent walk the call would otherwise
-// run.  Its lanes idle once their walks are absorbed, and its walks longer
-// than a stretch store their rows in pieces, so it loses to the record walk
-// (one read a step, N * L >= 4 E) past about N * L^2 = 2^31 and to the CSR
-// walk past 2^32.  Measured, us a call, rand given, int64 (flat / persistent):
+// run.  Few walks always: spread thin, in stretches of up to 1,024 positions,
+// they wait for their chains, and the flat walk has nothing else in them.  In
+// larger calls its lanes idle once their walks are absorbed and wavefronts of
+// 64 walks store rows longer than a stretch in pieces, so it loses to the
+// record walk (one read a step, N * L >= 4 E) past about N * L^2 = 2^31 and to
+// the CSR walk past 2^32.  Measured, us a call, rand given, int64 (flat /
+// persistent; up to 65,536 walks the call alone):
+//   E 54 K:   16 x 16,000  6,138 / 13,266,  1,300 x 1,300  559 / 1,329,
+//             8,192 x 16,000  8,676 / 14,442,  65,536 x 500  495 / 580,  x 1,300  1,416 / 1,485
 //   E 0.5 M:  2^18 x 80  192 / 278,  2^20 x 80   690 / 671,  2^24 x 20  3,064 / 3,444
-//   E 16 M:   2^18 x 80  298 / 396,  2^20 x 80 1,009 / 999,  2^22 x 20  1,172 / 1,259,
+//   E 16 M:   16 x 16,000  310 / 677,  1,300 x 1,300  361 / 775,  8,192 x 16,000  1,070 / 1,236,
+//             65,536 x 1,300  1,256 / 1,260,
+//             2^18 x 80  298 / 396,  2^20 x 80 1,009 / 999,  2^22 x 20  1,172 / 1,259,
 //             2^24 x 20  4,740 / 4,232
 //   E 263 M:  2^20 x 80  1,272 / 1,364,  2^22 x 20  1,437 / 1,668,
 //             2^22 x 80  5,171 / 4,496,  2^24 x 20  5,837 / 5,778
 bool flat_walk_pays(int64_t num_walks, int32_t walk_length, bool records) {
+    if (num_walks <= 8192) return true;
     const double l = walk_length > 0 ? walk_length : 1;
-    return static_cast<double>(num_walks) * l * l <= (records ? 0x1p31 : 0x1p32);
+    return static_cast<double>(num_walks) * l * l <=
+           (num_walks <= 65536 ? 0x1p36 : records ? 0x1p31 : 0x1p32);
 }
 
 // A workspace that holds the start records selects the persistent walks, one

@@ -302,3 +302,17 @@ def test_preferred_bytes_of_few_walks(V, E, N, L, p, q, rule, few):
         assert got == 64 + (E + 1) // 2 * 16 + 8192  # the row tables, for unsorted rows
     else:
         assert got == 64
+
+
+@pytest.mark.parametrize("E,N,L,flat", [
+    (53_531, 1_300, 1_300, True), (53_531, 8_192, 100_000, True), (53_531, 8_193, 2_800, True),
+    (53_531, 8_193, 3_000, False), (1 << 24, 65_536, 1_024, True), (1 << 24, 65_536, 1_025, False),
+    (1 << 24, 65_537, 181, True), (1 << 24, 65_537, 257, False), (1 << 28, 1 << 20, 64, True),
+    (1 << 28, 1 << 20, 65, False), (1 << 19, 1 << 20, 45, True), (1 << 19, 1 << 20, 46, False)])
+def test_preferred_bytes_of_the_flat_walk(E, N, L, flat):
+    """Uniform calls of few walks take the flat walk however long they are, larger
+    ones up to a product of walks and squared steps."""
+    lib = _lib.load()
+    got = lib.mlxc_random_walk_preferred_bytes(1 << 12, E, N, L)
+    assert got == (32 + 4 * min(N, 2048) if flat else
+                   lib.mlxc_random_walk_workspace_bytes(1 << 12, E, N, L))

@@ -697,3 +697,26 @@ def test_one_bad_start_is_found_in_any_block(N, cuda):
         start[at] = 2
         with pytest.raises(ValueError, match="outside"):
             mc.random_walk(rowptr, col, start, rand, 2)
+
+
+@pytest.mark.parametrize("N,L", [(1, 1022), (2, 1023), (300, 1024), (300, 1025), (2049, 1100),
+                                 (8192, 600)])
+@pytest.mark.parametrize("seeded", [False, True])
+def test_flat_walk_of_long_walks(N, L, seeded, cuda):
+    """Few long walks through the Python layer take the flat walk, in stretches
+    of up to 1,024 positions; nodes and edge ids are the oracle's."""
+    from mlx_cluster_amd import _lib
+    rowptr, col = synth.rmat_csr(12, 60_000, seed=L, device=cuda, symmetrize=True)
+    V = rowptr.numel() - 1
+    assert _lib.load().mlxc_random_walk_preferred_bytes(V, col.numel(), N, L) == \
+        32 + 4 * min(N, 2048)
+    start = (torch.arange(N, device=cuda) * 11) % V
+    rand = mc.philox_uniform((N, L), 9, device=cuda)
+    n, e = mc.random_walk(rowptr, col, start, None if seeded else rand, L,
+                          seed=9 if seeded else None, return_edges=True)
+    n_ref, e_ref, st, _ = oracle.uniform_walk(rowptr.cpu().numpy(), col.cpu().numpy(),
+                                              start.cpu().numpy(), rand.cpu().numpy(), L,
+                                              with_edges=True)
+    assert st == 0
+    np.testing.assert_array_equal(n.cpu().numpy(), n_ref)
+    np.testing.assert_array_equal(e.cpu().numpy(), e_ref)
