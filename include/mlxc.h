@@ -457,6 +457,10 @@ int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream
  */
 int mlxc_set_status_target(int64_t* h_status);
 
+/* The calling thread's status target (NULL: none), for code that sets one of
+ * its own around a call and puts the thread's back.  No reference counterpart. */
+int64_t* mlxc_status_target(void);
+
 /*
  * Measurement hook: times the walk kernel alone, without the preparation
  * launches before it (a call's last launch is its walk kernel).  After

@@ -104,6 +104,7 @@ SIGNATURES = {
     ),
     "mlxc_set_walk_events": (ctypes.c_int, [_ptr, _ptr]),
     "mlxc_set_status_target": (ctypes.c_int, [_ptr]),
+    "mlxc_status_target": (_ptr, []),
     "mlxc_publish_status": (ctypes.c_int, [_ptr, _ptr, _ptr]),
     "mlxc_gather_probe": (
         ctypes.c_int, [_ptr, _i64, _i32, _i32, _i32, _i32, _i64, _u64, _ptr, _ptr, _ptr],

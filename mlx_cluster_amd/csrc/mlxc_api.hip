@@ -21,7 +21,7 @@ thread_local std::string g_last_error;
 }
 
 thread_local hipEvent_t g_walk_events[2] = {nullptr, nullptr};
-thread_local StatusTarget g_status_target = {nullptr, false};
+thread_local StatusTarget g_status_target = {nullptr, nullptr, false};
 
 int fail(int code, const std::string& msg) {
     g_last_error = msg;
@@ -318,7 +318,7 @@ int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream
 }
 
 int mlxc_set_status_target(int64_t* h_status) {
-    g_status_target = {nullptr, false};
+    g_status_target = {nullptr, nullptr, false};
     if (!h_status) return MLXC_OK;
     if (reinterpret_cast<uintptr_t>(h_status) % 8 != 0)
         return fail(MLXC_ERR_INVALID_ARGUMENT, "h_status must be 8-byte aligned host memory");
@@ -326,8 +326,11 @@ int mlxc_set_status_target(int64_t* h_status) {
     if (!g_status_target.words)
         return fail(MLXC_ERR_INVALID_ARGUMENT,
                     "h_status is not host memory the device can write (hipHostMalloc)");
+    g_status_target.host = h_status;
     return MLXC_OK;
 }
+
+int64_t* mlxc_status_target(void) { return g_status_target.host; }
 
 int mlxc_set_walk_events(void* start_event, void* stop_event) {
     if ((start_event == nullptr) != (stop_event == nullptr))

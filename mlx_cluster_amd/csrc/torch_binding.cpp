@@ -55,19 +55,23 @@ int64_t* status_words() {
 }
 
 // For a validated call: makes the library publish the call's status word into
-// the calling thread's host words (mlxc_set_status_target).
+// the calling thread's host words (mlxc_set_status_target), and puts the
+// target that the thread had before back afterwards.
 class StatusTarget {
 public:
-    explicit StatusTarget(bool check) {
+    explicit StatusTarget(bool check) : before(mlxc_status_target()) {
         int64_t* h = check ? status_words() : nullptr;
         if (!h) return;
         __atomic_store_n(&h[0], int64_t{0}, __ATOMIC_RELAXED);
         if (mlxc_set_status_target(h) == MLXC_OK) words = h;
     }
     ~StatusTarget() {
-        if (words) mlxc_set_status_target(nullptr);
+        if (words || before) mlxc_set_status_target(before);
     }
     int64_t* words = nullptr;
+
+private:
+    int64_t* const before;
 };
 
 // The status word of the call just enqueued on `stream`.  Its last launch

@@ -36,9 +36,11 @@ inline int record_walk_event(int which, hipStream_t stream) {
 
 // Where the calling thread's walk calls publish their status word, and its CSR
 // builds theirs and their entry count (device address of the caller's host
-// words; null: nowhere), and whether the call in progress already has.
+// words, which are at `host`; null: nowhere), and whether the call in progress
+// already has.
 struct StatusTarget {
     int64_t* words;
+    int64_t* host;
     bool done;
 };
 extern thread_local StatusTarget g_status_target;

@@ -123,6 +123,14 @@ def test_other_entry_points_reject_bad_arguments():
         == _lib.MLXC_ERR_INVALID_ARGUMENT
 
 
+def test_status_target_checks_its_pointer():
+    lib = _lib.load()
+    assert lib.mlxc_status_target() is None
+    assert lib.mlxc_set_status_target(ctypes.c_void_p(0x1004)) == _lib.MLXC_ERR_INVALID_ARGUMENT
+    assert lib.mlxc_status_target() is None
+    assert lib.mlxc_set_status_target(None) == _lib.MLXC_OK
+
+
 def test_publish_status_checks_its_pointers():
     lib = _lib.load()
     assert lib.mlxc_publish_status(None, FAKE, None) == _lib.MLXC_ERR_INVALID_ARGUMENT

@@ -14,7 +14,7 @@ import pytest
 import torch
 
 import mlx_cluster_amd as mc
-from mlx_cluster_amd import _lib
+from mlx_cluster_amd import _lib, synth
 from tests import status_cases as sc
 
 pytestmark = pytest.mark.gpu
@@ -148,3 +148,110 @@ def test_published_status_is_the_workspace_word(case, cuda):
             mc.random_walk(r, c, s, None, L, seed=5)
     else:
         mc.random_walk(r, c, s, None, L, seed=5)
+
+
+@pytest.fixture
+def status_words():
+    """Three host words the device can write, with mlxc_set_status_target
+    undone afterwards."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    words = ctypes.c_void_p()
+    flags = 0x40000000 | 0x2 | 0x1  # hipHostMallocCoherent | Mapped | Portable
+    assert hip.hipHostMalloc(ctypes.byref(words), ctypes.c_size_t(24), ctypes.c_uint(flags)) == 0
+    yield words.value, (ctypes.c_int64 * 3).from_address(words.value)
+    _lib.load().mlxc_set_status_target(None)
+    torch.cuda.synchronize()
+    hip.hipHostFree(words)
+
+
+def test_status_target_of_every_kind_of_call(status_words, cuda):
+    """With a thread's status target set, every walk call and CSR build on the
+    thread leaves its status bits in word 1 (a build its entry count in word
+    2) and 1 in word 0, whichever of its launches publishes them: flat,
+    record, LDS and few-walks walks (with and without row tables), calls
+    without walks, noalloc, small, large and empty builds.  Validated calls of
+    the Python layer keep the target; after NULL nothing is written."""
+    lib = _lib.load()
+    address, h = status_words
+    stream = torch.cuda.current_stream().cuda_stream
+    rowptr, col = (t.to(cuda) for t in synth.rmat_csr(12, 40_000, seed=5, symmetrize=True))
+    V, E = rowptr.numel() - 1, col.numel()
+    N, L = 300, 9
+    out = torch.empty((N, L + 1), dtype=torch.int64, device=cuda)
+    ws = torch.zeros(1 << 20, dtype=torch.int64, device=cuda)
+    good = torch.arange(N, device=cuda) % V
+    bad = good.clone()
+    bad[7] = V
+
+    def uniform(start, nbytes, n=N):
+        return lib.mlxc_random_walk_seeded(rowptr.data_ptr(), V, col.data_ptr(), E,
+                                           start.data_ptr(), n, L, 3, 0, out.data_ptr(), None, 0,
+                                           ws.data_ptr(), nbytes, stream)
+
+    def n2v(start, nbytes, n=N):
+        return lib.mlxc_rejection_sampling(rowptr.data_ptr(), V, col.data_ptr(), E,
+                                           start.data_ptr(), n, L, 0.5, 2.0, 3, 0, 0,
+                                           _lib.MLXC_ROWS_DETECT, out.data_ptr(), None, 0,
+                                           ws.data_ptr(), nbytes, stream)
+
+    rand = torch.zeros(N * L, device=cuda)
+    noalloc = lambda start: lib.mlxc_random_walk_noalloc(
+        rowptr.data_ptr(), V, col.data_ptr(), E, start.data_ptr(), N, rand.data_ptr(), L,
+        out.data_ptr(), None, 0, None, stream)
+    tables = 64 + (E + 1) // 2 * 16 + 8192
+    walks = {"flat, zeroed word": lambda s: uniform(s, 32), "flat": lambda s: uniform(s, 32 + 4 * N),
+             "csr": lambda s: uniform(s, 256 + 16 * N),
+             "records": lambda s: uniform(s, 256 + 16 * (E + N)), "few": lambda s: n2v(s, 64),
+             "few, tables": lambda s: n2v(s, tables), "direct": lambda s: n2v(s, 32),
+             "n2v records": lambda s: n2v(s, lib.mlxc_rejection_sampling_layout_bytes(
+                 V, E, N, L, _lib.MLXC_N2V_LAYOUT_RECORDS_FULL)), "noalloc": noalloc}
+    small_rp, small_cl = (t.to(cuda) for t in synth.rmat_csr(8, 1000, seed=5))
+
+    def lds(start, nbytes):
+        return lib.mlxc_rejection_sampling(small_rp.data_ptr(), 256, small_cl.data_ptr(),
+                                           small_cl.numel(), start.data_ptr(), N, L, 0.5, 2.0, 3, 0,
+                                           0, _lib.MLXC_ROWS_DETECT, out.data_ptr(), None, 0,
+                                           ws.data_ptr(), nbytes, stream)
+
+    walks["lds, words of its blocks"] = lambda s: lds(s.clamp(max=255) + (s == V), 1280)
+    walks["lds"] = lambda s: lds(s.clamp(max=255) + (s == V), 256)
+
+    def run(call, *args):
+        h[0], h[1], h[2] = 0, -1, -1
+        assert call(*args) == 0, _lib.last_error()
+        torch.cuda.synchronize()
+        return list(h)
+
+    assert lib.mlxc_set_status_target(address) == 0, _lib.last_error()
+    assert lib.mlxc_status_target() == address
+    for name, call in walks.items():
+        assert run(call, good) == [1, 0, -1], name
+        assert run(call, bad) == [1, _lib.MLXC_STATUS_BAD_NODE, -1], name
+    assert run(uniform, good, 32, 0) == [1, 0, -1]
+    assert run(n2v, good, 64, 0) == [1, 0, -1]
+    ids = torch.randint(0, 4096, (2, 300_000), device=cuda)
+    rp2, cl2 = torch.empty(4097, dtype=torch.int64, device=cuda), torch.empty_like(ids[0])
+
+    def build(n, nodes=4096):
+        nbytes = lib.mlxc_csr_build_workspace_bytes(nodes, n, 0)
+        assert nbytes <= ws.numel() * 8
+        return lib.mlxc_csr_build(ids[0].data_ptr(), ids[1].data_ptr(), n, nodes, 0,
+                                  rp2.data_ptr(), cl2.data_ptr(), ws.data_ptr(), nbytes, stream)
+
+    for n in (0, 5_000, 300_000):
+        assert run(build, n) == [1, 0, n]
+    assert run(build, 5_000, 100)[:2] == [1, _lib.MLXC_STATUS_BAD_NODE]
+    assert run(build, 300_000, 100)[:2] == [1, _lib.MLXC_STATUS_BAD_NODE]
+    # validated calls of the Python layer wait on words of their own
+    mc.random_walk(rowptr, col, good, None, L, seed=3)
+    mc.rejection_sampling(rowptr, col, good, L, 0.5, 2.0, seed=3)
+    mc.to_csr(ids, 4096)
+    with pytest.raises(ValueError):
+        mc.random_walk(rowptr, col, bad, None, L, seed=3)
+    assert lib.mlxc_status_target() == address
+    assert run(walks["flat"], good) == [1, 0, -1]
+    assert lib.mlxc_set_status_target(None) == 0 and lib.mlxc_status_target() is None
+    assert run(walks["flat"], good) == [0, -1, -1]
+    assert run(build, 5_000) == [0, -1, -1]
+    mc.random_walk(rowptr, col, good, None, L, seed=3)
+    assert lib.mlxc_status_target() is None
