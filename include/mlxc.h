@@ -31,15 +31,16 @@ extern "C" {
 
 /* Device workspace.  Every walk entry point takes `d_workspace` (16-byte
  * aligned, at least MLXC_WORK_WORDS int64 words) and its size in bytes.  The
- * call zeroes the first MLXC_WORK_WORDS words on `stream` before its kernels
- * run; after the call has completed, word 0 holds the MLXC_STATUS_* bits of
- * that call (the other words are internal: the walk-queue counter).  A
+ * call writes the first MLXC_WORK_WORDS words on `stream`, whatever they held;
+ * once it has completed, word 0 holds the MLXC_STATUS_* bits of that call
+ * (until then, and in the other words, what its kernels count with).  A
  * workspace of the size the *_workspace_bytes queries return also holds
  * per-call layouts of the graph and the starts (8- or 16-byte records: node,
  * row begin, row degree) that cut the dependent reads per step; with a smaller
- * workspace the kernels read the CSR arrays directly.  For graphs small
- * enough (see the queries), a workspace of exactly the 256-byte header runs
- * the walk with the whole CSR in on-chip memory.  Same results every way. */
+ * workspace the kernels read the CSR arrays directly, which is faster in calls
+ * up to a size (the *_preferred_bytes queries).  For graphs small enough (see
+ * the queries), a workspace of the 256-byte header runs the node2vec walk with
+ * the whole CSR in on-chip memory.  Same results every way. */
 #define MLXC_WORK_WORDS 4
 
 /* Bits a walk kernel ORs into workspace word 0 when the graph or the starts
@@ -63,14 +64,15 @@ extern "C" {
 #define MLXC_RULE_NODE2VEC_EXACT 1 /* analytic node2vec: accept iff r < prob_d(t, x)      */
 
 /* Row order of the graph passed to mlxc_rejection_sampling. */
-#define MLXC_ROWS_UNSORTED 0  /* scan rows linearly, as the reference's is_neighbor does */
+#define MLXC_ROWS_UNSORTED 0  /* rows in any order (the reference's is_neighbor scans them) */
 #define MLXC_ROWS_SORTED 1    /* the caller promises every row is sorted ascending */
 #define MLXC_ROWS_DETECT 2    /* the call checks the rows on the device (and validates the CSR) */
 /* OR-ed into one of the three above: the caller promises the graph is
  * symmetric (every (u, v) entry has a (v, u) entry), so that "t in row(x)"
  * equals "x in row(t)" and the neighbour test may search the shorter row.
  * Results are those of the reference when the promise holds, unspecified
- * otherwise.  Record kernels only; the other paths ignore it. */
+ * otherwise.  The record, CSR-mode and few-walks kernels; the other paths
+ * ignore it. */
 #define MLXC_ROWS_SYMMETRIC 4
 
 /* Bits written by mlxc_csr_check. */
@@ -106,7 +108,7 @@ const char* mlxc_last_error(void);
 /* Workspace bytes that let mlxc_random_walk use its fastest layout for this
  * call:
  *   256 when num_nodes + 1 + num_edges <= 14336 and the call takes 1 to 2^20
- *     steps (num_walks <= 2^20): the walk runs with rowptr and col in LDS;
+ *     steps (num_walks <= 2^20): the flat walk (below);
  *   256 + R * (num_edges + num_walks) when the call takes at least
  *     4 * num_edges steps, or num_edges <= 32768 * walk_length (per-call edge
  *     records): R = 8 when the bits of num_nodes - 1 and of num_edges add up
@@ -120,10 +122,13 @@ const char* mlxc_last_error(void);
 size_t mlxc_random_walk_workspace_bytes(int64_t num_nodes, int64_t num_edges,
                                         int64_t num_walks, int32_t walk_length);
 
-/* Workspace bytes with which mlxc_random_walk is fastest for these arguments:
- * MLXC_WORK_WORDS * 8, which selects the flat walk (no queue and no per-call
- * layout: it reads the CSR arrays as they are), in calls up to a size, else
- * what mlxc_random_walk_workspace_bytes returns.  A workspace of that size or
+/* Workspace bytes with which mlxc_random_walk is fastest for these arguments.
+ * In calls up to a size MLXC_WORK_WORDS * 8 + 4 * min(num_walks, 2048): too
+ * little for the layouts above, which selects the flat walk (no queue and no
+ * per-call layout: it reads the CSR arrays as they are), with a status word for
+ * each of its blocks; MLXC_WORK_WORDS * 8 alone selects it too, at the price
+ * of one more launch in small calls.  Else what
+ * mlxc_random_walk_workspace_bytes returns.  A workspace of that size or
  * larger runs the record and CSR walks whatever the call's size.  No
  * reference counterpart. */
 size_t mlxc_random_walk_preferred_bytes(int64_t num_nodes, int64_t num_edges,
@@ -140,7 +145,7 @@ size_t mlxc_random_walk_preferred_bytes(int64_t num_nodes, int64_t num_edges,
  * 4 bytes per node of int32 row starts (the rows the preparation pass and the
  * CSR mode read).
  * Records are also chosen when num_edges <= 32768 * walk_length, and 256
- * bytes (the LDS walk) under the same conditions as for mlxc_random_walk.
+ * bytes (the LDS walk) under the conditions of mlxc_random_walk's 256.
  * When the call makes row searches (w > 0), the record layout ends with two
  * more parts: per-row hash tables (64 * (num_edges / 8 + num_nodes + 2)
  * bytes), which answer a membership test on a row of 2 to 1023 entries in
@@ -155,10 +160,20 @@ size_t mlxc_rejection_sampling_workspace_bytes(int64_t num_nodes, int64_t num_ed
                                                double p, double q, int32_t rule);
 
 /* Workspace bytes with which mlxc_rejection_sampling is fastest for these
- * arguments: 2 * MLXC_WORK_WORDS * 8, which selects the few-walks kernel (a
- * group of lanes per walk on the CSR arrays as they are; up to 65,536 walks),
- * in calls of few walks, else what mlxc_rejection_sampling_workspace_bytes
- * returns.  No reference counterpart. */
+ * arguments:
+ *   1280 where the older query says 256 and no other layout fits in them: the
+ *     LDS walk, with a status word for each of its blocks;
+ *   2 * MLXC_WORK_WORDS * 8 in calls of few walks (at most 65,536; fewer steps
+ *     the more of them there are and the smaller the graph; of any length
+ *     where num_nodes or num_edges is 2^31 or more): the few-walks kernel, a
+ *     group of lanes per walk on the CSR arrays as they are;
+ *   2 * MLXC_WORK_WORDS * 8 + 16 * ceil(num_edges / 2) + 8192 in such calls
+ *     where the older query asks for hash tables of the records and the call
+ *     takes over 20 steps or 65,536 of all walks together: the few-walks
+ *     kernel with hash tables of unsorted rows.  Exactly this size selects it,
+ *     for the layouts above may fit in it as well;
+ *   else what mlxc_rejection_sampling_workspace_bytes returns.
+ * No reference counterpart. */
 size_t mlxc_rejection_sampling_preferred_bytes(int64_t num_nodes, int64_t num_edges,
                                                int64_t num_walks, int32_t walk_length,
                                                double p, double q, int32_t rule);
@@ -275,11 +290,11 @@ int mlxc_random_walk_seeded(const int64_t* d_rowptr, int64_t num_nodes,
  * whole batch's call): word 0 picks the candidate as in mlxc_random_walk,
  * word 1 gives r = (x1 >> 8) * 2^-24 for the acceptance test against the FP64
  * constants of BiasedRandomWalk.cpp:52-55.  `rows` is one of MLXC_ROWS_*:
- * sorted rows are searched through a 16-ary index, unsorted rows scanned
- * linearly as the reference does; MLXC_ROWS_DETECT decides on the device in
- * the call's preparation pass, the pass that also validates the whole CSR
- * (status bits as above, for every MLXC_ROWS_* value).  No host
- * synchronisation on any path.
+ * sorted rows are searched, unsorted rows scanned linearly as the reference
+ * does or looked up in hash tables of the call's own; MLXC_ROWS_DETECT decides
+ * on the device, from the check that also validates the whole CSR (status
+ * bits as above, for every MLXC_ROWS_* value).  No host synchronisation on any
+ * path.
  */
 int mlxc_rejection_sampling(const int64_t* d_rowptr, int64_t num_nodes,
                             const int64_t* d_col, int64_t num_edges,
@@ -463,7 +478,10 @@ int64_t* mlxc_status_target(void);
 
 /*
  * Measurement hook: times the walk kernel alone, without the preparation
- * launches before it (a call's last launch is its walk kernel).  After
+ * launches before it and the gathering or publishing of the status after it
+ * (a few-walks call that detects the row order without hash tables walks in
+ * two launches, the second of which as a rule returns at once: both are
+ * timed, and the graph's check, which runs beside the first).  After
  * mlxc_set_walk_events(start_event, stop_event), with two hipEvent_t handles
  * created by the caller, every walk call the calling thread makes
  * (mlxc_random_walk*, mlxc_rejection_sampling) records start_event on its
