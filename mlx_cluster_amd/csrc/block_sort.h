@@ -1,5 +1,5 @@
-// Sort of up to kThreads * 16 keys by one block: a bitonic network over keys
-// held in registers, 16 consecutive keys a thread.
+// Sort of up to 16,384 keys of 32 bits by one block of 1,024 threads: a bitonic
+// network over keys held in registers, 16 consecutive keys a thread.
 //
 // Why a network and not radix passes: at 16 keys a thread a network stage
 // costs one VALU instruction a key inside a thread (a min or a max), two
@@ -15,6 +15,7 @@
 
 namespace mlxc {
 
+constexpr int kSortBlock = 1024;    // threads
 constexpr int kSortItems = 16;      // keys per thread
 constexpr int kSortItemBits = 4;
 constexpr int kWaveKeyBits = 10;    // keys of a wavefront: 1,024
@@ -22,12 +23,6 @@ constexpr int kWaveKeyBits = 10;    // keys of a wavefront: 1,024
 // min / max of two keys in one instruction each.
 __device__ __forceinline__ void sort_pair(uint32_t& a, uint32_t& b) {
     const uint32_t lo = a < b ? a : b, hi = a < b ? b : a;
-    a = lo;
-    b = hi;
-}
-__device__ __forceinline__ void sort_pair(uint64_t& a, uint64_t& b) {
-    const bool s = b < a;
-    const uint64_t lo = s ? b : a, hi = s ? a : b;
     a = lo;
     b = hi;
 }
@@ -44,11 +39,6 @@ __device__ __forceinline__ uint32_t lane_xor(uint32_t x) {
     return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true), 0x1B, 0xf,
                                     0xf, true);
 }
-template <int M>
-__device__ __forceinline__ uint64_t lane_xor(uint64_t x) {
-    return (static_cast<uint64_t>(lane_xor<M>(static_cast<uint32_t>(x >> 32))) << 32) |
-           lane_xor<M>(static_cast<uint32_t>(x));
-}
 
 // The smaller of a and b where upper is 0, the larger where it is ~0: the
 // median of the two and the bound.
@@ -57,12 +47,9 @@ __device__ __forceinline__ uint32_t keep_half(uint32_t a, uint32_t b, uint32_t u
     asm("v_med3_u32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(upper));
     return d;
 }
-__device__ __forceinline__ uint64_t keep_half(uint64_t a, uint64_t b, uint32_t upper) {
-    return (b < a) != (upper != 0) ? b : a;
-}
 
-template <int M, typename K>
-__device__ __forceinline__ void row_stage(K (&key)[kSortItems], int lane) {
+template <int M>
+__device__ __forceinline__ void row_stage(uint32_t (&key)[kSortItems], int lane) {
     const uint32_t upper = lane & M ? ~0u : 0u;
 #pragma unroll
     for (int r = 0; r < kSortItems; ++r) key[r] = keep_half(key[r], lane_xor<M>(key[r]), upper);
@@ -82,17 +69,7 @@ __device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
     b = r[1];
 }
 template <int M>
-__device__ __forceinline__ void swap_halves(uint64_t& a, uint64_t& b) {
-    uint32_t a0 = static_cast<uint32_t>(a), a1 = static_cast<uint32_t>(a >> 32);
-    uint32_t b0 = static_cast<uint32_t>(b), b1 = static_cast<uint32_t>(b >> 32);
-    swap_halves<M>(a0, b0);
-    swap_halves<M>(a1, b1);
-    a = (static_cast<uint64_t>(a1) << 32) | a0;
-    b = (static_cast<uint64_t>(b1) << 32) | b0;
-}
-
-template <int M, typename K>
-__device__ __forceinline__ void cross_row_stage(K (&key)[kSortItems]) {
+__device__ __forceinline__ void cross_row_stage(uint32_t (&key)[kSortItems]) {
 #pragma unroll
     for (int r = 0; r < kSortItems; r += 2) {
         swap_halves<M>(key[r], key[r + 1]);
@@ -102,8 +79,8 @@ __device__ __forceinline__ void cross_row_stage(K (&key)[kSortItems]) {
 }
 
 // Strides 2^(bits-1) .. 1 over the register index, ascending.
-template <int kBits, typename K>
-__device__ __forceinline__ void item_stages(K (&key)[kSortItems]) {
+template <int kBits>
+__device__ __forceinline__ void item_stages(uint32_t (&key)[kSortItems]) {
 #pragma unroll
     for (int s = 1 << (kBits - 1); s > 0; s >>= 1) {
 #pragma unroll
@@ -114,17 +91,15 @@ __device__ __forceinline__ void item_stages(K (&key)[kSortItems]) {
 
 // Flips every bit of the keys where m is ~0: an ascending network then sorts
 // them descending.
-template <typename K>
-__device__ __forceinline__ void flip_keys(K (&key)[kSortItems], uint32_t m) {
-    const K mask = static_cast<K>(static_cast<int64_t>(static_cast<int32_t>(m)));
+__device__ __forceinline__ void flip_keys(uint32_t (&key)[kSortItems], uint32_t m) {
 #pragma unroll
-    for (int r = 0; r < kSortItems; ++r) key[r] ^= mask;
+    for (int r = 0; r < kSortItems; ++r) key[r] ^= m;
 }
 
 // Merge step k (blocks of 2^k keys) from stride 2^kTop down, where kTop is
 // below a wavefront's 10 bits.
-template <int kTop, typename K>
-__device__ __forceinline__ void wave_stages(K (&key)[kSortItems], int lane) {
+template <int kTop>
+__device__ __forceinline__ void wave_stages(uint32_t (&key)[kSortItems], int lane) {
     if constexpr (kTop >= 9) cross_row_stage<32>(key);
     if constexpr (kTop >= 8) cross_row_stage<16>(key);
     if constexpr (kTop >= 7) row_stage<8>(key, lane);
@@ -140,26 +115,24 @@ __device__ __forceinline__ uint32_t step_mask(int t, int k) {
     return (t >> (k - kSortItemBits)) & 1 ? ~0u : 0u;
 }
 
-template <int kStep, typename K>
-__device__ __forceinline__ void wave_step(K (&key)[kSortItems], int t, int lane) {
+template <int kStep>
+__device__ __forceinline__ void wave_step(uint32_t (&key)[kSortItems], int t, int lane) {
     flip_keys(key, step_mask(t, kStep - 1) ^ step_mask(t, kStep));
     wave_stages<kStep - 1>(key, lane);
 }
 
 // LDS words of the sort: one key a slot, a pad every 16 so that a thread's 16
 // consecutive keys and a wavefront's consecutive keys both spread over the banks.
-template <int kThreads>
-constexpr int sort_lds_keys() { return kThreads * (kSortItems + 1); }
+constexpr int kSortLds = kSortBlock * (kSortItems + 1);
 __device__ __forceinline__ int sort_slot(int i) { return i + i / kSortItems; }
 
 // Sorts key i (i < n; thread t holds keys 16 t .. 16 t + 15, the ones from n on
-// set to the type's largest value by the caller) ascending over the block.
-// Every thread calls it; contains barriers.  lds: sort_lds_keys<kThreads>()
-// keys, free on entry and on return (after a barrier of the caller's).
-template <int kThreads, typename K>
-__device__ void block_sort(K (&key)[kSortItems], int n, K* lds) {
-    static_assert(kThreads == 256 || kThreads == 512 || kThreads == 1024, "whole wavefronts");
-    constexpr int kBits = kThreads == 256 ? 12 : kThreads == 512 ? 13 : 14;
+// set to ~0 by the caller) ascending over the block.  Every thread calls it;
+// contains barriers.  lds: kSortLds keys, free on entry and on return (after a
+// barrier of the caller's).
+__device__ inline void block_sort(uint32_t (&key)[kSortItems], int n, uint32_t* lds) {
+    constexpr int kBits = 14;
+    static_assert(kSortBlock * kSortItems == 1 << kBits, "16,384 keys");
     // The other layout: thread t holds keys (r << kLow) | t, so that the
     // strides 2^kLow and up lie inside a thread.
     constexpr int kLow = kBits - kSortItemBits;

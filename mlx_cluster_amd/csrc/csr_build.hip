@@ -720,7 +720,7 @@ struct SmallRange {
     uint32_t first, last; // the smallest and the largest
 };
 
-// A fixed scramble of sample numbers.
+// A fixed scramble of sample numbers: Wellons' lowbias32 integer hash.
 __host__ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
     x ^= x >> 16;
     x *= 0x7feb352du;
@@ -805,8 +805,8 @@ __device__ __forceinline__ void rank_keys(const uint32_t* keys, int n, int32_t* 
 __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
     EdgeSrc src, int total, int ways, bool dedup, uint32_t* __restrict__ keys,
     SmallRange* __restrict__ ranges, int64_t* __restrict__ work) {
-    static_assert(kSortItems == kItems, "16 keys a thread");
-    __shared__ __align__(16) uint32_t lds[sort_lds_keys<kSmallThreads>()];
+    static_assert(kSortItems == kItems && kSortBlock == kSmallThreads, "block_sort's layout");
+    __shared__ __align__(16) uint32_t lds[kSortLds];
     __shared__ int32_t rank[kSmallThreads];
     __shared__ uint32_t last[kSmallThreads];
     __shared__ int64_t wtot[kSmallThreads / kWave];
@@ -940,7 +940,7 @@ __global__ __launch_bounds__(kSmallThreads) void small_sort_kernel(
 #pragma unroll
         for (int q = 0; q < kItems; ++q) key[q] = at + q * kWave < n ? lds[at + q * kWave] : ~0u;
         __syncthreads();
-        block_sort<kSmallThreads>(key, n, lds);
+        block_sort(key, n, lds);
         last[t] = key[kItems - 1];
         __syncthreads();
         const uint32_t before = t > 0 ? last[t - 1] : prev_last;
