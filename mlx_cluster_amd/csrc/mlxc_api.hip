@@ -225,39 +225,6 @@ HostWalk host_walk(const int64_t* rowptr, int64_t num_nodes, const int64_t* col,
                     static_cast<uint32_t>(seed >> 32), first_walk};
 }
 
-__global__ void publish_status_kernel(const int64_t* work, int64_t* h_status, bool count) {
-    if (threadIdx.x != 0) return;
-    if (count) publish_count(work[0], work[1], h_status);
-    else publish(work[0], h_status);
-}
-
-// See launch_finish; h_status may be null.  Bound by its loads' latency: the
-// words of 2,000 blocks a word a read, up to eight in a row a thread, against
-// two reads of four words: a validated call of 2,000 walks x 5 steps 17.7 ->
-// 16.3 us.
-__global__ __launch_bounds__(kBlock) void finish_kernel(const uint32_t* __restrict__ block_status,
-                                                        int blocks, int64_t* __restrict__ work,
-                                                        int64_t* h_status) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
-    uint32_t bits = 0;
-    const int quads = blocks / 4;
-#pragma unroll 2
-    for (int i = threadIdx.x; i < quads; i += kBlock) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(block_status + 4 * i);
-        bits |= v.x | v.y | v.z | v.w;
-    }
-    const int rest = 4 * quads + static_cast<int>(threadIdx.x);
-    if (rest < blocks) bits |= block_status[rest];
-    const bool node = __syncthreads_or(bits & MLXC_STATUS_BAD_NODE);
-    const bool row = __syncthreads_or(bits & MLXC_STATUS_BAD_ROW);
-    if (threadIdx.x == 0) {
-        const int64_t all = (node ? MLXC_STATUS_BAD_NODE : 0) | (row ? MLXC_STATUS_BAD_ROW : 0);
-        work[0] = all;
-        for (int i = 1; i < MLXC_WORK_WORDS; ++i) work[i] = 0;
-        if (h_status) publish(all, h_status);
-    }
-}
-
 // Device address of host words the device can write, or null.
 int64_t* device_words(int64_t* h_status) {
     int64_t* d = nullptr;
@@ -275,22 +242,11 @@ int end_call(int rc, const int64_t* d_work, bool count, hipStream_t s) {
     const bool done = g_status_target.done;
     g_status_target.done = false;
     if (rc != MLXC_OK || !g_status_target.words || done) return rc;
-    hipLaunchKernelGGL(publish_status_kernel, dim3(1), dim3(kWave), 0, s, d_work,
-                       g_status_target.words, count);
-    MLXC_HIP_TRY(hipGetLastError());
-    return MLXC_OK;
+    return launch_publish(d_work, g_status_target.words, count, s);
 }
 int end_walk(int rc, const int64_t* d_work, hipStream_t s) { return end_call(rc, d_work, false, s); }
 
 }  // namespace
-
-int launch_finish(const uint32_t* block_status, int64_t blocks, int64_t* work, hipStream_t stream) {
-    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(kBlock), 0, stream, block_status,
-                       static_cast<int>(blocks), work, g_status_target.words);
-    MLXC_HIP_TRY(hipGetLastError());
-    g_status_target.done = g_status_target.words != nullptr;
-    return MLXC_OK;
-}
 
 }  // namespace mlxc
 
@@ -310,11 +266,8 @@ int mlxc_publish_status(const void* d_workspace, int64_t* h_status, void* stream
     if (!d_status)
         return fail(MLXC_ERR_INVALID_ARGUMENT,
                     "h_status is not host memory the device can write (hipHostMalloc)");
-    hipLaunchKernelGGL(publish_status_kernel, dim3(1), dim3(kWave), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const int64_t*>(d_workspace),
-                       d_status, false);
-    MLXC_HIP_TRY(hipGetLastError());
-    return MLXC_OK;
+    return launch_publish(static_cast<const int64_t*>(d_workspace), d_status, false,
+                          static_cast<hipStream_t>(stream));
 }
 
 int mlxc_set_status_target(int64_t* h_status) {

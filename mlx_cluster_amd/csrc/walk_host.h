@@ -50,6 +50,9 @@ extern thread_local StatusTarget g_status_target;
 // the thread has a target.  One launch in place of the reset before the walk
 // and the publication after it.
 int launch_finish(const uint32_t* block_status, int64_t blocks, int64_t* work, hipStream_t stream);
+// Stores a call's status word (count: and its entry count) into host words at
+// device address d_status.
+int launch_publish(const int64_t* work, int64_t* d_status, bool count, hipStream_t stream);
 
 struct DeviceInfo {
     int cus = 0;  // compute units of the current device
