@@ -130,6 +130,25 @@ def test_budgets_equal_the_unchunked_call(kind, out_dtype, cuda):
         assert torch.equal(gn.cpu(), n.cpu()) and torch.equal(ge.cpu(), e.cpu())
 
 
+@pytest.mark.parametrize("kind", ["uniform", "seeded"])
+def test_uniform_budgets_below_the_record_workspace(kind, cuda):
+    """A call long enough for the edge records with budgets that leave less than
+    they need: start records, then the status words alone."""
+    rowptr, col = synth.rmat_csr(14, 200_000, seed=4, device=cuda, symmetrize=True)
+    V, E = rowptr.numel() - 1, col.numel()
+    N, L = 70_001, 180
+    lib = mc._lib.load()
+    ws = lib.mlxc_random_walk_workspace_bytes(V, E, N, L)
+    assert ws == lib.mlxc_random_walk_preferred_bytes(V, E, N, L) > 256 + 8 * E
+    start = (torch.arange(N, device=cuda) * 7) % V
+    rand = mc.philox_uniform((N, L), 9, device=cuda)
+    n, e = _walk(kind, rowptr, col, start, L, rand)
+    outs = N * (2 * L + 1) * 8
+    for budget in (outs + ws - 1, outs + 256 + 16 * N + 15, outs + 64):
+        gn, ge = _walk(kind, rowptr, col, start, L, rand, memory_budget=budget)
+        assert gn.is_cuda and torch.equal(gn, n) and torch.equal(ge, e)
+
+
 def test_chunked_call_reports_a_bad_start_in_a_later_chunk(cuda):
     """The status bits of every chunk reach the caller: a start out of range
     in the last chunk raises ValueError, as in the unchunked call."""

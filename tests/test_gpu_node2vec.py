@@ -591,8 +591,8 @@ def test_lds_walk_lane_groups(N, cuda):
 def test_lds_walks_random_sweep(cuda):
     """Random small graphs (directed and undirected, duplicates and
     self-loops kept) under the LDS limit, random walk counts and lengths:
-    the uniform and node2vec LDS walks (the Python API's default for these
-    sizes) are bit-exact against the oracle for both rules and several
+    the uniform flat walk and the node2vec LDS walk (the Python API's default
+    for these sizes) are bit-exact against the oracle for both rules and several
     (p, q)."""
     from mlx_cluster_amd import _lib
     lib = _lib.load()
@@ -608,7 +608,7 @@ def test_lds_walks_random_sweep(cuda):
         N = int(rng.integers(1, 3000))
         L = int(rng.integers(1, 50))
         start = rng.integers(0, V, N)
-        # the Python API takes the LDS walks here, whatever N * L is
+        # the Python API takes those walks here, whatever N * L is
         assert lib.mlxc_random_walk_workspace_bytes(V, col.size, N, L) == 256
         assert lib.mlxc_rejection_sampling_workspace_bytes(V, col.size, N, L, 1.0, 1.0, 0) == 256
         rand = mc.philox_uniform((N, L), case, device=cuda)

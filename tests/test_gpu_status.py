@@ -19,7 +19,7 @@ from tests import status_cases as sc
 
 pytestmark = pytest.mark.gpu
 
-N2V_MODES = ("lds", "records", "csr", "direct")
+N2V_MODES = ("lds", "records", "csr", "few", "few_tables", "direct")
 ROWS = (_lib.MLXC_ROWS_UNSORTED, _lib.MLXC_ROWS_SORTED, _lib.MLXC_ROWS_DETECT)
 
 
@@ -34,8 +34,11 @@ def _n2v_status(rowptr, col, start, L, seed, rows, mode, cuda):
     p, q, rule = 0.5, 2.0, _lib.MLXC_RULE_REF_CHAIN
     query = lambda n_, l_: lib.mlxc_rejection_sampling_workspace_bytes(V, E, n_, l_, p, q, rule)
     layout = {"direct": _lib.MLXC_N2V_LAYOUT_DIRECT, "csr": _lib.MLXC_N2V_LAYOUT_CSR,
-              "records": _lib.MLXC_N2V_LAYOUT_RECORDS_FULL, "lds": _lib.MLXC_N2V_LAYOUT_LDS}[mode]
-    nbytes = max(lib.mlxc_rejection_sampling_layout_bytes(V, E, N, L, layout), 32)
+              "records": _lib.MLXC_N2V_LAYOUT_RECORDS_FULL, "lds": _lib.MLXC_N2V_LAYOUT_LDS}
+    if mode in layout:
+        nbytes = max(lib.mlxc_rejection_sampling_layout_bytes(V, E, N, L, layout[mode]), 32)
+    else:
+        nbytes = {"few": 64, "few_tables": 64 + (E + 1) // 2 * 16 + 8192}[mode]
     if mode == "lds":
         assert query(N, L) == 256  # the query itself selects the LDS walk here
     ws = torch.full(((nbytes + 7) // 8,), -1, dtype=torch.int64, device=cuda)
@@ -96,7 +99,7 @@ def _uniform_status(rowptr, col, start, L, mode, seeded, cuda):
 def test_uniform_status_same_on_every_path(case, cuda):
     """16 walks (the case's starts repeated), so that N * L is a multiple of
     4 and at least 16: the rand tensor then allows the windowed kernels, and
-    the record, CSR and LDS workspaces select those walks."""
+    the record and CSR workspaces select those walks, the others the flat walk."""
     name, rowptr, col, start, L, want = case
     lib = _lib.load()
     start = np.resize(np.asarray(start, np.int64), 16)

@@ -111,7 +111,8 @@ def test_repeatable_and_side_stream(cuda):
     assert torch.equal(a, b)
 
 
-def test_side_stream_call_is_ordered_and_keeps_its_memory(cuda):
+@pytest.mark.parametrize("L", [30, 200])
+def test_side_stream_call_is_ordered_and_keeps_its_memory(L, cuda):
     """A call on a side stream with check=False: its kernels run after the
     work queued on torch's current stream (here an input written there
     behind a spin kernel of bounded length), and the allocator hands out
@@ -121,8 +122,10 @@ def test_side_stream_call_is_ordered_and_keeps_its_memory(cuda):
     node2vec walks equal the oracle's."""
     rowptr, col = synth.rmat_csr(12, 40_000, seed=5)
     rowptr, col = rowptr.numpy(), col.numpy()
-    V, L = rowptr.size - 1, 30
-    start = (np.arange(20 * V) % V).astype(np.int64)   # many steps per edge: records
+    V = rowptr.size - 1
+    # many steps per edge: records (of the uniform walk at 200 steps, where the
+    # flat walk ends; of the node2vec walk at both)
+    start = (np.arange(20 * V) % V).astype(np.int64)
     rand = oracle.philox_uniform(start.size * L, 6).reshape(start.size, L)
     n_ref, e_ref, _, _ = oracle.uniform_walk(rowptr, col, start, rand, L, with_edges=True)
     n2v_ref, _, _, _ = oracle.node2vec_walk(rowptr, col, start, L, 0.5, 2.0, 9)
@@ -130,7 +133,9 @@ def test_side_stream_call_is_ordered_and_keeps_its_memory(cuda):
     s = torch.cuda.Stream(device=cuda)
     rand_dev = torch.full(rand.shape, 0.5, dtype=torch.float32, device=cuda)
     lib = mc._lib.load()
-    ws_words = lib.mlxc_random_walk_workspace_bytes(V, col.size, start.size, L) // 8 + 1
+    ws_bytes = lib.mlxc_random_walk_workspace_bytes(V, col.size, start.size, L)
+    assert (lib.mlxc_random_walk_preferred_bytes(V, col.size, start.size, L) == ws_bytes) == (L == 200)
+    ws_words = ws_bytes // 8 + 1
     torch.cuda._sleep(20_000_000)          # bounded spin on the current stream
     rand_dev.copy_(torch.from_numpy(rand).to(cuda, non_blocking=False))
     n, e = mc.random_walk(rowptr, col, start, rand_dev, L, stream=s, check=False,
@@ -171,7 +176,7 @@ def test_c2_full_size_properties(cuda):
     """Configuration 2 at full size (R-MAT 2^20, 10 walks per node, L=80):
     every one of the 838,860,800 steps is checked against numpy-free torch
     float32 arithmetic on the device, and a sample of walks bit-exactly
-    against the oracle; the unwindowed kernel gives the same walks in full."""
+    against the oracle; the flat walk gives the same walks in full."""
     rowptr, col = synth.rmat_csr(20, 1 << 24, seed=0, device=cuda)
     V = rowptr.numel() - 1
     N, L = 10 * V, 80
@@ -197,8 +202,7 @@ def test_c2_full_size_properties(cuda):
                                           rand[sample].cpu().numpy(), L)
     assert st == 0
     np.testing.assert_array_equal(n[sample].cpu().numpy(), n_ref)
-    # the unwindowed kernel (the path of graphs beyond int32 ids, forced by a
-    # minimal workspace) gives the same walks in full
+    # the flat walk (forced by a minimal workspace) gives the same walks in full
     n2 = torch.empty_like(n)
     _abi_walk(rowptr, col, start, rand.data_ptr(), L, n2.data_ptr(), ws_bytes=32)
     assert torch.equal(n2, n)
@@ -210,7 +214,7 @@ def test_c4_full_size_properties(cuda):
     than 4 steps per edge): every one of the 335,544,320 steps and its edge id
     is checked against torch float32 arithmetic on the device, and 4,000
     sampled walks bit-exactly against the oracle, nodes and edges; the
-    unwindowed kernel gives the same walks and edges in full."""
+    flat walk gives the same walks and edges in full."""
     rowptr, col = synth.rmat_csr(24, 1 << 28, seed=0, device=cuda)
     V, E = rowptr.numel() - 1, col.numel()
     N, L = V, 20
@@ -242,8 +246,7 @@ def test_c4_full_size_properties(cuda):
     assert st == 0
     np.testing.assert_array_equal(n[sample].cpu().numpy(), n_ref)
     np.testing.assert_array_equal(e[sample].cpu().numpy(), e_ref)
-    # the unwindowed kernel (the path of graphs beyond int32 ids, forced by a
-    # minimal workspace) gives the same walks and edges in full
+    # the flat walk (forced by a minimal workspace) gives the same walks and edges in full
     n2, e2 = torch.empty_like(n), torch.empty_like(e)
     _abi_walk(rowptr, col, start, rand.data_ptr(), L, n2.data_ptr(), e_out=e2, ws_bytes=32)
     assert torch.equal(n2, n) and torch.equal(e2, e)
@@ -253,8 +256,8 @@ def _abi_walk(rowptr, col, start, rand_t, L, n_out_t, *, e_out=None, ws_bytes=No
               out_type=0):
     """Calls mlxc_random_walk directly so each kernel path can be selected:
     edge records (full workspace, many steps per edge), CSR reads with start
-    records (workspace for start records only), and the unwindowed kernel
-    (minimal workspace, edge output or unaligned buffers)."""
+    records (workspace for start records only), and the flat walk (minimal
+    workspace or unaligned output buffers)."""
     from mlx_cluster_amd import _lib
     lib = _lib.load()
     V, E = rowptr.numel() - 1, col.numel()
@@ -270,12 +273,26 @@ def _abi_walk(rowptr, col, start, rand_t, L, n_out_t, *, e_out=None, ws_bytes=No
     assert int(ws[0].item()) == 0
 
 
+def _abi_seeded(rowptr, col, start, seed, L, n_out, e_out, ws_bytes, expect_status=0):
+    """mlxc_random_walk_seeded with a workspace of ws_bytes."""
+    from mlx_cluster_amd import _lib
+    ws = torch.empty((ws_bytes + 7) // 8, dtype=torch.int64, device=rowptr.device)
+    rc = _lib.load().mlxc_random_walk_seeded(
+        rowptr.data_ptr(), rowptr.numel() - 1, col.data_ptr(), col.numel(), start.data_ptr(),
+        start.numel(), L, seed, 0, n_out.data_ptr(), None if e_out is None else e_out.data_ptr(),
+        int(n_out.dtype == torch.int32), ws.data_ptr(), ws_bytes,
+        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.last_error()
+    torch.cuda.synchronize()
+    assert int(ws[0].item()) == expect_status
+
+
 @pytest.mark.parametrize("N,L", [(1, 1), (33, 5), (257, 4), (1000, 16), (4096, 23),
                                  (20_000, 80)])
 def test_all_kernel_paths_agree(N, L, cuda):
     # small graph (E <= 300) so that most shapes take >= 4 * E steps: the
-    # full workspace then selects the edge-record walk; N * L not a multiple
-    # of 4 selects the unwindowed kernel whatever the workspace
+    # full workspace then selects the edge-record walk, but for a rand tensor
+    # of fewer floats than a window
     rowptr, col = synth.rmat_csr(7, 300, seed=N, device=cuda)
     V = rowptr.numel() - 1
     start = (torch.arange(N, device=cuda) * 131) % V
@@ -295,7 +312,7 @@ def test_all_kernel_paths_agree(N, L, cuda):
             np.testing.assert_array_equal(out.cpu().numpy(), ref, err_msg=f"{name} {edges}")
             if edges:
                 np.testing.assert_array_equal(e.cpu().numpy(), ref_e, err_msg=f"{name} edges")
-    # unaligned rand (4-byte offset), n_out and e_out (8-byte offsets): unwindowed kernel
+    # unaligned rand (4-byte offset), n_out and e_out (8-byte offsets): the flat walk
     rand_u = mc.philox_uniform(N * L + 1, 0, device=cuda)
     rand_u[1:] = rand[:N * L]
     big = torch.full((N * (L + 1) + 1,), -7, dtype=torch.int64, device=cuda)
@@ -354,6 +371,16 @@ def test_record_formats_and_long_rows(packed, cuda):
     np.testing.assert_array_equal(n.cpu().numpy()[sample], n_ref)
     np.testing.assert_array_equal(e.cpu().numpy()[sample], e_ref)
     assert np.isin(n_ref[:, :-1], hubs[1:]).sum() > 1000   # steps leaving the long rows
+    # (the Python layer's calls take the flat walk at this size)
+    n_rec, e_rec = torch.empty_like(n), torch.empty_like(e)
+    _abi_walk(rp, cl, st, rand.data_ptr(), L, n_rec.data_ptr(), e_out=e_rec,
+              ws_bytes=256 + (8 if packed else 16) * (E + N))
+    assert torch.equal(n_rec, n) and torch.equal(e_rec, e)
+    _abi_seeded(rp, cl, st, 31, L, n_rec, e_rec, 256 + (8 if packed else 16) * (E + N))
+    assert torch.equal(n_rec, n) and torch.equal(e_rec, e)
+    n_rec32 = torch.empty_like(n, dtype=torch.int32)
+    _abi_seeded(rp, cl, st, 31, L, n_rec32, None, 256 + (8 if packed else 16) * (E + N))
+    assert torch.equal(n_rec32.long(), n)
     assert torch.equal(mc.random_walk(rp, cl, st, None, L, seed=31), n)
     n32 = mc.random_walk(rp, cl, st, None, L, seed=31, out_dtype=torch.int32)
     assert torch.equal(n32.long(), n)
@@ -382,13 +409,18 @@ def test_packed_degree_field_cap(cuda):
     np.testing.assert_array_equal(n.cpu().numpy()[sample], n_ref)
     np.testing.assert_array_equal(e.cpu().numpy()[sample], e_ref)
     assert np.isin(n_ref[:, :-1], hubs).sum() > 1000
+    n_rec, e_rec = torch.empty_like(n), torch.empty_like(e)
+    _abi_walk(rp, cl, st, rand.data_ptr(), L, n_rec.data_ptr(), e_out=e_rec,
+              ws_bytes=256 + 8 * (E + N))
+    assert torch.equal(n_rec, n) and torch.equal(e_rec, e)
 
 
 @pytest.mark.parametrize("N,L", [(1, 1), (37, 5), (1000, 16), (4096, 23), (30_000, 80)])
 def test_seeded_uniforms_match_rand_tensor(N, L, cuda):
     """rand=None, seed=s generates in the kernel exactly the stream
-    philox_uniform((N, L), s) holds: every kernel path (edge records, CSR
-    reads, edge output) gives the walks of the explicit tensor, and the oracle's."""
+    philox_uniform((N, L), s) holds: every kernel path (flat, and with the
+    workspaces that select them edge records and CSR reads; edge output) gives
+    the walks of the explicit tensor, and the oracle's."""
     rowptr, col = synth.rmat_csr(9, 3000, seed=N, device=cuda)
     V = rowptr.numel() - 1
     start = (torch.arange(N, device=cuda) * 17) % V
@@ -404,6 +436,10 @@ def test_seeded_uniforms_match_rand_tensor(N, L, cuda):
                                         start.cpu().numpy(), oracle.philox_uniform(N * L, seed), L)
     assert st == 0
     np.testing.assert_array_equal(got.cpu().numpy(), ref)
+    for ws_bytes in (256 + 16 * (col.numel() + N), 256 + 16 * N):
+        n, e = torch.empty_like(want_n), torch.empty_like(want_e)
+        _abi_seeded(rowptr, col, start, seed, L, n, e, ws_bytes)
+        assert torch.equal(n, want_n) and torch.equal(e, want_e)
 
 
 def test_cpu_twin_equals_gpu(cuda):
@@ -454,7 +490,7 @@ def test_long_and_block_sized_walks_with_sinks(L, cuda):
 def test_int32_output_all_kernel_paths(L, cuda):
     """out_type MLXC_OUT_INT32 (8-entry blocks of 32 bytes, two lanes per
     block in the wavefront stores): nodes and edges equal the int64 output
-    for the record walk, the CSR walk and the unwindowed kernel, and the
+    for the record walk, the CSR walk and the flat walk, and the
     oracle."""
     rowptr, col = synth.rmat_csr(10, 4000, seed=46, device=cuda)
     V, E = rowptr.numel() - 1, col.numel()
@@ -479,12 +515,12 @@ def test_int32_output_all_kernel_paths(L, cuda):
 
 @pytest.mark.parametrize("V,E_target", [(50, 300), (2708, 10556), (3000, 14336 - 3001)])
 def test_lds_walk(V, E_target, cuda):
-    """Graphs whose rowptr and col fit in LDS (V + 1 + E <= 14,336 entries) on
-    calls of 1 to 2^20 steps take the LDS walk (the workspace query asks for
-    the 256-byte header only).  Nodes and edges bit-exact against the oracle
-    with a rand tensor and generated uniforms, int64 and int32 output, sinks
-    included; a graph one entry over the limit takes the record walk with
-    the same results."""
+    """Graphs whose rowptr and col would fit in LDS (V + 1 + E <= 14,336 entries,
+    where the node2vec walk keeps them there) on calls of 1 to 2^20 steps: the
+    workspace query asks for the 256-byte header only, the flat walk.  Nodes
+    and edges bit-exact against the oracle with a rand tensor and generated
+    uniforms, int64 and int32 output, sinks included; for a graph one entry
+    over the limit the query asks for the record walk, with the same results."""
     from mlx_cluster_amd import _lib
     lib = _lib.load()
     rng = np.random.default_rng(V)
@@ -512,7 +548,7 @@ def test_lds_walk(V, E_target, cuda):
         np.testing.assert_array_equal(n32.cpu().numpy(), n_ref)
         g = mc.random_walk(t(rowptr), t(col), t(start), None, L, seed=N + L)
         np.testing.assert_array_equal(g.cpu().numpy(), n_ref)
-    # exactly at the limit (the LDS walk) and one entry over it (the record walk)
+    # exactly at the limit and one entry over it (the record walk)
     base = np.stack([np.repeat(np.arange(V), np.diff(rowptr)), col], 1)
     for total, lds in ((14336, True), (14337, False)):
         rp2, cl2 = csr(V, np.concatenate([base, np.tile([[0, 1]], (total - (V + 1 + E), 1))]))
@@ -526,11 +562,15 @@ def test_lds_walk(V, E_target, cuda):
         n = mc.random_walk(torch.as_tensor(rp2).to(cuda), torch.as_tensor(cl2).to(cuda),
                            torch.as_tensor(start).to(cuda), rand, L)
         np.testing.assert_array_equal(n.cpu().numpy(), n_ref)
+        _abi_walk(torch.as_tensor(rp2).to(cuda), torch.as_tensor(cl2).to(cuda),
+                  torch.as_tensor(start).to(cuda), rand.data_ptr(), L, n.fill_(-7).data_ptr(),
+                  ws_bytes=lib.mlxc_random_walk_workspace_bytes(V, cl2.size, N, L))
+        np.testing.assert_array_equal(n.cpu().numpy(), n_ref)
 
 
 def test_lds_walk_flags_bad_input(cuda):
-    """Out-of-range starts, col entries and rowptr entries met by an LDS walk
-    raise ValueError, as on the other paths."""
+    """Out-of-range starts, col entries and rowptr entries met by a walk on such
+    a graph raise ValueError, as on the other paths."""
     rowptr, col = csr(4, [(0, 1), (1, 2), (2, 3), (3, 0)])
     t = lambda a: torch.as_tensor(np.asarray(a, dtype=np.int64)).to(cuda)
     rand = torch.full((2, 3), 0.5, device=cuda)
@@ -565,14 +605,16 @@ def _check_steps(rowptr, col, rand, n, e, L):
 
 def test_graph_beyond_int32_edge_ids(cuda):
     """A graph of 2^31 + 2^20 CSR entries (2^20 nodes of degree 2049, 17.2 GB
-    of col): the workspace query asks for 16-byte start records, and the
-    wide CSR walk runs with int64 edge ids.  Every step and edge id is
-    re-derived on the device, the unwindowed kernel gives the same walks and
-    edges, and 2,000 walks are bit-exact against the oracle; 4,096 node2vec
-    walks (the direct kernel, linear scans of the unsorted rows) are too; a
-    bad col entry and a bad rowptr entry met by a walk raise.  Then a row of 2^31 + 5
-    entries: its start record marks it long, the walk reads its bounds from
-    rowptr and picks with the float32 rule's rounded degree."""
+    of col): the older workspace query asks for 16-byte start records, with
+    which the wide CSR walk runs with int64 edge ids; the Python layer takes
+    the flat walk.  Every step and edge id is re-derived on the device, the
+    wide CSR walk and the smallest workspace give the same walks and edges,
+    and 2,000 walks are bit-exact against the oracle; 4,096 node2vec walks (the
+    few-walks kernel and the direct one, linear scans of the unsorted rows)
+    are too; a bad col entry and a bad rowptr entry met by a walk raise, and
+    set the wide CSR walk's bits.  Then a row of 2^31 + 5 entries: its start
+    record marks it long, the wide CSR walk reads its bounds from rowptr and
+    picks with the float32 rule's rounded degree."""
     from mlx_cluster_amd import _lib
     q = _lib.load().mlxc_random_walk_workspace_bytes
     V, deg, L = 1 << 20, 2049, 20
@@ -592,6 +634,11 @@ def test_graph_beyond_int32_edge_ids(cuda):
     n2, e2 = torch.empty_like(n), torch.empty_like(e)
     _abi_walk(rowptr, col, start, rand.data_ptr(), L, n2.data_ptr(), e_out=e2, ws_bytes=32)
     assert torch.equal(n2, n) and torch.equal(e2, e)
+    n2.fill_(-7)
+    e2.fill_(-7)
+    _abi_walk(rowptr, col, start, rand.data_ptr(), L, n2.data_ptr(), e_out=e2,
+              ws_bytes=256 + 16 * N)
+    assert torch.equal(n2, n) and torch.equal(e2, e)
     del n2, e2
     sample = torch.randint(0, N, (2000,), generator=torch.Generator().manual_seed(3)).to(cuda)
     rp, cl = rowptr.cpu().numpy(), col.cpu().numpy()
@@ -600,8 +647,9 @@ def test_graph_beyond_int32_edge_ids(cuda):
     assert st == 0
     np.testing.assert_array_equal(n[sample].cpu().numpy(), n_ref)
     np.testing.assert_array_equal(e[sample].cpu().numpy(), e_ref)
-    # node2vec on the same graph takes its direct kernel (int64 positions);
-    # the rows are unsorted, so the device check picks linear scans
+    # node2vec on the same graph, with int64 positions: the few-walks kernel
+    # through the Python layer, the direct one with the smallest workspace; the
+    # rows are unsorted, so the device check picks linear scans
     w = mc.rejection_sampling(rowptr, col, start[:4096], 5, 0.5, 2.0, seed=13, return_edges=True)
     w_ref, we_ref, st, _ = oracle.node2vec_walk(rp, cl, start[:4096].cpu().numpy(), 5, 0.5, 2.0,
                                                 13, rule=oracle.RULE_REF_CHAIN, rows_sorted=False,
@@ -609,16 +657,29 @@ def test_graph_beyond_int32_edge_ids(cuda):
     assert st == 0
     np.testing.assert_array_equal(w[0].cpu().numpy(), w_ref)
     np.testing.assert_array_equal(w[1].cpu().numpy(), we_ref)
+    ws = torch.empty(4, dtype=torch.int64, device=cuda)
+    w[0].fill_(-7)
+    w[1].fill_(-7)
+    rc = _lib.load().mlxc_rejection_sampling(
+        rowptr.data_ptr(), V, col.data_ptr(), E, start.data_ptr(), 4096, 5, 0.5, 2.0, 13, 0, 0,
+        _lib.MLXC_ROWS_DETECT, w[0].data_ptr(), w[1].data_ptr(), _lib.MLXC_OUT_INT64,
+        ws.data_ptr(), 32, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and int(ws[0]) == 0
+    np.testing.assert_array_equal(w[0].cpu().numpy(), w_ref)
+    np.testing.assert_array_equal(w[1].cpu().numpy(), we_ref)
     del cl, rp, w
     # malformed input met by a walk: walk 0's first edge, then its start's row
     first = int(e[0, 0])
     col[first] = V
+    out = torch.empty((64, L + 1), dtype=torch.int64, device=cuda)
     with pytest.raises(ValueError, match="outside"):
         mc.random_walk(rowptr, col, start[:64], rand[:64], L)
+    _abi_seeded(rowptr, col, start[:64], 7, L, out, None, 256 + 16 * 64, _lib.MLXC_STATUS_BAD_NODE)
     col[first] = 0
     rowptr[1] = E + 1
     with pytest.raises(ValueError, match="rowptr"):
         mc.random_walk(rowptr, col, start[:64], rand[:64], L)
+    _abi_seeded(rowptr, col, start[:64], 7, L, out, None, 256 + 16 * 64, _lib.MLXC_STATUS_BAD_ROW)
     del col, n, e, rowptr
     torch.cuda.empty_cache()
 
@@ -635,6 +696,11 @@ def test_graph_beyond_int32_edge_ids(cuda):
     assert int(e[start == 0, 0].max()) > 2**30  # first steps spread over the long row
     n2, e2 = torch.empty_like(n), torch.empty_like(e)
     _abi_walk(rowptr, col, start, rand.data_ptr(), L, n2.data_ptr(), e_out=e2, ws_bytes=32)
+    assert torch.equal(n2, n) and torch.equal(e2, e)
+    n2.fill_(-7)
+    e2.fill_(-7)
+    _abi_walk(rowptr, col, start, rand.data_ptr(), L, n2.data_ptr(), e_out=e2,
+              ws_bytes=256 + 16 * N)
     assert torch.equal(n2, n) and torch.equal(e2, e)
     del col, n, e, n2, e2
     torch.cuda.empty_cache()
