@@ -734,6 +734,10 @@ enum class FewPass {
 // entries a round (1, 4, 8, 16):
 //   31 M entries:   1,300 walks 2,990, 1,270, 791, 530;  65,536 133,000, 54,100, 32,100, 19,900
 //   955 K entries:  1,300 walks 487, 287, 244, 225;  65,536 17,200, 6,510, 4,390, 3,430
+// (all with up to kFewSearches trials scanned at once, whatever the rows' length;
+// one at a time where the rows are long: 530 -> 474, 19,900 -> 13,200, 225 -> 225,
+// 3,430 -> 2,560; 65,536 walks x 20 over 2.1 G entries in rows of 2,049, p = 4,
+// q = 0.25, analytic: 59.7 -> 8.1 ms, the direct kernel 28.3)
 #ifndef MLXC_FEW_SCAN
 #define MLXC_FEW_SCAN 16
 #endif
@@ -752,9 +756,9 @@ constexpr int kFewScan = MLXC_FEW_SCAN;
 // no more than the launch that would repeat the walks.
 // Unsorted rows (detected), 40 steps, us a call, records / scans / tables:
 //   54 K entries, p = 0.5, q = 2, chain:   1,300 walks 178 / 171 / 114,
-//                                          65,536 walks 839 / 1,088 / 251
-//   955 K, p = 4, q = 0.25, analytic:      1,300 walks 273 / 288 / 192,
-//                                          65,536 walks 531 / 6,267 / 363
+//                                          65,536 walks 839 / 1,010 / 251
+//   955 K, p = 4, q = 0.25, analytic:      1,300 walks 273 / 285 / 192,
+//                                          65,536 walks 531 / 3,480 / 363
 __device__ __forceinline__ uint32_t row_slot(int32_t id, int64_t slots) {
     return static_cast<uint32_t>(
         (static_cast<uint64_t>(static_cast<uint32_t>(id) * 0x9E3779B1u) * static_cast<uint64_t>(slots)) >> 32);
@@ -1062,7 +1066,17 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
                     // trial order, on equal shares of its lanes
                     const int m = __popcll(open);
                     int Q = 1;
-                    while (Q < m && Q < kFewSearches && Q < G) Q *= 2;
+                    // (a scan takes as many rounds with all lanes on one trial
+                    // as with shares of them on several, of which the first may
+                    // do: several only where each share covers the first row)
+                    Id row_len = 0;
+                    if (kScan) {
+                        const Id len = s_hi - s_lo;
+                        row_len = __shfl(len, base + (open ? __builtin_ctzll(open) : 0), kWave);
+                        if (!scan || tables) row_len = 0;
+                    }
+                    while (Q < m && Q < kFewSearches && Q < G && row_len <= kFewScan * G / (2 * Q))
+                        Q *= 2;
                     const int C = G / Q, q = k / C, c = k % C;
                     uint64_t rest = open;
                     for (int i = 0; i < q; ++i) rest &= rest - 1;
