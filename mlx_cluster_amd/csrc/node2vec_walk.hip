@@ -705,10 +705,10 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 // The call must validate the whole graph.  The walk does not wait for that:
 // blocks from walk_blocks on check the CSR beside it (the walk bounds every
 // index it uses itself).  Only the row order of MLXC_ROWS_DETECT matters to
-// it: it assumes sorted rows, and a second launch (kAgain) repeats the walks
-// with scans when the check has found otherwise.  Scans are an instantiation
-// of their own (kScan), for their loads take 32 registers.  Calls with row
-// tables check first (kChecked).
+// it: it assumes sorted rows, and a second launch repeats the walks with scans
+// when the check has found otherwise.  Each way to search a row is code of its
+// own (FewFind): a scan's loads take 32 registers, and the choice made at each
+// search cost sorted rows up to 5%.  Calls with row tables check first.
 //
 // Measured (us a call, symmetrized R-MAT, 40 steps, p = 0.5, q = 2, chain rule;
 // before: the record walk's tail phase or its queue, after the preparation
@@ -721,11 +721,11 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 constexpr int kFewTrials = 16;
 constexpr int kFewSearches = 4;
 
-// What a launch of the few-walks kernel does.
-enum class FewPass {
-    kBeside,   // walks, and checks the graph in blocks beside them
-    kAgain,    // walks again, with scans, if that check found unsorted rows
-    kChecked,  // walks after few_check_kernel and few_table_kernel
+// How a search finds a node in a row.
+enum FewFind {
+    kFewSearch,  // sorted rows: by their order
+    kFewScanned, // by reading them
+    kFewTables,  // in their hash tables
 };
 
 // Entries of an unsorted row that a lane reads in one round of a scan, all in
@@ -880,16 +880,19 @@ __device__ __forceinline__ bool group_lookup(const int32_t* __restrict__ table, 
     return found;
 }
 
-// Whether tgt is in [lo, hi) of col: a search of sorted entries or a scan,
-// by the `lanes` lanes (a power of two, lane c of them) that share the arguments;
+// Whether tgt is in [lo, hi) of col: a search of sorted entries or a scan, by
+// the `lanes` lanes (a power of two, lane c of them) that share the arguments;
 // `bits` selects them in a ballot shifted down by their first lane.  Every
 // lane of the wavefront calls it (with lo == hi: no search).
-template <typename Id>
-__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, bool scan, Id lo,
-                                           Id hi, Id tgt, int lanes, int c, int first,
-                                           uint64_t bits) {
+template <FewFind kFind, typename Id>
+__device__ __forceinline__ bool group_find(const int64_t* __restrict__ col,
+                                           const int32_t* __restrict__ table, Id lo, Id hi, Id tgt,
+                                           int lanes, int c, int first, uint64_t bits) {
+    if (kFind == kFewTables)
+        return group_lookup(table, static_cast<int32_t>(lo), static_cast<int32_t>(hi),
+                            static_cast<int32_t>(tgt), lanes, c, first, bits);
     bool found = false;
-    if (scan) {
+    if (kFind == kFewScanned) {
         while (__any(lo < hi)) {
             bool hit = false;
             const Id left = hi - lo;
@@ -941,32 +944,13 @@ __device__ __forceinline__ bool group_find(const int64_t* __restrict__ col, bool
     return found;
 }
 
-template <int kRule, bool kEdges, typename OutT, typename Id, bool kScan>
-__global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int group, int steps,
-                                                              int walk_blocks, FewPass pass,
-                                                              const int32_t* table) {
+// The walks of block blockIdx.x, on groups of `group` lanes, in stretches of
+// `steps` positions.
+template <int kRule, bool kEdges, typename OutT, typename Id, FewFind kFind>
+__device__ __forceinline__ void few_walks(const N2VRecArgs& a, int group, int steps,
+                                          const int32_t* __restrict__ table) {
     const int64_t* const rowptr = a.w.rowptr;
     const int64_t* const col = a.w.col;
-    if (pass == FewPass::kBeside && blockIdx.x >= static_cast<unsigned>(walk_blocks)) {
-        CsrCheck check;
-        const int64_t stride = static_cast<int64_t>(gridDim.x - walk_blocks) * kBlock;
-        const int64_t gid =
-            static_cast<int64_t>(blockIdx.x - walk_blocks) * kBlock + threadIdx.x;
-        if (reinterpret_cast<uintptr_t>(col) % 16 == 0)
-            check.edges4(col, a.w.num_nodes, a.w.num_edges, gid, stride);
-        else
-            for (int64_t i = gid; i < a.w.num_edges; i += stride)
-                check.edge(col, a.w.num_nodes, i, col[i]);
-        check.nodes(rowptr, a.w.num_nodes, col, a.w.num_edges, gid, stride);
-        unsigned long long* w = reinterpret_cast<unsigned long long*>(a.w.work);
-        check.flush(w, MLXC_STATUS_BAD_ROW, MLXC_STATUS_BAD_NODE, w + 2);
-        return;
-    }
-    if (pass == FewPass::kAgain && a.w.work[2] == a.w.work[3]) return;  // the rows are sorted
-    // (kScan false: the rows are taken as sorted)
-    const bool scan = kScan && (pass != FewPass::kChecked || a.rows == MLXC_ROWS_UNSORTED ||
-                                a.w.work[2] != a.w.work[3]);
-    const bool tables = kScan && scan && pass == FewPass::kChecked && a.w.work[1] == 1;
     extern __shared__ __align__(16) unsigned char few_lds[];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int G = group, per_wave = kWave / G;
@@ -1066,17 +1050,17 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
                     // trial order, on equal shares of its lanes
                     const int m = __popcll(open);
                     int Q = 1;
-                    // (a scan takes as many rounds with all lanes on one trial
-                    // as with shares of them on several, of which the first may
-                    // do: several only where each share covers the first row)
-                    Id row_len = 0;
-                    if (kScan) {
+                    if (kFind == kFewScanned) {
+                        // A scan takes as many rounds with all lanes on one trial
+                        // as with shares of them on several, of which the first
+                        // may do: several only where a share covers its row.
                         const Id len = s_hi - s_lo;
-                        row_len = __shfl(len, base + (open ? __builtin_ctzll(open) : 0), kWave);
-                        if (!scan || tables) row_len = 0;
+                        const Id row = __shfl(len, base + (open ? __builtin_ctzll(open) : 0), kWave);
+                        while (Q < m && Q < kFewSearches && Q < G && row <= kFewScan * G / (2 * Q))
+                            Q *= 2;
+                    } else {
+                        while (Q < m && Q < kFewSearches && Q < G) Q *= 2;
                     }
-                    while (Q < m && Q < kFewSearches && Q < G && row_len <= kFewScan * G / (2 * Q))
-                        Q *= 2;
                     const int C = G / Q, q = k / C, c = k % C;
                     uint64_t rest = open;
                     for (int i = 0; i < q; ++i) rest &= rest - 1;
@@ -1086,13 +1070,9 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
                     const Id hi = __shfl(s_hi, src, kWave);
                     const Id tgt = __shfl(s_tgt, src, kWave);
                     const float rs = __shfl(r, src, kWave);
-                    const uint64_t bits = C == kWave ? ~0ull : (1ull << C) - 1;
-                    const bool found =
-                        tables ? group_lookup(table, static_cast<int32_t>(lo),
-                                              static_cast<int32_t>(valid ? hi : lo),
-                                              static_cast<int32_t>(tgt), C, c, base + q * C, bits)
-                               : group_find(col, scan, lo, valid ? hi : lo, tgt, C, c, base + q * C,
-                                            bits);
+                    const bool found = group_find<kFind>(col, table, lo, valid ? hi : lo, tgt, C, c,
+                                                         base + q * C,
+                                                         C == kWave ? ~0ull : (1ull << C) - 1);
                     const bool acc = valid && c == 0 && n2v_resolve<kRule>(a, rs, found);
                     const uint64_t won = (__ballot(acc) >> base) & group_bits;
                     if (won) {
@@ -1150,6 +1130,45 @@ __global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int 
         wave_sync();
     }
     if (status) atomicOr(reinterpret_cast<unsigned long long*>(a.w.work), static_cast<unsigned long long>(status));
+}
+
+// The walks in the blocks before walk_blocks, the check of the graph in those
+// from there on.  again: the launch after it, whose walks start over, with
+// scans, if the check found unsorted rows.
+template <int kRule, bool kEdges, typename OutT, typename Id, FewFind kFind>
+__global__ __launch_bounds__(kBlock) void node2vec_few_kernel(N2VRecArgs a, int group, int steps,
+                                                              int walk_blocks, bool again) {
+    const int64_t* const col = a.w.col;
+    if (blockIdx.x >= static_cast<unsigned>(walk_blocks)) {
+        CsrCheck check;
+        const int64_t stride = static_cast<int64_t>(gridDim.x - walk_blocks) * kBlock;
+        const int64_t gid =
+            static_cast<int64_t>(blockIdx.x - walk_blocks) * kBlock + threadIdx.x;
+        if (reinterpret_cast<uintptr_t>(col) % 16 == 0)
+            check.edges4(col, a.w.num_nodes, a.w.num_edges, gid, stride);
+        else
+            for (int64_t i = gid; i < a.w.num_edges; i += stride)
+                check.edge(col, a.w.num_nodes, i, col[i]);
+        check.nodes(a.w.rowptr, a.w.num_nodes, col, a.w.num_edges, gid, stride);
+        unsigned long long* w = reinterpret_cast<unsigned long long*>(a.w.work);
+        check.flush(w, MLXC_STATUS_BAD_ROW, MLXC_STATUS_BAD_NODE, w + 2);
+        return;
+    }
+    if (again && a.w.work[2] == a.w.work[3]) return;  // the rows are sorted
+    few_walks<kRule, kEdges, OutT, Id, kFind>(a, group, steps, nullptr);
+}
+
+// The walks after few_check_kernel and few_table_kernel.
+template <int kRule, bool kEdges, typename OutT>
+__global__ __launch_bounds__(kBlock) void node2vec_few_tables_kernel(N2VRecArgs a, int group,
+                                                                     int steps,
+                                                                     const int32_t* table) {
+    if (a.w.work[1] == 1)
+        few_walks<kRule, kEdges, OutT, int32_t, kFewTables>(a, group, steps, table);
+    else if (a.rows != MLXC_ROWS_UNSORTED && a.w.work[2] == a.w.work[3])
+        few_walks<kRule, kEdges, OutT, int32_t, kFewSearch>(a, group, steps, nullptr);
+    else  // malformed
+        few_walks<kRule, kEdges, OutT, int32_t, kFewScanned>(a, group, steps, nullptr);
 }
 
 // node2vec walk over edge records (num_nodes, num_edges below 2^31; n_out and
@@ -2135,8 +2154,8 @@ int launch_n2v_few(const N2VRecArgs& a, bool searches, int32_t* table, hipStream
         return rc;
     const size_t lds = static_cast<size_t>(kBlock / kWave) * per_wave * (steps + 1) *
                        (kEdges ? 2 : 1) * sizeof(Id);
-    auto* search = node2vec_few_kernel<kRule, kEdges, OutT, Id, false>;
-    auto* scan = node2vec_few_kernel<kRule, kEdges, OutT, Id, true>;
+    auto* search = node2vec_few_kernel<kRule, kEdges, OutT, Id, kFewSearch>;
+    auto* scan = node2vec_few_kernel<kRule, kEdges, OutT, Id, kFewScanned>;
     const dim3 block(kBlock);
     const int len = static_cast<int>(steps);
     if (table) {
@@ -2154,8 +2173,8 @@ int launch_n2v_few(const N2VRecArgs& a, bool searches, int32_t* table, hipStream
                            w.col, w.num_edges, a.rows, found, checks, w.work, table);
         MLXC_HIP_TRY(hipGetLastError());
         if (int rc = record_walk_event(0, stream)) return rc;
-        hipLaunchKernelGGL(scan, dim3(walk_blocks), block, lds, stream, a, G, len, walk_blocks,
-                           FewPass::kChecked, table);
+        hipLaunchKernelGGL((node2vec_few_tables_kernel<kRule, kEdges, OutT>), dim3(walk_blocks),
+                           block, lds, stream, a, G, len, table);
         MLXC_HIP_TRY(hipGetLastError());
         return record_walk_event(1, stream);
     }
@@ -2163,11 +2182,11 @@ int launch_n2v_few(const N2VRecArgs& a, bool searches, int32_t* table, hipStream
     if (int rc = record_walk_event(0, stream)) return rc;
     hipLaunchKernelGGL(a.rows == MLXC_ROWS_UNSORTED && searches ? scan : search,
                        dim3(walk_blocks + check_blocks), block, lds, stream, a, G, len,
-                       walk_blocks, FewPass::kBeside, nullptr);
+                       walk_blocks, false);
     MLXC_HIP_TRY(hipGetLastError());
     if (a.rows == MLXC_ROWS_DETECT && searches) {  // (else the order does not matter)
         hipLaunchKernelGGL(scan, dim3(walk_blocks), block, lds, stream, a, G, len, walk_blocks,
-                           FewPass::kAgain, nullptr);
+                           true);
         MLXC_HIP_TRY(hipGetLastError());
     }
     return record_walk_event(1, stream);
