@@ -268,9 +268,13 @@ _MIN_WORKSPACE = _lib.MLXC_WORK_WORDS * 8
 # chunk's rows of the rand tensor and of the staging outputs start 16-byte
 # aligned (the windowed kernels' requirement).
 _CHUNK_ALIGN = 64
+# Workspace of the node2vec few-walks kernel without row tables, and the most
+# walks it takes.
+_FEW_WORKSPACE = 2 * _MIN_WORKSPACE
+_FEW_WALKS = 65536
 
 
-def _plan(N: int, row_bytes: int, ws_query, budget: int):
+def _plan(N: int, row_bytes: int, ws_query, budget: int, few: int = 0):
     """How a call of N walks runs within `budget` bytes of device memory for
     its outputs (row_bytes per walk) and workspace (ws_query(n) bytes for n
     walks at the fastest layout; any smaller workspace of at least
@@ -278,13 +282,18 @@ def _plan(N: int, row_bytes: int, ws_query, budget: int):
 
     Returns ("device", None, ws): one call with device outputs and a
     workspace of ws bytes; or ("host", chunk, ws): chunks of `chunk` walks
-    into two device staging buffers, copied into pinned host outputs."""
+    into two device staging buffers, copied into pinned host outputs.  few
+    (0: none): chunks of up to _FEW_WALKS walks run well in `few` bytes,
+    whatever ws_query says of some sizes below, and instead of
+    _FEW_WORKSPACE."""
     out = N * row_bytes
     if out + ws_query(N) <= budget:
         return "device", None, ws_query(N)
     if out + _MIN_WORKSPACE <= budget:
         return "device", None, (budget - out) // 16 * 16
     cost = lambda c: 2 * c * row_bytes + ws_query(c)
+    most = min(N, _FEW_WALKS, (budget - _FEW_WORKSPACE) // (2 * row_bytes)) if few else 0
+    most -= most % _CHUNK_ALIGN
     hi = N // _CHUNK_ALIGN
     if hi >= 1 and cost(_CHUNK_ALIGN) <= budget:
         lo = 1  # the largest multiple k of _CHUNK_ALIGN with cost(k * _CHUNK_ALIGN) <= budget
@@ -294,8 +303,9 @@ def _plan(N: int, row_bytes: int, ws_query, budget: int):
                 lo = mid
             else:
                 hi = mid - 1
-        chunk = lo * _CHUNK_ALIGN
-        return "host", chunk, ws_query(chunk)
+        chunk = max(lo * _CHUNK_ALIGN, most)
+        ws = ws_query(chunk) if cost(chunk) <= budget else _FEW_WORKSPACE
+        return "host", chunk, few if few and ws == _FEW_WORKSPACE else ws
     chunk = min(N, (budget - _MIN_WORKSPACE) // (2 * row_bytes))
     if chunk >= _CHUNK_ALIGN:
         chunk -= chunk % _CHUNK_ALIGN
@@ -307,12 +317,14 @@ def _plan(N: int, row_bytes: int, ws_query, budget: int):
 
 
 def _run_walks(device, stream, handle, N: int, L: int, out_dtype, return_edges: bool,
-               ws_query, launch, budget: Optional[int], check: bool, what: str, inputs):
+               ws_query, launch, budget: Optional[int], check: bool, what: str, inputs,
+               plan_query=None):
     """Runs a walk call on the device.  launch(i0, n, n_ptr, e_ptr, ws_ptr,
     ws_bytes) enqueues walks [i0, i0 + n) of the call on `handle` and returns
     the library's code.  Without a budget the call runs once, with device
     outputs and the fastest workspace; when that allocation fails, or when
-    the outputs and workspace would exceed `budget` bytes, _plan decides."""
+    the outputs and workspace would exceed `budget` bytes, _plan decides
+    (with the query and the `few` that plan_query(), if given, returns)."""
     esize = 8 if out_dtype == torch.int64 else 4
     row_bytes = (2 * L + 1 if return_edges else L + 1) * esize
     if budget is None:
@@ -321,7 +333,10 @@ def _run_walks(device, stream, handle, N: int, L: int, out_dtype, return_edges: 
                              check, what, inputs)
         except torch.cuda.OutOfMemoryError:
             budget = _available_bytes(device)
-    mode, chunk, ws_bytes = _plan(N, row_bytes, ws_query, budget)
+    query, few = ws_query, 0
+    if plan_query is not None and N * row_bytes + ws_query(N) > budget:
+        query, few = plan_query()
+    mode, chunk, ws_bytes = _plan(N, row_bytes, query, budget, few)
     if mode == "device":
         return _run_once(device, stream, N, L, out_dtype, return_edges, ws_bytes, launch, check,
                          what, inputs)
@@ -650,10 +665,26 @@ def rejection_sampling(rowptr: TensorLike, col: TensorLike, start: TensorLike,
                                            offset + i0, rid, rows, n_p, e_p, otype, ws_p,
                                            ws_bytes, handle)
 
+    preferred = lambda n, steps=L: lib.mlxc_rejection_sampling_preferred_bytes(V, E, n, steps, p,
+                                                                               q, rid)
+    older = lambda n: lib.mlxc_rejection_sampling_workspace_bytes(V, E, n, L, p, q, rid)
+
+    def plan_query():
+        # The preferred size does not grow with the walks everywhere: where the
+        # largest call of few walks does not take the few-walks kernel, chunks
+        # are planned by the older query, whose sizes do.  Where its line ends
+        # at 48 steps, chunks without room for records or an index run the
+        # direct kernel (65,536 walks x 40 over 31 M entries, p = 4, q = 0.25,
+        # analytic: 512 us, the few-walks kernel 585; elsewhere it takes up to
+        # twice as long).
+        if preferred(_FEW_WALKS) >= older(_FEW_WALKS):
+            return older, 0
+        beyond = preferred(_FEW_WALKS, max(L, 49)) < older(_FEW_WALKS)
+        return preferred, _FEW_WORKSPACE if beyond else _MIN_WORKSPACE
+
     n_out, e_out = _run_walks(
-        device, stream, handle, N, L, out_dtype, return_edges,
-        lambda n: lib.mlxc_rejection_sampling_preferred_bytes(V, E, n, L, p, q, rid), launch,
-        budget, check, "rejection_sampling", (rowptr, col, start))
+        device, stream, handle, N, L, out_dtype, return_edges, preferred, launch, budget, check,
+        "rejection_sampling", (rowptr, col, start), plan_query)
     return (n_out, e_out) if return_edges else n_out
 
 

@@ -138,6 +138,42 @@ def test_plan_chunks_fit_the_budget(N, row, E, budget):
             2 * bigger * row + q(bigger) > budget
 
 
+@pytest.mark.parametrize("L,budget", [(40, 164 << 20), (40, 41 << 20), (100, 115 << 20),
+                                      (100, 28 << 20), (30, 20 << 20)])
+@pytest.mark.parametrize("p,q,rule", [(0.5, 2.0, 0), (4.0, 0.25, 1), (1.0, 1.0, 0)])
+def test_node2vec_chunks_are_not_cut_small(L, budget, p, q, rule):
+    """Chunked node2vec calls: the preferred workspace does not grow with the
+    walks everywhere (the few-walks kernel takes 2,048 walks of 100 steps but
+    not 10,000), which must not leave a call in many small chunks: a chunk
+    takes most of the budget, or 65,536 walks."""
+    from mlx_cluster_amd import _lib, walks
+    lib = _lib.load()
+    V, E, N = 1 << 20, 31_000_000, 1 << 20
+    row = (L + 1) * 8
+    plans = []
+    real = walks._plan
+
+    def plan(*args):
+        plans.append(real(*args))
+        raise InterruptedError
+
+    walks._plan = plan
+    try:
+        with pytest.raises(InterruptedError):
+            preferred = lambda n: lib.mlxc_rejection_sampling_preferred_bytes(V, E, n, L, p, q, rule)
+            older = lambda n: lib.mlxc_rejection_sampling_workspace_bytes(V, E, n, L, p, q, rule)
+            few = preferred(65536) < older(65536)
+            walks._run_walks(torch.device("cpu"), None, 0, N, L, torch.int64, False, preferred, None,
+                             budget, False, "node2vec", (),
+                             lambda: (preferred, 64) if few else (older, 0))
+    finally:
+        walks._plan = real
+    mode, chunk, ws = plans[0]
+    assert mode == "host" and 2 * chunk * row + ws <= budget and chunk % 64 == 0
+    fits = (budget - 64) // (2 * row)
+    assert chunk >= min(65536, fits // 64 * 64) or 2 * chunk * row + older(chunk) + 64 * 2 * row > budget
+
+
 def test_plan_rejects_a_budget_below_one_walk():
     from mlx_cluster_amd.walks import _plan
     with pytest.raises(ValueError, match="memory_budget"):
