@@ -712,9 +712,9 @@ __device__ void n2v_tail(const N2VRecArgs& a, int32_t* tab, int live, bool sorte
 //
 // Measured (us a call, symmetrized R-MAT, 40 steps, p = 0.5, q = 2, chain rule;
 // before: the record walk's tail phase or its queue, after the preparation
-// passes):  31 M entries: 1,300 walks 361 -> 165 (the check of the 251 MB of
-// col alone takes 60), 8,000 401 -> 228, 32,768 653 -> 386, 65,536
-// 1,391 -> 607;  64 K entries: 1,300 walks 173 -> 103, 65,536 686 -> 332.
+// passes):  31 M entries: 1,300 walks 354 -> 153 (the check of the 251 MB of
+// col alone takes 60), 8,192 389 -> 219, 32,768 641 -> 366, 65,536
+// 1,525 -> 584;  54 K entries: 1,300 walks 193 -> 109, 65,536 912 -> 342.
 // Where it is chosen: n2v_few_steps.
 // Trials a group tries at once, and searches it runs at once, at most: 8 and
 // 32 trials, 1, 2 and 8 searches were within 5% or slower.
