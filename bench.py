@@ -319,21 +319,26 @@ def line_ceiling(table_bytes):
 
 def random_footprint(mc, kind, V, E, N, L, extra):
     """Bytes of the tables a walk call reads at random addresses, by the layout
-    its workspace query selects: the uniform record walk its edge records (8
-    or 16 bytes each), the uniform CSR walk col and rowptr; the node2vec walk
-    its workspace less the start records (edge records or the CSR mode's row
-    starts, the search index, the hub bitmaps).  None for the LDS walks, which
-    read no global table at random."""
+    its preferred workspace selects: the uniform flat and CSR walks and the
+    node2vec few-walks kernel col and rowptr, the uniform record walk its edge
+    records (8 or 16 bytes each); the other node2vec walks their workspace
+    less the start records (edge records or the CSR mode's row starts, the
+    search index, the hub bitmaps).  None for small graphs, which are read
+    from LDS or the caches."""
     lib = mc._lib.load()
+    if V + 1 + E <= 14336:
+        return None
     if kind == "uniform":
         ws = lib.mlxc_random_walk_workspace_bytes(V, E, N, L)
-        if ws <= 256:
-            return None
+        if lib.mlxc_random_walk_preferred_bytes(V, E, N, L) < ws:
+            return 8 * E + 8 * (V + 1)
         rec = 8 if (V - 1).bit_length() + E.bit_length() <= 48 else 16
         return rec * E if ws >= 256 + rec * (E + N) else 8 * E + 8 * (V + 1)
     ws = lib.mlxc_rejection_sampling_workspace_bytes(V, E, N, L, extra["p"], extra["q"],
                                                      RULE_ID[extra["rule"]])
-    return None if ws <= 256 else ws - 256 - 16 * N
+    preferred = lib.mlxc_rejection_sampling_preferred_bytes(V, E, N, L, extra["p"], extra["q"],
+                                                            RULE_ID[extra["rule"]])
+    return 8 * E + 8 * (V + 1) if preferred < ws else ws - 256 - 16 * N
 
 
 def walk_kernel_event_ms(torch, mc, stream, step, calls):
